@@ -2792,48 +2792,80 @@ __global__ void __launch_bounds__(256) k_cells(const R* __restrict__ src, R* __r
 // adjoint of the gather for any in-range index (repeats allowed): the cell n of batch b
 // receives the fp32 sum, over the tokens t of row b with index[b,t] == n in ascending t,
 // of cells[b,t]; cells that no token selects receive zeros. One block per destination
-// cell: the batch row of the index is staged in LDS and every thread scans it in order
-// (a block-uniform test, so no divergence). No atomics: deterministic. The sum starts
-// from -0.0 (the identity of fp32 addition), so a cell with one contributor receives its
-// value bit for bit, as the scatter copy would. Out-of-range indices (only possible when
+// cell. The block first lists its contributors: its threads compare one index each, and a
+// wave's ballot gives every match its place, so the list is in ascending t and the GG
+// comparisons cost one pass per block. Then each thread sums the listed rows, CA_U vectors
+// at a time with all their loads issued together; a cells row belongs to one destination, so
+// the rows are streamed once (non-temporal, as k_cells). No atomics: deterministic. The sum
+// starts from -0.0 (the identity of fp32 addition), so a cell with one contributor receives
+// its value bit for bit, as the scatter copy would. Out-of-range indices (only possible when
 // the host-side validation is skipped) are clamped as the gather clamps them (to the last
 // cell), so the adjoint returns every gathered row's gradient to the cell it was read
-// from. Each block scans its batch row's GG indices per output vector: O(GG^2) work per
-// batch row, negligible at the benchmark grid (GG = 256) and bounded by GG <= 16384.
+// from. Bound by memory: the rows in, the carrier out, and GG indices per block from the L2
+// (11% of the bytes of a 4 x 1152 bf16 cell at GG = 256). 16,384 cells of 4 x 1152 bf16
+// under a permutation: 51 us, 5.9 TB/s, as the scatter copy; with every thread testing all
+// GG indices for each of its vectors 318 us.
 // ----------------------------------------------------------------------------------
+constexpr int CA_U = 4;  // vectors of a thread in flight
 template <typename T, int V, int K>
 __global__ void __launch_bounds__(256) k_cells_add(const T* __restrict__ cells, T* __restrict__ x,
                                                    const int32_t* __restrict__ index, Geo g) {
   constexpr int S = K * K;
-  extern __shared__ int32_t sidx[];
+  constexpr bool NTL = (SIHC_CELLS_NTM & 1) != 0, NTS = (SIHC_CELLS_NTM & 2) != 0;
+  extern __shared__ int32_t hit[];  // contributors of this cell, ascending (at most GG)
+  __shared__ int wave_hits[4];
   const int64_t m = blockIdx.x;  // destination cell b * GG + n
   const int b = int(m / g.GG), n = int(m - int64_t(b) * g.GG);
-  for (int t = threadIdx.x; t < g.GG; t += blockDim.x)
-    sidx[t] = int32_t(min(uint32_t(index[int64_t(b) * g.GG + t]), uint32_t(g.GG) - 1u));
-  __syncthreads();
+  const int tid = int(threadIdx.x), wave = tid / 64, lane = tid % 64;
+  int hits = 0;
+  for (int t0 = 0; t0 < g.GG; t0 += 256) {
+    const int t = t0 + tid;
+    const bool match = t < g.GG && int(index_cell(b * g.GG + min(t, g.GG - 1), g, index)) == n;
+    const uint64_t mask = __ballot(match);
+    if (lane == 0) wave_hits[wave] = __popcll(mask);
+    __syncthreads();
+    int before = hits;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      before += w < wave ? wave_hits[w] : 0;
+      hits += wave_hits[w];
+    }
+    if (match) hit[before + __popcll(mask & ((uint64_t(1) << lane) - 1))] = t;
+    __syncthreads();
+  }
   const int64_t pix0 = cell_pixel0(int(m), g, nullptr);
+  const int64_t row = int64_t(S) * g.C;  // elements of one token's cell
+  const T* __restrict__ src = cells + int64_t(b) * g.GG * row;
   const int nvec = S * g.C / V;
-  for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
-    const int e = i * V;
-    const int s = e / g.C;
-    const int c = e - s * g.C;
-    float acc[V];
+  for (int i0 = tid; i0 < nvec; i0 += CA_U * 256) {
+    float acc[CA_U][V];
 #pragma unroll
-    for (int v = 0; v < V; ++v) acc[v] = -0.f;
-    int hits = 0;
-    for (int t = 0; t < g.GG; ++t) {
-      if (sidx[t] != n) continue;
-      float val[V];
-      load_vec<T, V>(cells + ((int64_t(b) * g.GG + t) * S + s) * g.C + c, val);
+    for (int u = 0; u < CA_U; ++u)
 #pragma unroll
-      for (int v = 0; v < V; ++v) acc[v] += val[v];
-      ++hits;
+      for (int v = 0; v < V; ++v) acc[u][v] = hits ? -0.f : 0.f;
+    for (int h = 0; h < hits; ++h) {
+      const T* __restrict__ r = src + int64_t(hit[h]) * row;
+      RawVec<T, V> val[CA_U];
+#pragma unroll
+      for (int u = 0; u < CA_U; ++u)  // past the last vector: that vector again, not stored
+        load_raw<T, V, NTL>(r + int64_t(min(i0 + u * 256, nvec - 1)) * V, val[u]);
+      load_fence();
+#pragma unroll
+      for (int u = 0; u < CA_U; ++u) {
+        float f[V];
+        raw_to_f32<T, V>(val[u], f);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[u][v] += f[v];
+      }
     }
-    if (hits == 0) {
 #pragma unroll
-      for (int v = 0; v < V; ++v) acc[v] = 0.f;
+    for (int u = 0; u < CA_U; ++u) {
+      const int i = i0 + u * 256;
+      if (i < nvec) {
+        const int s = i * V / g.C, c = i * V - s * g.C;
+        store_vec<T, V, NTS>(x + slot_offset<K>(pix0, s, g, c), acc[u]);
+      }
     }
-    store_vec<T, V>(x + slot_offset<K>(pix0, s, g, c), acc);
   }
 }
 

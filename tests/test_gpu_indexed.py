@@ -124,3 +124,24 @@ def test_indexed_read_write_match_gather_apply_scatter(dtype):
     for i, (g, r) in enumerate(zip(grads, rgrads)):
         kind = "chained" if i == 0 else ("reduced" if i in (1, 2) else "elementwise")
         assert_parity(g, r, dtype, what=f"grad[{i}]", kind=kind)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("grid,slots,channels", [(5, 4, 8), (8, 16, 67), (17, 4, 264), (20, 4, 1160)])
+@pytest.mark.parametrize("pattern", ["permutation", "one", "two", "last"])
+def test_scatter_add_lists_every_contributor_in_order(dtype, grid, slots, channels, pattern):
+    # Contributor lists of 0, 1, 2 and all tokens, over fewer tokens than a wave, exactly one
+    # wave and several passes of a block with a remainder. Same order of the fp32 sums as the
+    # oracle: bit for bit.
+    announce(f"scatter_add {pattern} grid={grid} slots={slots} C={channels} dtype={dtype}")
+    gen = torch.Generator().manual_seed(3)
+    n = grid * grid
+    cells = torch.randn(2, n, slots, channels, generator=gen).to(dtype)
+    idx = {
+        "permutation": torch.stack([torch.randperm(n, generator=gen) for _ in range(2)]),
+        "one": torch.full((2, n), n // 2),
+        "two": torch.where(torch.arange(n) % 3 == 0, 0, n - 1).expand(2, n),
+        "last": torch.full((2, n), n - 1),
+    }[pattern].to(torch.int32).contiguous()
+    got = launch.scatter_add_cells(cells.cuda(), idx.cuda())
+    assert torch.equal(got.cpu(), O.scatter_add_cells(cells, idx))
