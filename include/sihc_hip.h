@@ -42,7 +42,7 @@ extern "C" {
 /* Tokens (batch*grid*grid) or workspace rows per call: fewer than 2^31 - 2^16, so a chunk's
  * end (chunks x tokens-per-chunk < tokens + chunks) and a thread's next token stay in int32. */
 #define SIHC_MAX_TOKENS (((int64_t)1 << 31) - ((int64_t)1 << 16))
-#define SIHC_ABI_VERSION 5
+#define SIHC_ABI_VERSION 6
 /* Bytes of the per-GPU scratch array of sihc_event_backward_noalloc (64 MiB). */
 #define SIHC_SCRATCH_BYTES (64u << 20)
 
@@ -82,6 +82,31 @@ int sihc_weight_grad(const void *x, const void *const *z, void *out, int events,
                      int64_t batch, int grid, int cell, int channels, const int32_t *index,
                      int dtype, int out_dtype, void *workspace, size_t workspace_bytes,
                      void *stream);
+
+/* Whole adjoint of sihc_read, in one pass over x and the E output gradients where the sizes
+ * allow it (4-slot cells, up to 24 events, at least 16 bytes of channels; otherwise
+ * sihc_weight_grad and a zero-carry sihc_write):
+ *   grad_x[m,s,c]     = sum_e alpha[e,c,s] * grads_e[m,c]
+ *   grad_alpha[e,c,s] = sum_m x[m,s,c] * grads_e[m,c]    (as sihc_weight_grad)
+ * alpha is in dtype. No output may overlap an input. Workspace:
+ * sihc_weight_grad_workspace_size.
+ * Replaces: sublayer_kernels.py:276-287 (the read's backward: `_write_impl` and
+ * `_weights_backward` on the same gradients). */
+int sihc_read_backward(const void *x, const void *const *grads, const void *alpha, void *grad_x,
+                       void *grad_alpha, int events, int64_t batch, int grid, int cell,
+                       int channels, const int32_t *index, int dtype, int out_dtype,
+                       void *workspace, size_t workspace_bytes, void *stream);
+
+/* Whole adjoint of sihc_write except the identity to x, in one pass over grad_out and the E
+ * updates under the same conditions (otherwise sihc_weight_grad and sihc_read):
+ *   grad_updates_e[m,c] = sum_s beta[e,c,s] * grad_out[m,s,c]
+ *   grad_beta[e,c,s]    = sum_m grad_out[m,s,c] * updates_e[m,c]
+ * Replaces: sublayer_kernels.py:295-306 (the write's backward: `sublayer_read` and
+ * `_weights_backward` on the same carrier gradient). */
+int sihc_write_backward(const void *grad_out, const void *const *updates, const void *beta,
+                        void *const *grad_updates, void *grad_beta, int events, int64_t batch,
+                        int grid, int cell, int channels, const int32_t *index, int dtype,
+                        int out_dtype, void *workspace, size_t workspace_bytes, void *stream);
 
 /* out[m,c] = base[m,c] + sum_j gamma[j,c] * updates_j[m,c] over `active` updates
  * (1..SIHC_MAX_EVENTS). gamma is [active, channels] in gamma_dtype (fp32 or dtype).

@@ -1,9 +1,10 @@
 // SiHC hyper-connection read/write path for MI355X (gfx950, CDNA4, wave64).
 //
 // All kernels here are weighted stream reductions and broadcasts over a packed NHWC
-// carrier and packed [tokens, channels] workspace tensors, HBM-bound at 4-slot cells.
-// There is no matrix-core work: per element the path does at most 2*E*S flops per
-// 2*(S+E) bytes.
+// carrier and packed [tokens, channels] workspace tensors, HBM-bound at 4-slot cells (per
+// element at most 2*E*S flops per 2*(S+E) bytes). The matrix cores run the one contraction
+// whose operands the lanes already hold, the carrier weight gradient (k_wgrad_mm), and the
+// carrier or update gradients of the same pass.
 //
 // Thread mapping of most kernels: a block is (BCG channel groups) x (TL token lanes).
 // A lane owns V adjacent channels (up to one 16-byte vector) and walks a run of tokens
@@ -17,8 +18,9 @@
 // measured faster. Every token is processed as "issue all loads, then
 // compute, then store" with no data-dependent branches in the loop body, so each lane
 // keeps all of a token's loads in flight at once (the write also issues the next event
-// group's loads early). The pipelined carrier weight gradient instead gives each lane
-// one channel and stages whole tiles of rows in LDS with 16-byte loads, one tile ahead.
+// group's loads early). The pipelined weight gradient (k_wgradz, k_wgradz_d2) instead gives
+// each lane one channel and stages whole tiles of rows in LDS with 16-byte loads, one tile
+// ahead.
 // All sums are fp32 with a single round-to-nearest-even per stored element. Reductions
 // over tokens (weight gradients) are per-lane fp32 partials (for the per-event backward,
 // one LDS pass per block), a per-block partial row, then a fixed-order sum over blocks:
@@ -1617,9 +1619,9 @@ __global__ void __launch_bounds__(512) k_wgrad16(const T* __restrict__ x, PtrPac
   }
 }
 
-// Pipelined carrier weight gradient (4- and 16-slot cells) for bf16 rows of whole
-// 16-byte vectors and up to 32 events. A lane owns ONE channel and EPL events (EPL x S
-// accumulators). The update rows join the carrier tile in LDS (16-byte loads: each wave
+// Pipelined weight gradient for bf16 rows of whole 16-byte vectors (launched for the gamma
+// gradient of 2 updates, one slot; k_wgradz_d2 is its 16-slot form). A lane owns ONE channel
+// and EPL events (EPL x S accumulators). The update rows join the carrier tile in LDS (16-byte loads: each wave
 // stages whole 64-channel rows of its own events, so the update pointer stays
 // wave-uniform), and the loads of tile k+1 are issued into registers before tile k is
 // reduced, so every tile's HBM latency overlaps the previous tile's arithmetic. Tokens
@@ -1629,9 +1631,6 @@ __global__ void __launch_bounds__(512) k_wgrad16(const T* __restrict__ x, PtrPac
 // and EPL per event count come from measurements (launch_wgrad): 4 or 8 waves where they
 // divide the events well (16 slots, E = 24: 6 waves of 4 events 2031 us, 8 waves of 3
 // events 1528 us at batch 256, D 1152), else the fastest measured shape.
-#ifndef SIHC_WGZ_K2  // 1: 4-slot carriers also use k_wgradz (from 2 events)
-#define SIHC_WGZ_K2 1
-#endif
 #ifndef SIHC_C16Z_MINW  // minimum waves per SIMD k_wgradz is compiled for
 #define SIHC_C16Z_MINW 1
 #endif
@@ -1965,86 +1964,391 @@ __global__ void __launch_bounds__(256) k_gamma_rows(const bf16_t* __restrict__ g
 }
 
 // ----------------------------------------------------------------------------------
-// 4-slot carrier weight-gradient partials on the same row lanes (bf16, 16-byte rows):
-// part[chunk][e][s][c] = sum over the chunk's tokens m of x[m,s,c] * z_e[m,c]. Lane = 8
-// channels of a 128-channel slice; update group y takes events y*NA .. y*NA + NA - 1 (past
-// E: the last event again, never written); each thread streams the chunk's tokens r,
-// r + 16 / G, ...: the cell's 4 slot vectors (through the state index if any) and its NA
-// update vectors, 4 x 8 x NA fp32 sums in registers. Every group loads the cell's slot
-// vectors (the other groups' copies come from L2); nothing is staged in LDS. Measured per
-// event count against the pipelined kernel at the XL shape (batch 256, D = 1152): E = 5
-// 280 -> 249 us, E = 12 414 -> 372, E = 16 525 -> 501, E = 24 734 -> 712, E = 32 1067 ->
-// 923; E = 3-4 and 17-18 keep the pipelined kernel (as fast there, or faster).
+// Carrier weight-gradient partials on the matrix cores:
+//   part[chunk][e][s][c] = sum over the chunk's tokens m of x[m,s,c] * z_e[m,c]
+// Per channel this is a [slots x tokens] . [tokens x events] product, and a 4x4 matrix
+// instruction of 16 blocks does 16 channels at once: block b of the wave, its lanes 4b + q,
+// holds one channel of channel group b, row q of the left operand is slot 4*sg + q and column
+// q of the right operand is event 4*eg + q. So lane 4b + q streams the row of ITS slot and the
+// rows of ITS events (VC channels of each, one 16-byte load per token), 4 tokens at a time;
+// nothing is staged in LDS and no row is loaded twice by a wave, where a vector-ALU lane needs
+// all slots beside its events' rows. bf16: the 4 tokens of a channel are packed into the 4 k
+// values of v_mfma_f32_4x4x4_16b_bf16 with two v_perm_b32 per channel (products exact, one
+// fp32 rounding per 4 tokens, which measured closer to the exact sum than 4 chained fused
+// multiply-adds). fp32: v_mfma_f32_4x4x1_16b_f32, one token at a time (bit for bit a fused
+// multiply-add). acc[sg][eg][v] holds, in lane 4b + q, slots 4*sg + 0..3 of event 4*eg + q at
+// channel v of group b.
+//
+// A block is WP parts (SGW of the slot groups x EGW of the event groups each) x WT token
+// waves, for one slice of 16 * VC channels and one chunk of tokens; token wave w takes the
+// groups of 4 tokens w, w + WT, ... The token waves' sums meet in LDS once per chunk, in
+// ascending order. Channel groups past the width are idle; the last one is moved back to end
+// with the width, so its first channels repeat the previous group's (the same sums, stored
+// twice), and any width of at least VC channels takes whole vectors at any alignment.
+//
+// The fused modes compute the other gradient of the same inputs in the same pass: a quad
+// transposes its 4 x 4 words (DPP), so that lane q holds token q with the 4 events (MM_READ)
+// or slots (MM_WRITE) as its 4 k values, and multiplies them by the staged weights; the output
+// of lane 4b + q is then slot or event q of 4 tokens, the layout of its loads.
+//
+// Bound by memory. Measured against the vector-ALU kernels it replaced, one pass of 65,536
+// tokens x 1152 channels, 4 slots, bf16: E = 4 215 -> 203 us, E = 8 285 -> 274, E = 16
+// 501 -> 447 (6.76 TB/s), E = 24 711 -> 631 (6.71 TB/s), E = 12 371 -> 380; fp32, 16,384
+// tokens, E = 24 384 -> 345; 6,144 tokens x 627 channels, bf16, E = 16 166 -> 63; 16 slots,
+// fp32, 8,192 tokens x 768, E = 1 294 -> 87, E = 12 228 -> 169, E = 24 348 -> 254; 16 slots,
+// bf16, 32,768 tokens x 1152, E = 8 355 -> 295 (6.15 TB/s). Read backward against the zero-carry
+// write and the weight gradient, 65,536 x 1152: E = 4 431 -> 325 us, E = 8 601 -> 412, E = 16
+// 1034 -> 651, E = 24 1482 -> 905 (5.3 TB/s: 28 arrays in, the carrier out). Write backward
+// against the read and the weight gradient: E = 4 426 -> 335, E = 8 611 -> 560; from 9 events
+// the one pass with up to 24 arrays out is no faster, and two kernels run (E = 16 1116 one
+// pass, 1030 two).
 // ----------------------------------------------------------------------------------
-template <int NA>
-__global__ void __launch_bounds__(256) k_wgrad_rows(const bf16_t* __restrict__ x, PtrPack z, float* __restrict__ part,
-                                                    const int32_t* __restrict__ index, int E, Geo g, int tpb,
-                                                    int nslices) {
-  constexpr int S = 4;
-  __shared__ float red[256 * 8];  // [token row][group][lane][8]
-  const int lx = int(threadIdx.x), gy = int(threadIdx.y), r = int(threadIdx.z);
-  const int G = int(blockDim.y), TR = int(blockDim.z);
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+template <typename T, int VC>
+struct MMRow {  // VC channels of one row as the words a load returns
+  static constexpr int NW = VC * int(sizeof(T)) / 4;
+  uint32_t w[NW];
+};
+template <typename T, int VC>
+__device__ __forceinline__ void mm_load(const T* p, MMRow<T, VC>& r) {
+  typedef typename RawT<VC * int(sizeof(T))>::type R;
+  typedef R RU __attribute__((aligned(sizeof(T))));  // any element alignment
+  const R v = __builtin_nontemporal_load(reinterpret_cast<const RU*>(p));
+  __builtin_memcpy(r.w, &v, sizeof(R));
+}
+// acc[v] += the 4x4 products of rows a (tokens x the lane's slot) and b (tokens x its event)
+template <int VC>
+__device__ __forceinline__ void mm_acc(const MMRow<bf16_t, VC> (&a)[4], const MMRow<bf16_t, VC> (&b)[4],
+                                       f32x4 (&acc)[VC]) {
+#pragma unroll
+  for (int k = 0; k < VC / 2; ++k) {
+    const uint32_t al[2] = {pair_lo(a[0].w[k], a[1].w[k]), pair_lo(a[2].w[k], a[3].w[k])};
+    const uint32_t ah[2] = {pair_hi(a[0].w[k], a[1].w[k]), pair_hi(a[2].w[k], a[3].w[k])};
+    const uint32_t bl[2] = {pair_lo(b[0].w[k], b[1].w[k]), pair_lo(b[2].w[k], b[3].w[k])};
+    const uint32_t bh[2] = {pair_hi(b[0].w[k], b[1].w[k]), pair_hi(b[2].w[k], b[3].w[k])};
+    acc[2 * k] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, al), __builtin_bit_cast(s16x4, bl),
+                                                        acc[2 * k], 0, 0, 0);
+    acc[2 * k + 1] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, ah),
+                                                            __builtin_bit_cast(s16x4, bh), acc[2 * k + 1], 0, 0, 0);
+  }
+}
+template <int VC>
+__device__ __forceinline__ void mm_acc(const MMRow<float, VC> (&a)[4], const MMRow<float, VC> (&b)[4],
+                                       f32x4 (&acc)[VC]) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int v = 0; v < VC; ++v)
+      acc[v] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(a[t].w[v]), __uint_as_float(b[t].w[v]), acc[v], 0,
+                                                  0, 0);
+}
+
+template <typename T, int VC>
+__device__ __forceinline__ void mm_store(T* p, const float (&v)[VC]) {
+  typedef typename RawT<VC * int(sizeof(T))>::type R;
+  typedef R RU __attribute__((aligned(sizeof(T))));
+  T e[VC];
+#pragma unroll
+  for (int i = 0; i < VC; ++i) e[i] = from_f32<T>(v[i]);
+  R r;
+  __builtin_memcpy(&r, e, sizeof(R));
+  asm volatile("" : "+v"(r));  // as in st(): keeps the non-temporal hint
+  __builtin_nontemporal_store(r, reinterpret_cast<RU*>(p));
+}
+// Transpose the 4 x 4 words that a quad of lanes holds (lane q, word t -> lane t, word q)
+// with two exchanges inside the quad (DPP quad permutes).
+__device__ __forceinline__ void quad_transpose(uint32_t& r0, uint32_t& r1, uint32_t& r2, uint32_t& r3, int q) {
+  auto swap1 = [&](uint32_t& a, uint32_t& b) {  // lanes q, q ^ 1
+    const bool o = q & 1;
+    const uint32_t got = uint32_t(__builtin_amdgcn_update_dpp(0, int(o ? a : b), 0xB1, 0xF, 0xF, true));
+    a = o ? got : a;
+    b = o ? b : got;
+  };
+  auto swap2 = [&](uint32_t& a, uint32_t& b) {  // lanes q, q ^ 2
+    const bool o = q & 2;
+    const uint32_t got = uint32_t(__builtin_amdgcn_update_dpp(0, int(o ? a : b), 0x4E, 0xF, 0xF, true));
+    a = o ? got : a;
+    b = o ? b : got;
+  };
+  swap1(r0, r1);
+  swap1(r2, r3);
+  swap2(r0, r2);
+  swap2(r1, r3);
+}
+template <typename T, int VC>
+__device__ __forceinline__ void quad_transpose(MMRow<T, VC> (&r)[4], int q) {
+#pragma unroll
+  for (int k = 0; k < MMRow<T, VC>::NW; ++k) quad_transpose(r[0].w[k], r[1].w[k], r[2].w[k], r[3].w[k], q);
+}
+// d[v] += sum over k of a[k] (lane q: token q) * w[k] (lane q: the output column q), the
+// weights of the 4 k values staged per channel: bf16 as one 8-byte word quad per (channel,
+// lane), fp32 as VC floats per (k, lane).
+template <int VC>
+__device__ __forceinline__ void mm_out(const MMRow<bf16_t, VC> (&a)[4], const float* wl, int lane, f32x4 (&d)[VC]) {
+#pragma unroll
+  for (int k = 0; k < VC / 2; ++k) {
+    const u32x4 w = reinterpret_cast<const u32x4*>(wl)[k * 64 + lane];  // channels 2k, 2k + 1
+    const uint32_t al[2] = {pair_lo(a[0].w[k], a[1].w[k]), pair_lo(a[2].w[k], a[3].w[k])};
+    const uint32_t ah[2] = {pair_hi(a[0].w[k], a[1].w[k]), pair_hi(a[2].w[k], a[3].w[k])};
+    const uint32_t wa[2] = {w[0], w[1]}, wb[2] = {w[2], w[3]};
+    d[2 * k] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, al), __builtin_bit_cast(s16x4, wa),
+                                                      d[2 * k], 0, 0, 0);
+    d[2 * k + 1] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, ah),
+                                                          __builtin_bit_cast(s16x4, wb), d[2 * k + 1], 0, 0, 0);
+  }
+}
+template <int VC>
+__device__ __forceinline__ void mm_out(const MMRow<float, VC> (&a)[4], const float* wl, int lane, f32x4 (&d)[VC]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const f32x4 w = reinterpret_cast<const f32x4*>(wl)[k * 64 + lane];
+    static_assert(VC == 4, "fp32 lanes hold 4 channels");
+#pragma unroll
+    for (int v = 0; v < VC; ++v)
+      d[v] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(a[k].w[v]), w[v], d[v], 0, 0, 0);
+  }
+}
+constexpr int MM_GRAD = 0;   // the weight gradient alone
+constexpr int MM_READ = 1;   // backward of the read: also dx[m,s,c] = sum_e w[e,c,s] * z_e[m,c]
+constexpr int MM_WRITE = 2;  // backward of the write: also dz_e[m,c] = sum_s w[e,c,s] * x[m,s,c]
+// LDS floats of one event group's staged weights (the same for both element types)
+template <typename T, int VC>
+constexpr int MM_WG = 64 * VC * 4 * int(sizeof(T)) / 4;
+
+template <typename T, int K, int SGW, int EGW, int VC, int MODE>
+__global__ void __launch_bounds__(256) k_wgrad_mm(const T* __restrict__ x, PtrPack z, float* __restrict__ part,
+                                                  const int32_t* __restrict__ index, int E, Geo g, int gs,
+                                                  int nchunks, int nslices, int wt, int segs,
+                                                  const T* __restrict__ w,
+                                                  T* __restrict__ dx, PtrPack dz) {
+  constexpr int S = K * K, LW = 64 * VC * 4;  // LW: floats of one wave's accumulators of a group pair
+  static_assert(MODE == MM_GRAD || S == 4, "fused outputs: 4-slot cells, one part per block");
+  extern __shared__ __align__(16) float mmred[];  // [waves][4 slots][4 events][16 * VC]; before: staged weights
+  const int tid = int(threadIdx.x), lane = tid % 64, b = lane >> 2, q = lane & 3;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int tw = wave % wt, pw = wave / wt;                    // token wave, part
+  const int sg0 = (pw % segs) * SGW, eg0 = (pw / segs) * EGW;  // this part's first slot / event group
   int slice, chunk;
-  slice_chunk(int(blockIdx.x), nslices, slice, chunk);
-  const int c0 = slice * 128 + lx * 8;
-  const int j0 = gy * NA;
-  float acc[NA][S][8];
+  slice_chunk_unless8(int(blockIdx.x), nslices, slice, chunk);
+  const int cb = (slice * 16 + b) * VC;
+  const int c0 = min(cb, g.C - VC);
+  if constexpr (MODE != MM_GRAD) {
+    // weights of event group eg: MM_READ lane q = slot q, k = event; MM_WRITE lane q = event, k = slot
+    for (int i = tid; i < (E + 3) / 4 * VC * 64 * 4; i += int(blockDim.x)) {  // [eg][k][v][lane]
+      const int ln = i % 64, v = (i / 64) % VC, k = (i / (64 * VC)) % 4, eg = i / (64 * VC * 4);
+      const int e = eg * 4 + (MODE == MM_READ ? k : (ln & 3)), sl = MODE == MM_READ ? (ln & 3) : k;
+      const int c = min((slice * 16 + (ln >> 2)) * VC, g.C - VC) + v;
+      const T val = e < E ? w[(int64_t(e) * g.C + c) * S + sl] : T(0);
+      T* ws = reinterpret_cast<T*>(mmred + eg * MM_WG<T, VC>);
+      if constexpr (sizeof(T) == 2) {
+        ws[((v >> 1) * 64 + ln) * 8 + (v & 1) * 4 + k] = val;
+      } else {
+        ws[(k * 64 + ln) * VC + v] = val;
+      }
+    }
+    __syncthreads();
+  }
+  const T* zp[EGW];
+  T* dzp[MODE == MM_WRITE ? EGW : 1];
 #pragma unroll
-  for (int q = 0; q < NA; ++q)
+  for (int eg = 0; eg < EGW; ++eg) {
+    const int e = min((eg0 + eg) * 4 + q, E - 1);
+    zp[eg] = static_cast<const T*>(z.p[e]) + c0;
+    if constexpr (MODE == MM_WRITE) dzp[eg] = static_cast<T*>(const_cast<void*>(dz.p[e])) + c0;
+  }
+  const T* xp[SGW];
 #pragma unroll
-    for (int s = 0; s < S; ++s)
+  for (int sg = 0; sg < SGW; ++sg) xp[sg] = x + slot_offset<K>(0, (sg0 + sg) * 4 + q, g, c0);
+  T* dxp = nullptr;
+  if constexpr (MODE == MM_READ) dxp = dx + slot_offset<K>(0, q, g, c0);
+  f32x4 acc[SGW][EGW][VC];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) acc[q][s][k] = 0.f;
-  if (c0 < g.C) {
-    const int m_end = min(chunk * tpb + tpb, g.M);
-    const u32x4* up[NA];
+  for (int sg = 0; sg < SGW; ++sg)
 #pragma unroll
-    for (int q = 0; q < NA; ++q) up[q] = static_cast<const u32x4*>(z.p[min(j0 + q, E - 1)]);
-    for (int m = chunk * tpb + r; m < m_end; m += TR) {
-      const int64_t p0 = cell_pixel0(m, g, index);
-      u32x4 xv[S];
+    for (int eg = 0; eg < EGW; ++eg)
 #pragma unroll
-      for (int s = 0; s < S; ++s) xv[s] = ld<true>(reinterpret_cast<const u32x4*>(x + slot_offset<2>(p0, s, g, c0)));
-      const int64_t o = (int64_t(m) * g.C + c0) >> 3;  // 16-byte vector index of the update rows
-      u32x4 uv[NA];
+      for (int v = 0; v < VC; ++v) acc[sg][eg][v] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // The chunk's tokens: groups of gs tokens (a multiple of 4 * wt), group `chunk` and every
+  // nchunks-th one after it, so that the blocks resident at one time stream through a narrow
+  // window of each array. (m0, mi): this wave's next 4 tokens, m0 + mi.
+  int m0 = chunk * gs, mi = tw * 4;
+  if (cb < g.C && m0 + mi < g.M) {
+    // The rows of the wave's next 4 tokens are loaded into each row set as soon as its
+    // current rows are used up, so the loads of one group or another are in flight all the
+    // time. Past a group's end its last token is loaded again and zeroed.
+    MMRow<T, VC> xn[SGW][4], zr[EGW][4];
+    int64_t p0[4], zo[4], p1[4], z1[4];  // row offsets of the current and of the next 4 tokens
+    auto offsets = [&](int m, int m_end) {
 #pragma unroll
-      for (int q = 0; q < NA; ++q) uv[q] = ld<true>(up[q] + o);
-      load_fence();
-      float xf[S][8];
+      for (int t = 0; t < 4; ++t) {
+        const int mt = min(m + t, m_end - 1);
+        p1[t] = cell_pixel0(mt, g, index) * g.C;
+        z1[t] = int64_t(mt) * g.C;
+      }
+    };
+    auto load_x = [&]() {
 #pragma unroll
-      for (int s = 0; s < S; ++s)
+      for (int sg = 0; sg < SGW; ++sg)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          xf[s][2 * k] = __uint_as_float(xv[s][k] << 16);
-          xf[s][2 * k + 1] = __uint_as_float(xv[s][k] & 0xffff0000u);
+        for (int t = 0; t < 4; ++t) mm_load<T, VC>(xp[sg] + p1[t], xn[sg][t]);
+    };
+    auto load_z = [&](int eg) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) mm_load<T, VC>(zp[eg] + z1[t], zr[eg][t]);
+    };
+    // one iteration: the current 4 tokens (tn of them real); with MORE, the next ones' loads
+    auto step = [&](int tn, auto more) {
+      constexpr bool MORE = decltype(more)::value;
+      MMRow<T, VC> xr[SGW][4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int sg = 0; sg < SGW; ++sg) xr[sg][t] = xn[sg][t];
+      if (tn < 4) {  // both operands: a zero factor alone would turn an Inf into NaN
+#pragma unroll
+        for (int t = 1; t < 4; ++t)
+          if (t >= tn) {
+#pragma unroll
+            for (int k = 0; k < MMRow<T, VC>::NW; ++k) {
+#pragma unroll
+              for (int sg = 0; sg < SGW; ++sg) xr[sg][t].w[k] = 0u;
+#pragma unroll
+              for (int eg = 0; eg < EGW; ++eg) zr[eg][t].w[k] = 0u;
+            }
+          }
+      }
+      if constexpr (MORE) {
+        load_x();
+        load_fence();
+      }
+      MMRow<T, VC> xt[4];  // MM_WRITE: lane q: token q, row k: slot k
+      f32x4 d[VC];
+      if constexpr (MODE == MM_WRITE) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) xt[t] = xr[0][t];
+        quad_transpose<T, VC>(xt, q);
+      }
+      if constexpr (MODE == MM_READ) {
+#pragma unroll
+        for (int v = 0; v < VC; ++v) d[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int eg = 0; eg < EGW; ++eg) {
+#pragma unroll
+        for (int sg = 0; sg < SGW; ++sg) mm_acc<VC>(xr[sg], zr[eg], acc[sg][eg]);
+        if constexpr (MODE == MM_READ) {
+          if (eg * 4 + 4 > E) {  // lanes past the last event repeat it: nothing of theirs may be summed
+            const bool real = eg * 4 + q < E;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+              for (int k = 0; k < MMRow<T, VC>::NW; ++k) zr[eg][t].w[k] = real ? zr[eg][t].w[k] : 0u;
+          }
+          quad_transpose<T, VC>(zr[eg], q);  // lane q: token q, row k: event 4 eg + k
+          mm_out<VC>(zr[eg], mmred + eg * MM_WG<T, VC>, lane, d);
         }
+        if constexpr (MORE) {
+          load_z(eg);
+          load_fence();
+        }
+        if constexpr (MODE == MM_WRITE) {
 #pragma unroll
-      for (int q = 0; q < NA; ++q)
+          for (int v = 0; v < VC; ++v) d[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+          mm_out<VC>(xt, mmred + (eg0 + eg) * MM_WG<T, VC>, lane, d);
+          const bool real = (eg0 + eg) * 4 + q < E;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float z0 = __uint_as_float(uv[q][k] << 16), z1 = __uint_as_float(uv[q][k] & 0xffff0000u);
+          for (int t = 0; t < 4; ++t) {
+            float o[VC];
 #pragma unroll
-          for (int s = 0; s < S; ++s) {
-            acc[q][s][2 * k] = fmaf(xf[s][2 * k], z0, acc[q][s][2 * k]);
-            acc[q][s][2 * k + 1] = fmaf(xf[s][2 * k + 1], z1, acc[q][s][2 * k + 1]);
+            for (int v = 0; v < VC; ++v) o[v] = d[v][t];
+            if (real && t < tn) mm_store<T, VC>(dzp[eg] + zo[t], o);
           }
         }
+      }
+      if constexpr (MODE == MM_READ) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          float o[VC];
+#pragma unroll
+          for (int v = 0; v < VC; ++v) o[v] = d[v][t];
+          if (t < tn) mm_store<T, VC>(dxp + p0[t], o);
+        }
+      }
+    };
+    offsets(m0 + mi, min(m0 + gs, g.M));
+    load_x();
+#pragma unroll
+    for (int eg = 0; eg < EGW; ++eg) load_z(eg);
+    load_fence();
+    while (true) {
+      const int tn = min(4, min(m0 + gs, g.M) - (m0 + mi));
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        p0[t] = p1[t];
+        zo[t] = z1[t];
+      }
+      mi += wt * 4;
+      if (mi >= gs) {
+        mi = tw * 4;
+        m0 = nchunks * gs < g.M - m0 ? m0 + nchunks * gs : g.M;  // the last chunk's sum stays below 2^31
+      }
+      const bool last = m0 + mi >= g.M;
+      if constexpr (SGW * EGW * VC <= 32) {
+        if (last) {
+          step(tn, std::false_type{});
+          break;
+        }
+        offsets(m0 + mi, min(m0 + gs, g.M));
+        step(tn, std::true_type{});
+      } else {
+        // a second body would not fit the registers beside more than 128 sums per lane: the
+        // last iteration loads its first token's rows again, to no use
+        if (last) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            p1[t] = p0[0];
+            z1[t] = zo[0];
+          }
+        } else {
+          offsets(m0 + mi, min(m0 + gs, g.M));
+        }
+        step(tn, std::true_type{});
+        if (last) break;
+      }
     }
   }
-  const int tid = (r * G + gy) * 16 + lx;
+  if constexpr (MODE != MM_GRAD) __syncthreads();  // the staged weights give way to the sums
+  // per group pair: the token waves' sums, then whole rows of the partial
 #pragma unroll
-  for (int q = 0; q < NA; ++q)
+  for (int sg = 0; sg < SGW; ++sg)
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
+    for (int eg = 0; eg < EGW; ++eg) {
+      float* mine = mmred + wave * LW;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) red[tid * 8 + k] = acc[q][s][k];
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int v = 0; v < VC; v += 4) {
+          f32x4 r;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) r[j] = acc[sg][eg][v + j][i];
+          *reinterpret_cast<f32x4*>(mine + (i * 4 + q) * 16 * VC + b * VC + v) = r;
+        }
       __syncthreads();
-      for (int i = tid; i < G * 128; i += 256) {  // (group, channel of the slice)
-        const int gi = i >> 7, cl = i & 127;
-        float sum = 0.f;
-        for (int rr = 0; rr < TR; ++rr) sum += red[(rr * G + gi) * 128 + cl];
-        const int e = gi * NA + q, c = slice * 128 + cl;
-        if (e < E && c < g.C) part[((int64_t(chunk) * E + e) * S + s) * g.C + c] = sum;
+      // the part's waves share its 16 rows of 4 * VC quads
+      for (int k = tw * 64 + lane; k < 16 * 4 * VC; k += wt * 64) {
+        const float* src = mmred + pw * wt * LW + k * 4;
+        f32x4 sum = *reinterpret_cast<const f32x4*>(src);
+        for (int u = 1; u < wt; ++u) sum += *reinterpret_cast<const f32x4*>(src + u * LW);
+        const int row = k / (4 * VC), cq = (k - row * 4 * VC) * 4;  // row = slot of the group * 4 + event
+        const int sl = (sg0 + sg) * 4 + row / 4, e = (eg0 + eg) * 4 + (row & 3);
+        const int cg = slice * 16 * VC + cq / VC * VC;  // this quad's channel group
+        if (e < E && cg < g.C) {
+          typedef f32x4 f32x4_u __attribute__((aligned(4)));
+          float* dst = part + ((int64_t(chunk) * E + e) * S + sl) * g.C + min(cg, g.C - VC) + cq % VC;
+          *reinterpret_cast<f32x4_u*>(dst) = sum;
+        }
       }
       __syncthreads();
     }
@@ -3408,6 +3712,87 @@ int cells_add(const char* what, const void* cells, const int32_t* index, void* x
   });
 }
 
+// Launch k_wgrad_mm with EG event groups per part; `chunks` (at most max_chunks) is set to the
+// partial rows it writes. `mode` and the pointers after it as in the kernel.
+struct MMArgs {
+  const void* x;
+  PtrPack z;
+  float* part;
+  const int32_t* index;
+  int events;
+  Geo g;
+  const void* w;
+  void* dx;
+  PtrPack dz;
+};
+template <typename T, int K, int SGW, int EGW, int MODE>
+int launch_mm(const char* what, const MMArgs& a, int max_chunks, int* chunks, hipStream_t st) {
+  constexpr int VC = 16 / int(sizeof(T));
+  const int segs = K * K / 4 / SGW, parts = segs * (((a.events + 3) / 4 + EGW - 1) / EGW);
+  const int slices = (a.g.C + 16 * VC - 1) / (16 * VC);
+  auto* kfn = &k_wgrad_mm<T, K, SGW, EGW, VC, MODE>;
+  const size_t weights = MODE == MM_GRAD ? 0 : size_t((a.events + 3) / 4) * MM_WG<T, VC> * sizeof(float);
+  auto lds_for = [&](int waves) { return std::max(size_t(waves) * 64 * VC * 4 * sizeof(float), weights); };
+  // Chunks of a launch with wt token waves per block: whole rounds of resident blocks, so
+  // that the last round is not part-empty.
+  auto chunks_for = [&](int wt) {
+    const int waves = parts * wt;
+    return whole_rounds(slices, max_chunks,
+                        resident_blocks(reinterpret_cast<const void*>(kfn), waves * 64, lds_for(waves)));
+  };
+  // Token waves per block. One wave per chunk and slice streams best once the waves' loads
+  // (SGW + EGW groups of 4 KB) fill the memory system; with fewer bytes in flight the waves
+  // of a block split their chunk's tokens. The lines are where the two sides crossed (bf16
+  // and fp32, 512-65,536 tokens x 627-1152 channels, 1-24 events); the plain gradient of 5-8
+  // events runs better with two waves at every size (65,536 x 1152: 302 -> 274 us).
+  const int64_t enough = int64_t(MODE == MM_GRAD ? 15 : 11) << 20;
+  int wt = MODE == MM_GRAD && parts == 1 && SGW == 1 && EGW == 2 ? 2 : 1;
+  while (wt * 2 * parts <= 4 && int64_t(slices) * chunks_for(wt) * parts * wt * (SGW + EGW) * 4096 < enough) wt *= 2;
+  int n = chunks_for(wt);
+  const int threads = parts * wt * 64;
+  if (threads > 256) return fail(SIHC_ERR_INVALID, "%s: internal weight-gradient shape", what);
+  const int gs = std::max(8, 4 * wt);  // 8-token groups: B = 256, E = 16 read backward 653 us (64 tokens: 742)
+  n = int(std::min<int64_t>(n, (int64_t(a.g.M) + gs - 1) / gs));  // no chunk without a token
+  hipLaunchKernelGGL(kfn, dim3(blocks1d(slices, n)), dim3(threads), lds_for(parts * wt), st,
+                     static_cast<const T*>(a.x), a.z, a.part, a.index, a.events, a.g, gs, n, slices, wt, segs,
+                     static_cast<const T*>(a.w), static_cast<T*>(a.dx), a.dz);
+  *chunks = n;
+  return check_launch(what);
+}
+// 4-slot cells: one part with all event groups.
+template <typename T, int MODE>
+int launch_mm_k2(const char* what, const MMArgs& a, int max_chunks, int* chunks, hipStream_t st) {
+  if (a.events <= 4) return launch_mm<T, 2, 1, 1, MODE>(what, a, max_chunks, chunks, st);
+  if (a.events <= 8) return launch_mm<T, 2, 1, 2, MODE>(what, a, max_chunks, chunks, st);
+  if constexpr (MODE == MM_WRITE) return fail(SIHC_ERR_INVALID, "%s: internal weight-gradient shape", what);
+  switch ((a.events + 3) / 4) {
+    case 3: return launch_mm<T, 2, 1, 3, MODE>(what, a, max_chunks, chunks, st);
+    case 4: return launch_mm<T, 2, 1, 4, MODE>(what, a, max_chunks, chunks, st);
+    case 5: return launch_mm<T, 2, 1, 5, MODE>(what, a, max_chunks, chunks, st);
+    case 6: return launch_mm<T, 2, 1, 6, MODE>(what, a, max_chunks, chunks, st);
+    default: break;
+  }
+  if constexpr (MODE == MM_GRAD) {
+    if (a.events <= 32)
+      return a.events <= 28 ? launch_mm<T, 2, 1, 7, MODE>(what, a, max_chunks, chunks, st)
+                            : launch_mm<T, 2, 1, 8, MODE>(what, a, max_chunks, chunks, st);
+  }
+  return fail(SIHC_ERR_INVALID, "%s: internal weight-gradient shape", what);
+}
+
+// 16-slot cells: all slot groups in a wave, up to 4 (fp32) or 2 (bf16) event groups per part.
+template <typename T>
+int launch_mm_k4(const char* what, const MMArgs& a, int max_chunks, int* chunks, hipStream_t st) {
+  const int groups = (a.events + 3) / 4;
+  if (groups == 1) return launch_mm<T, 4, 4, 1, MM_GRAD>(what, a, max_chunks, chunks, st);
+  if constexpr (sizeof(T) == 4) {
+    if (groups == 3 || groups == 5 || groups == 6)
+      return launch_mm<T, 4, 4, 3, MM_GRAD>(what, a, max_chunks, chunks, st);
+    if (groups >= 4) return launch_mm<T, 4, 4, 4, MM_GRAD>(what, a, max_chunks, chunks, st);
+  }
+  return launch_mm<T, 4, 4, 2, MM_GRAD>(what, a, max_chunks, chunks, st);
+}
+
 // Shared launcher of the atomics-free weight-gradient reduction + finalize. With
 // `dout` (workspace mode), the update gradients dout[e] = x * gamma[e] are written in
 // the same pass.
@@ -3508,14 +3893,25 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
           // Shapes of the pipelined kernel (waves x events per lane), measured per event count
           // at the XL shape (batch 256, D 1152). Every shape stages every event row (waves x
           // events per lane >= E) and covers the carrier tile (64 x waves x vectors per
-          // thread >= 256 vectors at 4 slots, 1024 at 16).
+          // thread >= 1024 vectors at 16 slots).
+          // Carriers of at least one 16-byte vector of channels: the matrix-core kernel, except
+          // where another one measured faster (65,536 tokens x 1152 channels, bf16, and 32,768
+          // for 16 slots): one event of aligned 4-slot rows on the direct kernel (136 us, here
+          // 143), 9 and more events of aligned bf16 16-slot rows on the pipelined one (E = 12
+          // 416 us, here 447; E = 8 355, here 295).
+          if constexpr (CAR) {
+            const bool direct = KK == 2 && events == 1 && VV * int(sizeof(T)) == 16;
+            if (g.C >= 16 / int(sizeof(T)) && !direct && !(KK == 4 && bf && events > 8)) {
+              const MMArgs a{x, pk, part, index, events, g, nullptr, nullptr, PtrPack{}};
+              if constexpr (KK == 2) return launch_mm_k2<T, MM_GRAD>(what, a, max_chunks, &chunks, st);
+              else return launch_mm_k4<T>(what, a, max_chunks, &chunks, st);
+            }
+          }
           if constexpr (CAR && KK == 4) {
             if (bf) {
               // 16 slots: E = 9 3 x 3 730 us (2 x 5 of 4: 907), E = 17-21 8 x 3 1095-1142 us
               // (5-6 x 4: 1320-1429), E = 28 / 32 8 x 4 1405 / 1421 us (k_wgrad16: 2290 / 2089)
-              if (events <= 4) goz(IC<4>{}, IC<4>{}, IC<1>{}, 4);        // idle waves only stage
-              else if (events <= 8) goz(IC<4>{}, IC<8>{}, IC<4>{}, 2);
-              else if (events == 9) goz(IC<4>{}, IC<6>{}, IC<3>{}, 3);
+              if (events == 9) goz(IC<4>{}, IC<6>{}, IC<3>{}, 3);
               else if (events <= 12) goz(IC<4>{}, IC<4>{}, IC<3>{}, 4);
               else if (events <= 16) goz(IC<4>{}, IC<4>{}, IC<4>{}, 4);
               else if (events <= 24) goz(IC<4>{}, IC<2>{}, IC<3>{}, 8);
@@ -3525,34 +3921,6 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
               hipLaunchKernelGGL((k_wgrad16<T>), dim3(blocks1d(slices16, chunks)), dim3(C16_LANES, nw), 0, st,
                                  static_cast<const T*>(x), pk, part, index, events, g, tpb, slices16, vs16);
             }
-          } else if (CAR && KK == 2 && bf && (events == 2 || (events >= 5 && events <= 16) ||
-                                               (events >= 19 && events <= 32))) {
-            // 4 slots on row lanes (k_wgrad_rows), update groups per block measured per event
-            // count at the XL shape: 2 for E = 2 and 5-6, 4 for 7-16, 8 for 19-32
-            const int G = events <= 6 ? 2 : events <= 16 ? 4 : 8;
-            const int slr = (g.C + 127) / 128;
-            auto gorows = [&](auto na) {
-              constexpr int NA = decltype(na)::value;
-              chunks = whole_rounds(slr, max_chunks,
-                                    resident_blocks(reinterpret_cast<const void*>(&k_wgrad_rows<NA>), 256, 0));
-              const int tpr = int((int64_t(g.M) + chunks - 1) / chunks);
-              if (tpr > 0) chunks = int((int64_t(g.M) + tpr - 1) / tpr);  // no chunk past the last token
-              hipLaunchKernelGGL((k_wgrad_rows<NA>), dim3(blocks1d(slr, chunks)), dim3(16, G, 16 / G), 0, st,
-                                 reinterpret_cast<const bf16_t*>(x), pk, part, index, events, g, tpr, slr);
-            };
-            switch ((events + G - 1) / G) {
-              case 1: gorows(IC<1>{}); break;
-              case 2: gorows(IC<2>{}); break;
-              case 3: gorows(IC<3>{}); break;
-              case 4: gorows(IC<4>{}); break;
-              default: return fail(SIHC_ERR_INVALID, "%s: internal weight-gradient shape", what);
-            }
-          } else if (CAR && KK == 2 && bf && SIHC_WGZ_K2 && events >= 2) {
-            // 4 slots, 3-4 and 17-18 events (one event keeps its direct kernel): E = 3 4 x 1
-            // 201 us (k_wgrad: 504), E = 17-18 6 x 3 558-573 us (k_wgrad: 933-941; row lanes
-            // 579-592)
-            if (events <= 4) goz(IC<2>{}, IC<1>{}, IC<1>{}, 4);  // idle waves only stage
-            else goz(IC<2>{}, IC<1>{}, IC<3>{}, (events + 2) / 3);
           } else if (!CAR && !SD && bf && events == 2) {
             // gamma gradient of 2 updates: the pipelined kernel on one-slot rows (1 wave x 2
             // updates: 77 us at 65,536 rows x 1152 channels; row lanes 81)
@@ -3634,6 +4002,32 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
   });
   if (rc) return rc;
   return launch_finalize(what, part, out, nullptr, chunks, events, S, g.C, false, 0, out_dtype, st);
+}
+
+// Backward of the read (MM_READ: x, the E output gradients z, alpha -> grad_x, dalpha) or of
+// the write (MM_WRITE: x = grad_out, the E updates z, beta -> the E update gradients, dbeta)
+// in one pass over its inputs, for 4-slot cells.
+bool fused_backward(const Geo& g, int events, int max_events, int dtype) {
+  return g.K == 2 && events <= max_events && g.C >= 16 / elem_size(dtype);
+}
+template <int MODE>
+int launch_stage_backward(const char* what, const void* x, const void* const* z, const void* w, void* dx,
+                          void* const* dz, void* dw, int events, const Geo& g, const int32_t* index, int dtype,
+                          int out_dtype, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  const int S = g.K * g.K;
+  const int max_chunks = wgrad_chunks(g.M, events, g.C, g.K);
+  const size_t need = size_t(max_chunks) * events * S * g.C * sizeof(float);
+  if (!workspace || workspace_bytes < need)
+    return fail(SIHC_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", what, need, workspace_bytes);
+  if (!aligned(workspace, 16)) return fail(SIHC_ERR_INVALID, "%s: workspace must be 16-byte aligned", what);
+  MMArgs a{x, pack(z, events), static_cast<float*>(workspace), index, events, g, w, dx, PtrPack{}};
+  if (MODE == MM_WRITE) a.dz = pack(const_cast<const void* const*>(dz), events);
+  int chunks = 0;
+  if (int rc = with_dtype(dtype, [&](auto t) {
+        return launch_mm_k2<decltype(t), MODE>(what, a, max_chunks, &chunks, st);
+      }))
+    return rc;
+  return launch_finalize(what, a.part, dw, nullptr, chunks, events, S, g.C, false, 0, out_dtype, st);
 }
 
 // Vector width of the per-event kernels: registers hold up to 2*S*V weights and 2*S*V
@@ -3900,6 +4294,53 @@ int sihc_weight_grad(const void* x, const void* const* z, void* out, int events,
   if (int rc = check_events(what, events, z)) return rc;
   return launch_wgrad(what, x, z, out, events, g, cell * cell, true, index, dtype, out_dtype, workspace,
                       workspace_bytes, st);
+}
+
+int sihc_read_backward(const void* x, const void* const* grads, const void* alpha, void* grad_x, void* grad_alpha,
+                       int events, int64_t batch, int grid, int cell, int channels, const int32_t* index, int dtype,
+                       int out_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  const char* what = "sihc_read_backward";
+  Geo g;
+  if (int rc = check_geometry(what, batch, grid, cell, channels, &g)) return rc;
+  if (!valid_dtype(dtype) || !valid_dtype(out_dtype)) return fail(SIHC_ERR_INVALID, "%s: bad dtype", what);
+  if (int rc = check_count(what, events)) return rc;
+  if (!grad_alpha) return fail(SIHC_ERR_INVALID, "%s: null output", what);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (g.M == 0) return fill_zero(out_dtype, grad_alpha, int64_t(events) * cell * cell * channels, st, what);
+  if (!x || !alpha || !grad_x) return fail(SIHC_ERR_INVALID, "%s: null tensor", what);
+  if (int rc = check_events(what, events, grads)) return rc;
+  if (fused_backward(g, events, 24, dtype))
+    return launch_stage_backward<MM_READ>(what, x, grads, alpha, grad_x, nullptr, grad_alpha, events, g, index, dtype,
+                                          out_dtype, workspace, workspace_bytes, st);
+  if (int rc = sihc_weight_grad(x, grads, grad_alpha, events, batch, grid, cell, channels, index, dtype, out_dtype,
+                                workspace, workspace_bytes, stream))
+    return rc;
+  return sihc_write(nullptr, grads, alpha, grad_x, events, batch, grid, cell, channels, 0, index, dtype, dtype,
+                    stream);
+}
+
+int sihc_write_backward(const void* grad_out, const void* const* updates, const void* beta, void* const* grad_updates,
+                        void* grad_beta, int events, int64_t batch, int grid, int cell, int channels,
+                        const int32_t* index, int dtype, int out_dtype, void* workspace, size_t workspace_bytes,
+                        void* stream) {
+  const char* what = "sihc_write_backward";
+  Geo g;
+  if (int rc = check_geometry(what, batch, grid, cell, channels, &g)) return rc;
+  if (!valid_dtype(dtype) || !valid_dtype(out_dtype)) return fail(SIHC_ERR_INVALID, "%s: bad dtype", what);
+  if (int rc = check_count(what, events)) return rc;
+  if (!grad_beta) return fail(SIHC_ERR_INVALID, "%s: null output", what);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (g.M == 0) return fill_zero(out_dtype, grad_beta, int64_t(events) * cell * cell * channels, st, what);
+  if (!grad_out || !beta) return fail(SIHC_ERR_INVALID, "%s: null tensor", what);
+  if (int rc = check_events(what, events, updates)) return rc;
+  if (int rc = check_events(what, events, const_cast<const void* const*>(grad_updates))) return rc;
+  if (fused_backward(g, events, 8, dtype))
+    return launch_stage_backward<MM_WRITE>(what, grad_out, updates, beta, nullptr, grad_updates, grad_beta, events, g,
+                                           index, dtype, out_dtype, workspace, workspace_bytes, st);
+  if (int rc = sihc_weight_grad(grad_out, updates, grad_beta, events, batch, grid, cell, channels, index, dtype,
+                                out_dtype, workspace, workspace_bytes, stream))
+    return rc;
+  return sihc_read(grad_out, beta, grad_updates, events, batch, grid, cell, channels, index, dtype, stream);
 }
 
 int sihc_triangular(const void* base, const void* const* updates, const void* gamma, void* out, int active,

@@ -10,7 +10,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().with_name("libsihc_hip.so")
-ABI_VERSION = 5
+ABI_VERSION = 6
 MAX_EVENTS = 32
 DTYPE_F32 = 0
 DTYPE_BF16 = 1
@@ -29,6 +29,10 @@ PROTOTYPES: dict[str, tuple] = {
     "sihc_write": (_i32, [_vp, _vpp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp, _i32, _i32, _vp]),
     "sihc_weight_grad_workspace_size": (_sz, [_i32, _i64, _i32, _i32, _i32]),
     "sihc_weight_grad": (_i32, [_vp, _vpp, _vp, _i32, _i64, _i32, _i32, _i32, _vp, _i32, _i32, _vp, _sz, _vp]),
+    "sihc_read_backward": (_i32, [_vp, _vpp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp, _i32, _i32,
+                                  _vp, _sz, _vp]),
+    "sihc_write_backward": (_i32, [_vp, _vpp, _vp, _vpp, _vp, _i32, _i64, _i32, _i32, _i32, _vp, _i32, _i32,
+                                   _vp, _sz, _vp]),
     "sihc_triangular": (_i32, [_vp, _vpp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp]),
     "sihc_triangular_gamma_grad_workspace_size": (_sz, [_i32, _i64, _i32]),
     "sihc_triangular_gamma_grad": (_i32, [_vp, _vpp, _vp, _i32, _i64, _i32, _i32, _i32, _vp, _sz, _vp]),

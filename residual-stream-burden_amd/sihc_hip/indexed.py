@@ -106,6 +106,31 @@ def _indexed_weight_grad_fake(x, updates, weights, index):
     return weights.new_empty((len(updates), weights.shape[1], weights.shape[2]))
 
 
+@custom_op("sihc::indexed_read_backward", mutates_args=())
+def _indexed_read_grads(x: Tensor, grads: list[Tensor], alpha: Tensor, index: Tensor) -> tuple[Tensor, Tensor]:
+    _validate_updates(x, alpha, grads)
+    _same_device(index, x)
+    return launch.read_backward(x, grads, alpha, index=index)
+
+
+@_indexed_read_grads.register_fake
+def _indexed_read_grads_fake(x, grads, alpha, index):
+    return torch.empty_like(x), torch.empty_like(alpha)
+
+
+@custom_op("sihc::indexed_write_backward", mutates_args=())
+def _indexed_write_grads(grad: Tensor, updates: list[Tensor], beta: Tensor,
+                         index: Tensor) -> tuple[list[Tensor], Tensor]:
+    _validate_updates(grad, beta, updates)
+    _same_device(index, grad)
+    return launch.write_backward(grad, updates, beta, index=index)
+
+
+@_indexed_write_grads.register_fake
+def _indexed_write_grads_fake(grad, updates, beta, index):
+    return [torch.empty_like(u) for u in updates], torch.empty_like(beta)
+
+
 def _iread_setup(ctx, inputs, output):
     ctx.save_for_backward(*inputs)
 
@@ -114,7 +139,7 @@ def _iread_backward(ctx, grads):
     x, alpha, index = ctx.saved_tensors
     shape = (x.shape[0], x.shape[1] * x.shape[2] // alpha.shape[2], x.shape[3])
     gs = [g.contiguous() if g is not None else x.new_zeros(shape) for g in grads]
-    return (_indexed_write_impl(x, gs, alpha, index, False), _indexed_weight_grad(x, gs, alpha, index), None)
+    return (*_indexed_read_grads(x, gs, alpha, index), None)
 
 
 register_autograd(_indexed_read, _iread_backward, setup_context=_iread_setup)
@@ -138,7 +163,9 @@ def _iwrite_setup(ctx, inputs, output):
 def _iwrite_backward(ctx, grad):
     beta, index, *updates = ctx.saved_tensors
     grad = grad.contiguous()
-    return grad, _indexed_read(grad, beta, index), _indexed_weight_grad(grad, updates, beta, index), None
+    if torch.is_grad_enabled():  # create_graph: the read keeps its own autograd rule
+        return grad, _indexed_read(grad, beta, index), _indexed_weight_grad(grad, updates, beta, index), None
+    return (grad, *_indexed_write_grads(grad, updates, beta, index), None)
 
 
 register_autograd(_indexed_write, _iwrite_backward, setup_context=_iwrite_setup)

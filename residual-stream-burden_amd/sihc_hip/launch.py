@@ -113,6 +113,40 @@ def weight_grad(x: Tensor, updates: Sequence[Tensor], weights: Optional[Tensor],
 
 
 @_on_tensor_device
+def read_backward(x: Tensor, grads: Sequence[Tensor], alpha: Tensor, index: Optional[Tensor] = None,
+                  out_dtype: Optional[torch.dtype] = None) -> tuple[Tensor, Tensor]:
+    """Adjoint of `read`: (dx, dalpha [E,C,S]); dalpha in out_dtype (default alpha's dtype)."""
+    b, g, k, c = carrier_geometry(x, alpha.shape[2])
+    events = len(grads)
+    dx = torch.empty_like(x)
+    da = torch.empty((events, c, k * k), device=x.device, dtype=out_dtype or alpha.dtype)
+    L = lib()
+    ws = _workspace(L.sihc_weight_grad_workspace_size(events, b, g, k, c), x.device)
+    check(L.sihc_read_backward(x.data_ptr(), ptr_array(t.data_ptr() for t in grads), alpha.data_ptr(), dx.data_ptr(),
+                               da.data_ptr(), events, b, g, k, c, _ptr(index), dtype_code(x.dtype),
+                               dtype_code(da.dtype), ws.data_ptr(), ws.numel() * 4, _stream(x.device)))
+    return dx, da
+
+
+@_on_tensor_device
+def write_backward(grad: Tensor, updates: Sequence[Tensor], beta: Tensor, index: Optional[Tensor] = None,
+                   out_dtype: Optional[torch.dtype] = None) -> tuple[list[Tensor], Tensor]:
+    """Adjoint of `write` except the identity to x: (update gradients, dbeta [E,C,S]); dbeta in
+    out_dtype (default beta's dtype)."""
+    b, g, k, c = carrier_geometry(grad, beta.shape[2])
+    events = len(updates)
+    ddz = [torch.empty((b, g * g, c), device=grad.device, dtype=grad.dtype) for _ in range(events)]
+    db = torch.empty((events, c, k * k), device=grad.device, dtype=out_dtype or beta.dtype)
+    L = lib()
+    ws = _workspace(L.sihc_weight_grad_workspace_size(events, b, g, k, c), grad.device)
+    check(L.sihc_write_backward(grad.data_ptr(), ptr_array(u.data_ptr() for u in updates), beta.data_ptr(),
+                                ptr_array(d.data_ptr() for d in ddz), db.data_ptr(), events, b, g, k, c, _ptr(index),
+                                dtype_code(grad.dtype), dtype_code(db.dtype), ws.data_ptr(), ws.numel() * 4,
+                                _stream(grad.device)))
+    return ddz, db
+
+
+@_on_tensor_device
 def triangular(base: Tensor, updates: Sequence[Tensor], gamma: Tensor) -> Tensor:
     """base + sum_j gamma[j] * updates_j over a [B,N,C] workspace."""
     c = base.shape[-1]
@@ -260,7 +294,8 @@ def copy_(dst: Tensor, src: Tensor) -> Tensor:
 
 
 __all__ = [
-    "MAX_EVENTS", "dtype_code", "carrier_geometry", "read", "write", "weight_grad", "triangular",
+    "MAX_EVENTS", "dtype_code", "carrier_geometry", "read", "write", "weight_grad", "read_backward",
+    "write_backward", "triangular",
     "triangular_gamma_grad", "triangular_backward", "event_forward", "event_backward", "gather_cells",
     "scatter_cells", "scatter_add_cells", "copy_",
 ]

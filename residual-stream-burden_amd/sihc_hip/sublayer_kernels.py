@@ -88,6 +88,22 @@ def _weights_backward(x: Tensor, updates: list[Tensor], weights: Tensor) -> Tens
     return launch.weight_grad(x, updates, weights)
 
 
+@custom_op("sihc::sublayer_read_backward", mutates_args=())
+def _read_grads(x: Tensor, grads: list[Tensor], alpha: Tensor) -> tuple[Tensor, Tensor]:
+    """(dx, dalpha) of the read from one pass over x and the output gradients: the values of
+    `_write_impl(x, grads, alpha, False)` and `_weights_backward(x, grads, alpha)`."""
+    _validate_updates(x, alpha, grads)
+    return launch.read_backward(x, grads, alpha)
+
+
+@custom_op("sihc::sublayer_write_backward", mutates_args=())
+def _write_grads(grad: Tensor, updates: list[Tensor], beta: Tensor) -> tuple[list[Tensor], Tensor]:
+    """(update gradients, dbeta) of the write: the values of `sublayer_read(grad, beta)` and
+    `_weights_backward(grad, updates, beta)`, from one pass for up to 8 events."""
+    _validate_updates(grad, beta, updates)
+    return launch.write_backward(grad, updates, beta)
+
+
 def _read_setup(ctx, inputs, output):
     ctx.save_for_backward(*inputs)
 
@@ -104,8 +120,7 @@ def _read_backward(ctx, grads):
         a = alpha
     else:
         a = alpha[used].contiguous()
-    dx = _write_impl(x, gs, a, False)
-    da_used = _weights_backward(x, gs, a)
+    dx, da_used = _read_grads(x, gs, a)
     if len(used) == alpha.shape[0]:
         return dx, da_used
     da = alpha.new_zeros(alpha.shape)
@@ -132,7 +147,9 @@ def _write_backward(ctx, grad):
     updates, and the weight reduction for beta."""
     beta, *updates = ctx.saved_tensors
     grad = grad.contiguous()
-    return grad, sublayer_read(grad, beta), _weights_backward(grad, updates, beta)
+    if torch.is_grad_enabled():  # create_graph: the read keeps its own autograd rule
+        return grad, sublayer_read(grad, beta), _weights_backward(grad, updates, beta)
+    return grad, *_write_grads(grad, updates, beta)
 
 
 register_autograd(sublayer_write, _write_backward, setup_context=_write_setup)
@@ -244,6 +261,18 @@ def _weight_fake(x, updates, weights):
     return torch.empty_like(weights)
 
 
+@_read_grads.register_fake
+def _read_grads_fake(x, grads, alpha):
+    _validate_updates(x, alpha, grads)
+    return torch.empty_like(x), torch.empty_like(alpha)
+
+
+@_write_grads.register_fake
+def _write_grads_fake(grad, updates, beta):
+    _validate_updates(grad, beta, updates)
+    return [torch.empty_like(u) for u in updates], torch.empty_like(beta)
+
+
 @sublayer_triangular.register_fake
 def _tri_fake(base, updates, gamma):
     _validate_triangular(base, updates, gamma)
@@ -263,4 +292,4 @@ def _tri_backward_fake(grad, updates, gamma):
 
 
 __all__ = ["sublayer_read", "sublayer_write", "sublayer_triangular", "_write_impl", "COMPILED_TRIANGULAR_BACKWARD",
-           "_weights_backward", "_tri_gamma_backward", "_tri_backward", "_require_packed", "_geometry"]
+           "_weights_backward", "_read_grads", "_write_grads", "_tri_gamma_backward", "_tri_backward", "_require_packed", "_geometry"]
