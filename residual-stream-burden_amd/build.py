@@ -1,4 +1,5 @@
-"""Build libsihc_hip.so (HIP kernels + C ABI) for gfx950 with hipcc, in-tree.
+"""Build libsihc_hip.so (HIP kernels + C ABI) for gfx950 with hipcc, and the native eager
+dispatch _sihc_torch.so (C++ against the installed torch), in-tree.
 
 Usage: python residual-stream-burden_amd/build.py [--verbose]
 
@@ -20,6 +21,8 @@ SOURCES = [PKG_ROOT / "csrc" / "sihc_kernels.hip"]
 OUTPUT = PKG_ROOT / "sihc_hip" / "libsihc_hip.so"
 SELFTEST_SOURCE = PKG_ROOT / "csrc" / "abi_selftest.c"
 SELFTEST = PKG_ROOT / "sihc_hip" / "sihc_abi_selftest"
+NATIVE_SOURCE = PKG_ROOT / "csrc" / "sihc_torch.cpp"
+NATIVE = PKG_ROOT / "sihc_hip" / "_sihc_torch.so"
 ARCH = "gfx950"
 
 
@@ -61,6 +64,29 @@ def selftest_command(output: Path = SELFTEST) -> list[str]:
     ]
 
 
+def native_command(output: Path = NATIVE) -> list[str]:
+    """The C++ dispatch of the eager ops, linked against torch and the library next to it."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    torch_lib = str(Path(torch.__file__).resolve().parent / "lib")
+    flags: list[str] = []
+    for inc in (*include_paths(), sysconfig.get_paths()["include"], os.path.join(rocm, "include")):
+        flags += ["-isystem", inc]
+    return [
+        shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+        "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+        "-I", str(REPO_ROOT / "include"), *flags, str(NATIVE_SOURCE),
+        "-L", str(OUTPUT.parent), "-lsihc_hip",
+        "-L", torch_lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python",
+        "-Wl,-rpath,$ORIGIN", "-o", str(output),
+    ]
+
+
 def _run(cmd: list[str], verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -76,14 +102,17 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile the library and the C-ABI self-test (always; atomically replaces an
-    existing build)."""
+    """Compile the library, the C-ABI self-test and the native dispatch (always; atomically
+    replaces an existing build)."""
     tmp = OUTPUT.with_suffix(".so.tmp")
     _run(command(tmp), verbose)
     os.replace(tmp, OUTPUT)
     tmp = SELFTEST.with_name(SELFTEST.name + ".tmp")
     _run(selftest_command(tmp), verbose)
     os.replace(tmp, SELFTEST)
+    tmp = NATIVE.with_suffix(".so.tmp")
+    _run(native_command(tmp), verbose)
+    os.replace(tmp, NATIVE)
     return OUTPUT
 
 

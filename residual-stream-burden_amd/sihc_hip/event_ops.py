@@ -26,6 +26,7 @@ from torch import Tensor
 from torch.library import custom_op, register_autograd
 
 from . import launch
+from ._native import native
 from .sublayer_kernels import _require_packed, sublayer_read, sublayer_write
 
 
@@ -94,6 +95,7 @@ def _event_autograd(ctx, grad_x_out, grad_z_out):
 
 
 register_autograd(event_write_read, _event_autograd, setup_context=_event_setup)
+native(event_write_read, "event_write_read")
 
 
 def literal_stage(x0: Tensor, alpha: Tensor, beta: Tensor,

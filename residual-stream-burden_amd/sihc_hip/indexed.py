@@ -31,6 +31,7 @@ from torch import Tensor
 from torch.library import custom_op, register_autograd
 
 from . import launch
+from ._native import native
 from .sublayer_kernels import _geometry, _require_packed, _validate_updates
 
 
@@ -143,6 +144,7 @@ def _iread_backward(ctx, grads):
 
 
 register_autograd(_indexed_read, _iread_backward, setup_context=_iread_setup)
+native(_indexed_read, "indexed_read")
 
 
 @custom_op("sihc::indexed_write", mutates_args=())
@@ -169,6 +171,7 @@ def _iwrite_backward(ctx, grad):
 
 
 register_autograd(_indexed_write, _iwrite_backward, setup_context=_iwrite_setup)
+native(_indexed_write, "indexed_write")
 
 
 @custom_op("sihc::gather_cells", mutates_args=())
@@ -229,7 +232,9 @@ def _scatter_backward(ctx, grad):
 
 
 register_autograd(_gather_cells, _gather_backward, setup_context=_gather_setup)
+native(_gather_cells, "gather_cells")
 register_autograd(_scatter_cells, _scatter_backward, setup_context=_scatter_setup)
+native(_scatter_cells, "scatter_cells")
 
 
 def _carrier_grid(x: Tensor, slots: int) -> tuple[int, int]:

@@ -27,7 +27,8 @@ from torch import Tensor
 from torch.library import custom_op, register_autograd
 
 from . import launch
-from .sublayer_kernels import _read_backward, _read_setup, _require_packed
+from ._native import native
+from .sublayer_kernels import _read_backward, _read_setup, _require_packed, _write_grads
 
 # tag -> (carrier edge, cell edge, blocks)
 GEOMETRY = {"b4_12": (64, 4, 12), "b4_8": (64, 4, 8), "p8_12": (32, 2, 12)}
@@ -113,6 +114,15 @@ def _make_all_base(tag: str):
     # without stacking them first (reference :2285-2292 stacks, then runs the two
     # kernels above).
     register_autograd(split, _read_backward, setup_context=_read_setup)
+
+    def of_this_stage(read):
+        def entry(x0, alpha, *rest):
+            fits = not rest and isinstance(x0, Tensor) and isinstance(alpha, Tensor) and x0.ndim == 4 \
+                and x0.shape[1] == edge and alpha.ndim == 3 and alpha.shape[0] == blocks and alpha.shape[2] == slots
+            return read(x0, alpha) if fits else NotImplemented
+        return entry
+
+    native(split, "sublayer_read", of_this_stage)
     return split, grad_x, grad_alpha
 
 
@@ -194,11 +204,16 @@ def _make_final_accumulate(tag: str):
         saved = ctx.saved_tensors
         dzs, betas = saved[:blocks], saved[blocks:]
         grad_out = grad_out.contiguous()
+        if dzs[0].dtype == grad_out.dtype and not torch.is_grad_enabled():
+            # one pass, the weight gradients reduced in fp32 and stored in the betas' dtype
+            gdz, gbeta = _write_grads(grad_out, list(dzs), torch.stack(betas))
+            return (grad_out, *gdz, *gbeta.unbind(0))
         gdz = grad_dz(grad_out, *betas)
         gbeta = grad_beta(grad_out, *dzs)
         return (grad_out, *gdz.unbind(0), *(g.to(b.dtype) for g, b in zip(gbeta.unbind(0), betas)))
 
     register_autograd(fa, backward, setup_context=setup)
+    native(fa, "block_write", lambda entry: lambda *args: entry(edge, blocks, slots, *args))
     return fa, grad_dz, grad_beta
 
 

@@ -18,6 +18,7 @@ from torch import Tensor
 from torch.library import custom_op, register_autograd
 
 from . import launch
+from ._native import native
 
 MAX_EVENTS = launch.MAX_EVENTS
 
@@ -129,6 +130,7 @@ def _read_backward(ctx, grads):
 
 
 register_autograd(sublayer_read, _read_backward, setup_context=_read_setup)
+native(sublayer_read, "sublayer_read")
 
 
 @custom_op("sihc::sublayer_write", mutates_args=())
@@ -153,6 +155,7 @@ def _write_backward(ctx, grad):
 
 
 register_autograd(sublayer_write, _write_backward, setup_context=_write_setup)
+native(sublayer_write, "sublayer_write")
 
 
 def _validate_triangular(base: Tensor, updates: list[Tensor], gamma: Tensor) -> None:
@@ -231,6 +234,7 @@ def _tri_autograd(ctx, grad):
 
 
 register_autograd(sublayer_triangular, _tri_autograd, setup_context=_tri_setup)
+native(sublayer_triangular, "sublayer_triangular")
 
 
 # Fake implementations (reference :387-416): device-free shape functions for fullgraph

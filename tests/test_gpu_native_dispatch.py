@@ -1,0 +1,226 @@
+"""GPU: the native eager entries of the custom ops against the registered Python ops.
+
+A plain call takes the C++ node (its grad_fn says so) and gives the Python op's bits, forward
+and backward. What a registered op lets other machinery see is still seen: dispatch and
+function modes, vmap, forward-mode tangents, create_graph, saved-tensor hooks, tensor
+subclasses, no_grad and inference mode, version checks; what it refuses is still refused.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from sihc_hip import indexed as ix
+from sihc_hip import kernels as legacy
+from sihc_hip import sublayer_kernels as sk
+from sihc_hip.event_ops import event_write_read
+
+pytestmark = pytest.mark.gpu
+
+B, G, C, E = 2, 16, 24, 3
+
+
+def _t(*shape, dtype=torch.float32, grad=True):
+    return torch.randn(*shape, device="cuda").to(dtype).requires_grad_(grad)
+
+
+def _calls(dtype):
+    """name -> (op, arguments with lists in place, the registered op of the same arguments)"""
+    torch.manual_seed(1)
+    x, dz = _t(B, 2 * G, 2 * G, C, dtype=dtype), [_t(B, G * G, C, dtype=dtype) for _ in range(12)]
+    w, idx = _t(E, C, 4, dtype=dtype), ix.group_index(B, G, 5, 2).cuda()
+    ops = torch.ops.sihc
+    return {
+        "read": (sk.sublayer_read, (x, w), ops.sublayer_read),
+        "write": (sk.sublayer_write, (x, dz[:E], w), ops.sublayer_write),
+        "triangular": (sk.sublayer_triangular, (dz[0], dz[1:4], _t(3, C)), ops.sublayer_triangular),
+        "event": (event_write_read, (x, dz[0], _t(C, 4, dtype=dtype), _t(C, 4, dtype=dtype)), ops.event_write_read),
+        "indexed_read": (ix._indexed_read, (x, w, idx), ops.indexed_read),
+        "indexed_write": (ix._indexed_write, (x, dz[:E], w, idx), ops.indexed_write),
+        "gather": (ix._gather_cells, (x, idx, 4), ops.gather_cells),
+        "scatter": (ix._scatter_cells, (_t(B, G * G, 4, C, dtype=dtype), idx), ops.scatter_cells),
+        "all_base": (legacy.all_base_p8_12_split_traceable, (x, _t(12, C, 4, dtype=dtype)),
+                     ops.all_base_p8_12_split_traceable),
+        "final_accumulate": (legacy.final_accumulate_p8_12_traceable,
+                             (x, *dz, *(_t(C, 4, dtype=dtype) for _ in range(12))),
+                             ops.final_accumulate_p8_12_traceable),
+    }
+
+
+NAMES = ["read", "write", "triangular", "event", "indexed_read", "indexed_write", "gather", "scatter", "all_base",
+         "final_accumulate"]
+
+
+def _flat(v):
+    return [t for a in v for t in (_flat(a) if isinstance(a, (list, tuple)) else [a])]
+
+
+def _leaves(args):
+    return [t for t in _flat(args) if isinstance(t, torch.Tensor) and t.requires_grad]
+
+
+def _outs(r):
+    return _flat([r])
+
+
+def _grads(out, args, seed=3):
+    torch.manual_seed(seed)
+    up = [torch.randn_like(o) for o in out]
+    return torch.autograd.grad(out, _leaves(args), up)
+
+
+def _is_native(t):
+    return "Fn" in type(t.grad_fn).__name__ + t.grad_fn.name() and "GeneratedBackward" not in type(t.grad_fn).__name__
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("name", NAMES)
+def test_same_bits_as_the_registered_op(name, dtype):
+    op, args, registered = _calls(dtype)[name]
+    out, want = op(*args), registered(*args)
+    assert type(out) is type(want)
+    out, want = _outs(out), _outs(want)
+    assert _is_native(out[0]) and not _is_native(want[0])
+    assert all(torch.equal(a, b) for a, b in zip(out, want))
+    for a, b in zip(_grads(out, args), _grads(want, args)):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+    # an unused output's gradient is zeros for both
+    a, b = (torch.autograd.grad(_outs(f(*args))[0].float().square().sum(), _leaves(args), allow_unused=True)
+            for f in (op, registered))
+    assert all((p is None and q is None) or torch.equal(p, q) for p, q in zip(a, b))
+    with torch.no_grad():
+        r = _outs(op(*args))
+        assert r[0].grad_fn is None and all(torch.equal(p, q) for p, q in zip(r, want))
+    with torch.inference_mode():
+        r = _outs(op(*args))
+        assert r[0].is_inference() and all(torch.equal(p, q) for p, q in zip(r, want))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_modes_and_transforms_still_see_the_op(name):
+    op, args, _ = _calls(torch.float32)[name]
+
+    class Count(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, a=(), kw=None):
+            self.seen += str(func).startswith("sihc.")
+            return func(*a, **(kw or {}))
+
+    with Count() as m:
+        out = _outs(op(*args))
+    assert m.seen >= 1 and not _is_native(out[0])
+
+    class Functions(torch.overrides.TorchFunctionMode):
+        seen = 0
+
+        def __torch_function__(self, func, types, a=(), kw=None):
+            self.seen += "sihc" in str(func)
+            return func(*a, **(kw or {}))
+
+    with Functions() as f:
+        op(*args)
+    assert f.seen >= 1
+
+
+def test_backward_under_a_mode_calls_the_registered_ops():
+    op, args, _ = _calls(torch.float32)["event"]
+    out = op(*args)
+    assert _is_native(out[0])
+    seen = []
+
+    class Log(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, a=(), kw=None):
+            seen.append(str(func))
+            return func(*a, **(kw or {}))
+
+    want = _grads(out, args)
+    out = op(*args)
+    with Log():
+        got = _grads(out, args)
+    assert any("event_write_read_backward" in s for s in seen)  # engine threads carry the caller's modes
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_create_graph_keeps_the_differentiable_rule_of_the_write():
+    op, (x, dz, beta), registered = _calls(torch.float32)["write"]
+    second = []
+    for f in (op, registered):
+        v = torch.ones_like(x, requires_grad=True)
+        (g,) = torch.autograd.grad(f(x, dz, beta), dz[:1], v, create_graph=True)
+        second.append(torch.autograd.grad(g.square().sum(), (v, beta)))
+    assert all(torch.equal(a, b) for a, b in zip(*second))
+
+
+def test_saved_tensor_hooks_and_version_checks():
+    for name in ("read", "write", "event", "triangular"):
+        op, args, _ = _calls(torch.float32)[name]
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t.clone(), lambda t: t):
+            out = _outs(op(*args))
+        assert _is_native(out[0]) and len(packed) >= 2
+        _grads(out, args)
+    op, (x, w), _ = _calls(torch.float32)["read"]
+    out = op(x, w)
+    with torch.no_grad():
+        w.add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        _grads(out, (x, w))
+
+
+def test_vmap_forward_mode_and_subclasses_take_the_registered_op():
+    op, args, registered = _calls(torch.float32)["event"]
+    x, *rest = (t.detach() for t in args)
+    got = torch.func.vmap(lambda a: op(a, *rest))(torch.stack([x, 2 * x]))
+    assert all(torch.equal(a[1], b) for a, b in zip(got, registered(2 * x, *rest)))
+    op, (x, w), registered = _calls(torch.float32)["read"]
+    import torch.autograd.forward_ad as fw
+    with fw.dual_level():
+        out = op(fw.make_dual(x.detach(), torch.ones_like(x)), w.detach())
+        assert torch.equal(out[0], registered(x.detach(), w.detach())[0])
+
+    class Sub(torch.Tensor):
+        pass
+
+    out = op(x.detach().as_subclass(Sub), w.detach())
+    assert isinstance(out[0], Sub)
+    out = op(x, torch.nn.Parameter(w.detach()))
+    assert _is_native(out[0])
+
+
+def test_refusals_are_unchanged():
+    op, (x, w), _ = _calls(torch.float32)["read"]
+    with pytest.raises(ValueError, match="contiguous"):
+        op(x.transpose(1, 2), w)
+    with pytest.raises(ValueError, match="share CUDA device and dtype"):
+        op(x, w.bfloat16())
+    with pytest.raises(ValueError, match="1..32 events"):
+        op(x, w[:, :5].contiguous())
+    _, (base, dz, gamma), _ = _calls(torch.float32)["triangular"]
+    with pytest.raises(ValueError, match="active updates"):
+        sk.sublayer_triangular(base, [dz[0], dz[1][:, :4].contiguous(), dz[2]], gamma)
+
+
+def test_keywords_other_streams_and_capture():
+    op, args, _ = _calls(torch.bfloat16)["event"]
+    x, dz, beta, alpha = (t.detach() for t in args)
+    want = op(x, dz, beta, alpha)
+    got = op(x=x, dz=dz, beta=beta, alpha_next=alpha)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        out = op(*args)
+        grads = _grads(out, args)
+    s.synchronize()
+    ref = _grads(op(*args), args)
+    assert all(torch.equal(a, b) for a, b in zip(grads, ref))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = op(x, dz, beta, alpha)
+    for k in range(3):
+        x.mul_(0.5)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(captured, op(x, dz, beta, alpha)))
