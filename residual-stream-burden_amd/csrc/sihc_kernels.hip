@@ -96,7 +96,7 @@
 #define SIHC_EV_GROUP 32
 #endif
 #ifndef SIHC_EV_GROUP_K4  // the same for 16-slot cells
-#define SIHC_EV_GROUP_K4 64
+#define SIHC_EV_GROUP_K4 8  // 32,768 tokens x 1152: 8 705 us, 16 717, 32 746, 64 788
 #endif
 #ifndef SIHC_EV_BWD_NT  // non-temporal hints in the per-event backward: 1 loads, 2 stores, 3 both
 #define SIHC_EV_BWD_NT 3
@@ -462,6 +462,16 @@ __device__ __forceinline__ void slice_chunk_unless8(int blk, int nslices, int& s
   chunk = blk / nslices;
   const int r = blk - chunk * nslices;
   slice = (nslices & 7) == 0 ? r : (r + chunk) % nslices;
+}
+
+// Block order of the 16-slot per-event kernels over n blocks: the hardware's, with the slice
+// rotated by the chunk, so that the 8 XCDs stream through one window of tokens (with an
+// XCD-contiguous order each has a window of its own: 32,768 tokens x 1152 bf16, backward
+// 764 -> 726 us, forward 452 -> 443; 16,384 tokens, forward 228 -> 215; fp32 backward 743 ->
+// 702); but XCD-contiguous for slice rows narrower than a 128-byte line, whose neighbours
+// share lines (2,048 x 768, 64-byte rows: 70 us in the hardware order, 63 in this one).
+__device__ __forceinline__ int event16_block(int row_bytes, int n) {
+  return row_bytes < 128 ? logical_block_of<true>(n) : int(blockIdx.x);
 }
 
 // Carrier pixel of slot 0 of the cell token m reads/writes. Token m = b*GG + n owns
@@ -2647,7 +2657,8 @@ __global__ void __launch_bounds__(SIHC_EV_FWD_THREADS, SIHC_EV_MINW) k_event_fwd
   constexpr int K = 4, S = 16, V = 2;
   constexpr int U = SIHC_EV_UNROLL;  // tokens per lane per iteration
   const int BCG = blockDim.x, TL = blockDim.y;
-  const int blk = logical_block<true>(), slice = blk % nslices, chunk = blk / nslices;
+  int slice, chunk;
+  slice_chunk(event16_block(BCG * V * 2, int(gridDim.x)), nslices, slice, chunk);
   const int c0 = (slice * BCG + threadIdx.x) * V;
   if (c0 >= g.C) return;
   uint32_t bw[16], aw[16];  // word v * 8 + p: channel c0 + v, slots 2p, 2p + 1
@@ -2780,9 +2791,8 @@ __global__ void __launch_bounds__(256, SIHC_EV_MINW) k_event_bwd(const T* __rest
   if (run_carry<T>(carry, S, g.C, red)) return;
   const int BCG = blockDim.x, TL = blockDim.y;
   const int BC = BCG * V;
-  const int blk = logical_block_of<K == 4>(carry.nmain);
   int slice, chunk;
-  slice_chunk(blk, nslices, slice, chunk);
+  slice_chunk(K == 4 ? event16_block(BC * int(sizeof(T)), carry.nmain) : int(blockIdx.x), nslices, slice, chunk);
   const int c0 = slice * BC + threadIdx.x * V;
   float db[S][V], da[S][V];
 #pragma unroll
@@ -2950,7 +2960,8 @@ __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_
   if (run_carry<bf16_t>(carry, S, g.C, red)) return;
   const int BCG = blockDim.x, TL = blockDim.y;
   const int BC = BCG * V;
-  const int blk = logical_block_of<true>(carry.nmain), slice = blk % nslices, chunk = blk / nslices;
+  int slice, chunk;
+  slice_chunk(event16_block(BC * 2, carry.nmain), nslices, slice, chunk);
   const int c0 = slice * BC + threadIdx.x * V;
   float db[S][V], da[S][V];
 #pragma unroll
@@ -3364,22 +3375,37 @@ Shape2D shape_for(int C, int V, int bcg0, int lds_per_channel, int lds_cap = 64 
 // into LDS; with 16-slot cells that staging is large enough that blocks must cover more
 // tokens as E grows (measured at batch 256, D 1152: E = 24 read 1872 -> 1624 us with
 // 64 tokens per lane, while E = 1 is fastest with 8).
-int rw_tokens_per_lane(int cell, int events, bool read = false, bool dot2_read = false) {
+int rw_tokens_per_lane(int cell, int events, bool read, bool dot2) {
   // 4-slot reads: 32-token blocks (64 with one event) stream through a narrower window
   // than 128-token ones (E = 2..16: 6-7% faster)
   // 4-slot writes: 4 tokens per lane from 4 events (XL shape: E = 8 426 -> 417 us, E = 16
   // 655 -> 647, E = 24 889 -> 883; fewer events measured the same as with 8)
   if (cell == 2) return read ? (events == 1 ? 4 : 2) : (events >= 4 ? 4 : SIHC_RW_TPT);
-  // 16-slot bf16 reads on k_read_d2 (packed weights, cheap to stage): short blocks past 12
-  // events (XL shape: E = 16 957 -> 929 us with 8 tokens, E = 24 1251 -> 1206 us with 16,
-  // E = 32 2210 -> 2078; 3-12 events do not care)
-  if (dot2_read && events > 12) return events <= 16 ? 8 : 16;
+  if (dot2) {
+    // 16-slot bf16 on k_read_d2 / k_write_d2, whose packed weights are cheap to stage: reads 8
+    // tokens and 16 past 16 events, writes 16 and 32 past 16 (32,768 tokens x 1152: read E = 12
+    // 432 us with 32 tokens, 420 with 8; write E = 12 662 with 32, 645 with 16; E = 24 907 with
+    // 64, 861 with 32; 8,192 x 768: read E = 8 71 with 32, 65 with 8; write E = 24 302 with 64,
+    // 192 with 32, 157 with 16, where the grid rule below lands)
+    if (read) return events <= 16 ? 8 : 16;
+    return events <= 4 ? 8 : events <= 16 ? 16 : 32;
+  }
   // 16 slots: the weight slice staged per block grows with E, so blocks grow too; with
   // hinted loads and stores reads with 3-12 events and writes with 9-12 gain from twice
   // the tokens again (read E = 8: 794 -> 745 us), 1-2 and 13+ events do not
   if (read && events >= 3 && events <= 12) return events <= 4 ? 16 : 32;
   if (!read && events > 8 && events <= 12) return 32;
   return events <= 4 ? SIHC_RW_TPT : events <= 16 ? 16 : 64;
+}
+// The same for a launch of M tokens in blocks of tl token lanes x `slices` slices: halved, down
+// to one iteration of `unroll` tokens, while the grid holds fewer than three blocks per CU
+// (1,024 tokens x 768, 16 slots, E = 12: read 58 -> 32 us, write 88 -> 26).
+int device_cus();
+int rw_tokens(int cell, int events, bool read, bool dot2, int unroll, int64_t M, int tl, int slices) {
+  int t = rw_tokens_per_lane(cell, events, read, dot2);
+  const int64_t blocks = 3 * int64_t(std::max(device_cus(), 1));
+  while (t / 2 >= unroll && ((M + tl * t - 1) / (tl * t)) * slices < blocks) t /= 2;
+  return t;
 }
 
 int chunk_count(int64_t M, int tokens_per_chunk, int max_chunks) {
@@ -4127,7 +4153,8 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
   const Shape2D sh = cell == 2 ? shape_for(channels, V, SIHC_RW_BCG, events * S * wbytes)
                                : shape_for(channels, V, events <= 8 ? 64 : SIHC_RW_BCG_K4, events * S * wbytes,
                                            SIHC_RW_LDS_K4);  // 64 lanes to 8 events: E = 4 569 -> 542 us
-  const int tpb = sh.tl * rw_tokens_per_lane(cell, events, true, d2 && V == 2);
+  const int unroll = d2 ? SIHC_RD2_U : cell == 2 ? SIHC_RW_UNROLL : SIHC_RW_UNROLL_K4;
+  const int tpb = sh.tl * rw_tokens(cell, events, true, d2, unroll, g.M, sh.tl, sh.slices);
   const int64_t chunks = (int64_t(g.M) + tpb - 1) / tpb;
   const int gs = tpb;  // one contiguous run per block (interleaved groups measured no faster)
   const size_t lds = size_t(events) * S * sh.bcg * V * wbytes;
@@ -4212,7 +4239,8 @@ int sihc_write(const void* x, const void* const* updates, const void* beta, void
   const Shape2D sh = cell == 2 ? shape_for(channels, V, SIHC_RW_BCG, E4 * S * wbytes)
                                : shape_for(channels, V, E4 <= 8 ? 64 : SIHC_RW_BCG_K4, E4 * S * wbytes,
                                            SIHC_RW_LDS_K4);  // 64 lanes to 8 events: E = 4 1010 -> 964 us
-  const int tpb = sh.tl * rw_tokens_per_lane(cell, E4);
+  const int unroll = d2 ? SIHC_WR2_U : cell == 2 ? SIHC_RW_UNROLL : SIHC_RW_UNROLL_K4;
+  const int tpb = sh.tl * rw_tokens(cell, E4, false, d2, unroll, g.M, sh.tl, sh.slices);
   const int64_t chunks = (int64_t(g.M) + tpb - 1) / tpb;
   const int gs = tpb;  // one contiguous run per block (interleaved groups measured no faster)
   const size_t lds = size_t(E4) * S * sh.bcg * V * wbytes;
@@ -4592,7 +4620,18 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
   while (V > 1 && ((beta && !aligned(beta, std::min(16, V * S * es))) ||
                    (has_g && !aligned(alpha_next, std::min(16, V * S * es)))))
     V /= 2;
-  const Shape2D sh = shape_for(channels, V, SIHC_EV_BCG, 0);
+  // Channel lanes per block: 32; 16 for 16-byte fp32 lanes (256-byte rows, 65,536 tokens x
+  // 1152: 823 -> 798 us, 8,192 x 768: 79.5 -> 73.6); 64 for 16-slot bf16, whose 4-byte lanes
+  // else stream 128-byte pieces, where they leave a block per CU (32,768 x 1152: 726 -> 705,
+  // 8,192 x 1024: 190 -> 178; 8,192 x 768, 192 blocks: 141 -> 152). With less than a block on
+  // every other CU narrower slices, whose blocks take more tokens at a time (16 slots, 2,048 x
+  // 768: 76 -> 63 us, 256 x 768: 57 -> 37; 4,096 x 768, 192 blocks: 84 -> 118).
+  const int64_t cus = std::max(device_cus(), 1);
+  auto blocks_with = [&](int bcg) { return int64_t(max_chunks) * shape_for(channels, V, bcg, 0).slices; };
+  int lanes = cell == 2 && V * es == 16 ? 16 : SIHC_EV_BCG;
+  if (cell == 4 && es == 2 && V == 2 && blocks_with(64) >= cus) lanes = 64;
+  while (lanes > 4 && blocks_with(lanes) < cus / 2) lanes /= 2;
+  const Shape2D sh = shape_for(channels, V, lanes, 0);
   const size_t lds = size_t(sh.tl) * sh.bcg * S * V * sizeof(float);  // TL x (BCG*S*V) floats
   if (carry && (sh.tl * sh.bcg != 256 || lds < FINALIZE_LDS(4) * sizeof(float)))
     return fail(SIHC_ERR_INVALID, "%s: internal block shape of the carried finalize", what);

@@ -321,3 +321,33 @@ def test_chained_finalize_rejects_overlapping_workspaces():
         _run_partial(L, "chain", cases[0], c, k, _lib.DTYPE_BF16, other, slot(1),
                      (p(work), work.numel() * 4, slot(0), p(got[2]), p(got[3])), st, reuse=got)
     torch.cuda.synchronize()
+
+
+# Launch shapes of the backward: (slots, dtype, batch, grid, channels) for 64 channel lanes per
+# block with a partial last slice, 32, 16 (fp32 vectors), and 16, 8 and 4 where few chunks
+# leave the device idle.
+SHAPES = [(16, torch.bfloat16, 128, 16, 136), (16, torch.bfloat16, 16, 16, 264), (16, torch.bfloat16, 8, 16, 520),
+          (16, torch.bfloat16, 4, 16, 200), (16, torch.bfloat16, 1, 16, 136), (16, torch.float32, 4, 13, 136),
+          (4, torch.float32, 8, 16, 328), (4, torch.bfloat16, 1, 16, 264), (4, torch.float32, 1, 3, 7)]
+
+
+@pytest.mark.parametrize("slots,dtype,batch,grid,channels", SHAPES,
+                         ids=[f"s{s}-{str(d)[6:]}-b{b}-g{g}-c{c}" for s, d, b, g, c in SHAPES])
+def test_event_backward_launch_shapes(slots, dtype, batch, grid, channels):
+    announce(f"event bwd shapes dtype={dtype} slots={slots} b={batch} g={grid} C={channels}")
+    gen = torch.Generator().manual_seed(channels + batch)
+    k = O.cell_edge(slots)
+
+    def draw(*shape, mean=0.0, std=1.0):
+        return (mean + std * torch.randn(*shape, generator=gen)).to(dtype)
+
+    xo, gx = draw(batch, k * grid, k * grid, channels), draw(batch, k * grid, k * grid, channels, std=0.1)
+    dz, gz = draw(batch, grid * grid, channels), draw(batch, grid * grid, channels, std=0.1)
+    beta, alpha = draw(channels, slots, mean=1.0, std=0.02), draw(channels, slots, mean=1 / slots, std=0.02)
+    got = launch.event_backward(*(t.cuda() for t in (gx, gz, xo, dz, beta, alpha)))
+    want = O.event_backward(gx, gz, xo, dz, beta, alpha)
+    for name, a, b, kind in zip(("dX", "ddz", "dbeta", "dalpha"), got, want, ("elementwise",) * 2 + ("reduced",) * 2):
+        assert_parity(a, b.to(dtype), dtype, what=name, kind=kind)
+    index = torch.arange(grid * grid, dtype=torch.int32).repeat(batch, 1).cuda()
+    again = launch.event_backward(*(t.cuda() for t in (gx, gz, xo, dz, beta, alpha)), index=index)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
