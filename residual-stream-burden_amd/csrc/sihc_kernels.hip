@@ -272,6 +272,11 @@ template <> struct RawT<2> { using type = uint16_t; };
 // triangular with 7+ updates); hinted loads without hinted stores slow the balanced
 // streams down (1-3%); slices narrower than a 128-byte line take no hint (16-slot
 // read/write with 16+ events: 7-60% slower).
+// First channel of the lane whose vector nominally starts at channel cb of a C-wide row: the
+// last vector of a row that V does not divide is moved back to end with the row, so its first
+// channels are computed twice, with the same result, by two lanes. Lanes with cb >= C are idle.
+__device__ __forceinline__ int lane_channel(int cb, int V, int C) { return min(cb, C - V); }
+
 template <bool NT = false, typename R>
 __device__ __forceinline__ R ld(const R* p) {
   if constexpr (NT) {
@@ -293,6 +298,31 @@ __device__ __forceinline__ void st(R* p, R v) {
   }
 }
 
+// BYTES of a row at p. Rows of any width start at any element, so these promise only the
+// alignment of the element; the instruction is the same wide load or store (gfx950 takes
+// global accesses at any byte address), and an aligned row costs nothing.
+template <int BYTES, bool NT = false, typename T>
+__device__ __forceinline__ typename RawT<BYTES>::type ld_row(const T* p) {
+  typedef typename RawT<BYTES>::type R;
+  typedef R RU __attribute__((aligned(sizeof(T))));
+  if constexpr (NT) {
+    return __builtin_nontemporal_load(reinterpret_cast<const RU*>(p));
+  } else {
+    return *reinterpret_cast<const RU*>(p);
+  }
+}
+template <int BYTES, bool NT = false, typename T>
+__device__ __forceinline__ void st_row(T* p, typename RawT<BYTES>::type v) {
+  typedef typename RawT<BYTES>::type R;
+  typedef R RU __attribute__((aligned(sizeof(T))));
+  if constexpr (NT) {
+    asm volatile("" : "+v"(v));  // as in st()
+    __builtin_nontemporal_store(v, reinterpret_cast<RU*>(p));
+  } else {
+    *reinterpret_cast<RU*>(p) = v;
+  }
+}
+
 template <typename T, int V, bool NT = false>
 __device__ __forceinline__ void load_vec(const T* __restrict__ p, float* o) {
   constexpr int BYTES = V * int(sizeof(T));
@@ -301,7 +331,7 @@ __device__ __forceinline__ void load_vec(const T* __restrict__ p, float* o) {
   using R = typename RawT<CH>::type;
 #pragma unroll
   for (int q = 0; q < BYTES / CH; ++q) {
-    R r = ld<NT>(reinterpret_cast<const R*>(p) + q);
+    const R r = ld_row<CH, NT>(p + q * EPC);
     T e[EPC];
     __builtin_memcpy(e, &r, CH);
 #pragma unroll
@@ -322,7 +352,7 @@ __device__ __forceinline__ void store_vec(T* __restrict__ p, const float* v) {
     for (int i = 0; i < EPC; ++i) e[i] = from_f32<T>(v[q * EPC + i]);
     R r;
     __builtin_memcpy(&r, e, CH);
-    st<NT>(reinterpret_cast<R*>(p) + q, r);
+    st_row<CH, NT>(p + q * EPC, r);
   }
 }
 
@@ -335,7 +365,7 @@ __device__ __forceinline__ void load_vec_cached(const T* __restrict__ p, float* 
   using R = typename RawT<CH>::type;
 #pragma unroll
   for (int q = 0; q < BYTES / CH; ++q) {
-    R r = reinterpret_cast<const R*>(p)[q];
+    const R r = ld_row<CH>(p + q * EPC);
     T e[EPC];
     __builtin_memcpy(e, &r, CH);
 #pragma unroll
@@ -356,7 +386,7 @@ template <typename T, int V, bool NT = false>
 __device__ __forceinline__ void load_raw(const T* __restrict__ p, RawVec<T, V>& o) {
   using RV = RawVec<T, V>;
 #pragma unroll
-  for (int q = 0; q < RV::BYTES / RV::CH; ++q) o.r[q] = ld<NT>(reinterpret_cast<const typename RV::R*>(p) + q);
+  for (int q = 0; q < RV::BYTES / RV::CH; ++q) o.r[q] = ld_row<RV::CH, NT>(p + q * (RV::CH / int(sizeof(T))));
 }
 template <typename T, int V>
 __device__ __forceinline__ void raw_to_f32(const RawVec<T, V>& in, float* o) {
@@ -464,14 +494,23 @@ __device__ __forceinline__ void slice_chunk_unless8(int blk, int nslices, int& s
   slice = (nslices & 7) == 0 ? r : (r + chunk) % nslices;
 }
 
-// Block order of the 16-slot per-event kernels over n blocks: the hardware's, with the slice
-// rotated by the chunk, so that the 8 XCDs stream through one window of tokens (with an
-// XCD-contiguous order each has a window of its own: 32,768 tokens x 1152 bf16, backward
-// 764 -> 726 us, forward 452 -> 443; 16,384 tokens, forward 228 -> 215; fp32 backward 743 ->
-// 702); but XCD-contiguous for slice rows narrower than a 128-byte line, whose neighbours
-// share lines (2,048 x 768, 64-byte rows: 70 us in the hardware order, 63 in this one).
-__device__ __forceinline__ int event16_block(int row_bytes, int n) {
-  return row_bytes < 128 ? logical_block_of<true>(n) : int(blockIdx.x);
+// Block order of a kernel whose rows V does not divide (ragged): neighbouring slices share a
+// line at each end of every row piece, so they run on one XCD (contiguous order) and meet in
+// its L2; such launches also carry no non-temporal hints, which would let a shared line go
+// before its second use and write it in two partial pieces. The 16-slot per-event kernels take
+// this order where a slice row is narrower than a line (2,048 tokens x 768, 64-byte rows: 70 us
+// in the hardware's order, 63 in this one), and the hardware's, with the slice rotated, where
+// it is not, so that the 8 XCDs stream through one window of tokens (32,768 x 1152 bf16,
+// backward 764 -> 726 us, forward 452 -> 443; 16,384 tokens, forward 228 -> 215; fp32 backward
+// 743 -> 702).
+__device__ __forceinline__ void slice_chunk_row(int n, int nslices, bool ragged, int& slice, int& chunk) {
+  if (ragged) {
+    const int blk = logical_block_of<true>(n);
+    chunk = blk / nslices;
+    slice = blk - chunk * nslices;
+  } else {
+    slice_chunk(int(blockIdx.x), nslices, slice, chunk);
+  }
 }
 
 // Carrier pixel of slot 0 of the cell token m reads/writes. Token m = b*GG + n owns
@@ -527,9 +566,9 @@ __device__ __forceinline__ void stage_weights(float* lds, const TW* __restrict__
     const int r = i - e * BC * S;
     const int cl = r / S;
     const int s = r - cl * S;
-    const int c = cs + cl;
-    const int cg = cl / V;
-    lds[lds_w<V>(e * S + s, cg, cl - cg * V, BCG)] = (e < E && c < C) ? to_f32(w[(int64_t(e) * C + c) * S + s]) : 0.f;
+    const int cg = cl / V, cb = cs + cg * V;
+    const int c = lane_channel(cb, V, C) + (cl - cg * V);
+    lds[lds_w<V>(e * S + s, cg, cl - cg * V, BCG)] = (e < E && cb < C) ? to_f32(w[(int64_t(e) * C + c) * S + s]) : 0.f;
   }
   __syncthreads();
 }
@@ -551,10 +590,10 @@ __device__ __forceinline__ void stage_weights_bf16(uint32_t* lds, const bf16_t* 
     const int r = i - e * BP * S;
     const int pr = r / S;
     const int s = r - pr * S;
-    const int c = cs + 2 * pr;
-    const uint32_t lo = (e < E && c < C) ? uint32_t(w[(int64_t(e) * C + c) * S + s]) : 0u;
-    const uint32_t hi = (e < E && c + 1 < C) ? uint32_t(w[(int64_t(e) * C + c + 1) * S + s]) : 0u;
-    const int cg = pr / NW, q = pr - cg * NW;
+    const int cg = pr / NW, q = pr - cg * NW, cb = cs + cg * V;
+    const int c = lane_channel(cb, V, C) + 2 * q;
+    const uint32_t lo = (e < E && cb < C) ? uint32_t(w[(int64_t(e) * C + c) * S + s]) : 0u;
+    const uint32_t hi = (e < E && cb < C) ? uint32_t(w[(int64_t(e) * C + c + 1) * S + s]) : 0u;
     lds[((e * S + s) * BCG + cg) * NW + q] = lo | (hi << 16);
   }
   __syncthreads();
@@ -604,8 +643,8 @@ __global__ void __launch_bounds__(256, SIHC_RW_MINW) k_read(const T* __restrict_
   } else {
     stage_weights<V>(lds, alpha, E, E, S, BCG, cs, g.C);
   }
-  const int c0 = cs + threadIdx.x * V;
-  if (c0 >= g.C) return;
+  const int cb = cs + threadIdx.x * V, c0 = lane_channel(cb, V, g.C);
+  if (cb >= g.C) return;
   // The block's tokens: groups of gs tokens (a multiple of U * TL), group `chunk` and
   // every nchunks-th one after it (the launchers pass gs = the block's whole run).
   for (int64_t m0 = int64_t(chunk) * gs; m0 < g.M; m0 += int64_t(nchunks) * gs) {
@@ -682,9 +721,9 @@ __device__ __forceinline__ void stage_read_pairs(uint32_t* lds, const bf16_t* __
     const int e = i / (BC * 8);
     const int r = i - e * BC * 8;
     const int cl = r >> 3, pr = r & 7;
-    const int c = cs + cl;
+    const int cb = cs + (cl & ~1), c = lane_channel(cb, 2, C) + (cl & 1);
     lds[((e * 4 + (pr >> 1)) * BCG + (cl >> 1)) * 4 + (pr & 1) * 2 + (cl & 1)] =
-        c < C ? w[(int64_t(e) * C + c) * 8 + pr] : 0u;
+        cb < C ? w[(int64_t(e) * C + c) * 8 + pr] : 0u;
   }
   __syncthreads();
 }
@@ -710,12 +749,10 @@ __global__ void __launch_bounds__(256, SIHC_RW_MINW) k_read_d2(const bf16_t* __r
   const int cs = slice * BCG * 2;
   stage_read_pairs(reinterpret_cast<uint32_t*>(lds), alpha, E, BCG, cs, g.C);
   const u32x4* wl = reinterpret_cast<const u32x4*>(lds);
-  const int c0 = cs + threadIdx.x * 2;
-  if (c0 >= g.C) return;
-  // slot s of a cell: carrier row s / 4, pixel s % 4 of the cell's 4-pixel run; in words
-  // (2 channels each, C even on this path) a pixel is C / 2 words and a row GK * C / 2
-  const int64_t row_w = int64_t(g.GK) * (g.C >> 1);
-  const int pix_w = g.C >> 1;
+  const int cb = cs + threadIdx.x * 2, c0 = lane_channel(cb, 2, g.C);
+  if (cb >= g.C) return;
+  // slot s of a cell: carrier row s / 4, pixel s % 4 of the cell's 4-pixel run
+  const int64_t row = int64_t(g.GK) * g.C;
   for (int64_t m0 = int64_t(chunk) * gs; m0 < g.M; m0 += int64_t(nchunks) * gs) {
     const int64_t m_end = min(m0 + gs, int64_t(g.M));
     for (int64_t mi = m0; mi < m_end; mi += U * TL) {
@@ -727,12 +764,12 @@ __global__ void __launch_bounds__(256, SIHC_RW_MINW) k_read_d2(const bf16_t* __r
       for (int u = 0; u < U; ++u) {
         ok[u] = m + u * TL < m_end;
         const int mu = int(ok[u] ? m + u * TL : mi);  // tail: reload a valid token, store nothing
-        const uint32_t* px = reinterpret_cast<const uint32_t*>(x + cell_pixel0(mu, g, index) * g.C + c0);
+        const bf16_t* px = x + cell_pixel0(mu, g, index) * g.C + c0;
         zoff[u] = int64_t(mu) * g.C + c0;
 #pragma unroll
         for (int uy = 0; uy < K; ++uy)
 #pragma unroll
-          for (int ux = 0; ux < K; ++ux) xw[u][uy * K + ux] = ld<NTL>(px + uy * row_w + ux * pix_w);
+          for (int ux = 0; ux < K; ++ux) xw[u][uy * K + ux] = ld_row<4, NTL>(px + uy * row + ux * int64_t(g.C));
       }
       load_fence();
       uint32_t xp[U][S / 2][2];  // [token][slot pair][channel]
@@ -798,8 +835,8 @@ __global__ void __launch_bounds__(256, SIHC_RW_MINW) k_write(const TX* __restric
   } else {
     stage_weights<V>(lds, beta, E, E4, S, BCG, cs, g.C);
   }
-  const int c0 = cs + threadIdx.x * V;
-  if (c0 >= g.C) return;
+  const int cb = cs + threadIdx.x * V, c0 = lane_channel(cb, V, g.C);
+  if (cb >= g.C) return;
   // The block's tokens: groups of gs tokens (a multiple of U * TL), group `chunk` and
   // every nchunks-th one after it (the launchers pass gs = the block's whole run).
   for (int64_t m0 = int64_t(chunk) * gs; m0 < g.M; m0 += int64_t(nchunks) * gs) {
@@ -898,9 +935,9 @@ __device__ __forceinline__ void stage_write_pairs(uint32_t* lds, const bf16_t* _
     const int j = i / (BC * 16);
     const int r = i - j * BC * 16;
     const int cl = r >> 4, sl = r & 15;
-    const int c = cs + cl;
+    const int cb = cs + (cl & ~1), c = lane_channel(cb, 2, C) + (cl & 1);
     uint32_t lo = 0u, hi = 0u;
-    if (c < C) {
+    if (cb < C) {
       lo = w[(int64_t(2 * j) * C + c) * 16 + sl];
       if (2 * j + 1 < E) hi = w[(int64_t(2 * j + 1) * C + c) * 16 + sl];
     }
@@ -932,15 +969,10 @@ __global__ void __launch_bounds__(256, SIHC_RW_MINW) k_write_d2(const bf16_t* __
   const int cs = slice * BCG * 2;
   stage_write_pairs(reinterpret_cast<uint32_t*>(lds), beta, E, BCG, cs, g.C);
   const u32x4* wl = reinterpret_cast<const u32x4*>(lds);
-  const int c0 = cs + threadIdx.x * 2;
-  if (c0 >= g.C) return;
+  const int cb = cs + threadIdx.x * 2, c0 = lane_channel(cb, 2, g.C);
+  if (cb >= g.C) return;
   const int J = (E + 1) / 2;
-  // carrier words (2 channels each, C even on this path): a pixel is C / 2 words, a
-  // carrier row GK * C / 2
-  const int64_t row_w = int64_t(g.GK) * (g.C >> 1);
-  const int pix_w = g.C >> 1;
-  const uint32_t* xw = reinterpret_cast<const uint32_t*>(x);
-  uint32_t* ow = reinterpret_cast<uint32_t*>(out);
+  const int64_t row = int64_t(g.GK) * g.C, pix = g.C;  // elements of a carrier row and pixel
   for (int64_t m0 = int64_t(chunk) * gs; m0 < g.M; m0 += int64_t(nchunks) * gs) {
     const int64_t m_end = min(m0 + gs, int64_t(g.M));
     for (int64_t mi = m0; mi < m_end; mi += U * TL) {
@@ -952,14 +984,14 @@ __global__ void __launch_bounds__(256, SIHC_RW_MINW) k_write_d2(const bf16_t* __
       for (int u = 0; u < U; ++u) {
         ok[u] = m + u * TL < m_end;
         const int mu = int(ok[u] ? m + u * TL : mi);  // tail: reload a valid token, store nothing
-        b0[u] = (cell_pixel0(mu, g, index) * g.C + c0) >> 1;
+        b0[u] = cell_pixel0(mu, g, index) * g.C + c0;
         zoff[u] = int64_t(mu) * g.C + c0;
         if constexpr (ADD_X) {
 #pragma unroll
           for (int uy = 0; uy < K; ++uy)
 #pragma unroll
             for (int ux = 0; ux < K; ++ux) {
-              const uint32_t v = ld<NTL>(xw + b0[u] + uy * row_w + ux * pix_w);
+              const uint32_t v = ld_row<4, NTL>(x + b0[u] + uy * row + ux * pix);
               acc[u][uy * K + ux][0] = __uint_as_float(v << 16);
               acc[u][uy * K + ux][1] = __uint_as_float(v & 0xffff0000u);
             }
@@ -974,7 +1006,7 @@ __global__ void __launch_bounds__(256, SIHC_RW_MINW) k_write_d2(const bf16_t* __
         for (int q = 0; q < 2; ++q) {
           const bf16_t* z = static_cast<const bf16_t*>(upd.p[min(2 * j + q, E - 1)]);
 #pragma unroll
-          for (int u = 0; u < U; ++u) zr[q][u] = ld<NTL>(reinterpret_cast<const uint32_t*>(z + zoff[u]));
+          for (int u = 0; u < U; ++u) zr[q][u] = ld_row<4, NTL>(z + zoff[u]);
         }
       };
       issue(0);
@@ -1008,8 +1040,7 @@ __global__ void __launch_bounds__(256, SIHC_RW_MINW) k_write_d2(const bf16_t* __
           for (int uy = 0; uy < K; ++uy)
 #pragma unroll
             for (int ux = 0; ux < K; ++ux)
-              store_vec<bf16_t, 2, NTS>(reinterpret_cast<bf16_t*>(ow + b0[u] + uy * row_w + ux * pix_w),
-                                        acc[u][uy * K + ux]);
+              store_vec<bf16_t, 2, NTS>(out + b0[u] + uy * row + ux * pix, acc[u][uy * K + ux]);
         }
     }
   }
@@ -1049,18 +1080,18 @@ __global__ void __launch_bounds__(256) k_read_w(const bf16_t* __restrict__ x, co
   const uint32_t* aw = reinterpret_cast<const uint32_t*>(alpha);
   for (int i = tid; i < E * BC * 2; i += 256) {
     const int e = i / (BC * 2), r = i - e * BC * 2, cl = r >> 1, pr = r & 1;
-    const int c = cs + cl;
-    ap[(e * 2 + pr) * BC + cl] = c < g.C ? aw[(int64_t(e) * g.C + c) * 2 + pr] : 0u;
+    const int cb = cs + cl / V * V, c = lane_channel(cb, V, g.C) + cl % V;
+    ap[(e * 2 + pr) * BC + cl] = cb < g.C ? aw[(int64_t(e) * g.C + c) * 2 + pr] : 0u;
   }
   // cell tile: unit u = (token t, channel group j): 4 slot vectors of 8 channels ->
   // 8 pair words per slot pair
   for (int u = tid; u < RDW_TT * LX; u += 256) {
-    const int t = u / LX, j = u % LX, c = cs + j * V;
-    if (t < tn && c < g.C) {
+    const int t = u / LX, j = u % LX, cb = cs + j * V, c = lane_channel(cb, V, g.C);
+    if (t < tn && cb < g.C) {
       const int64_t p0 = cell_pixel0(m0 + t, g, index);
       u32x4 v[4];
 #pragma unroll
-      for (int sl = 0; sl < 4; ++sl) v[sl] = ld<NTL>(reinterpret_cast<const u32x4*>(x + slot_offset<K>(p0, sl, g, c)));
+      for (int sl = 0; sl < 4; ++sl) v[sl] = ld_row<16, NTL>(x + slot_offset<K>(p0, sl, g, c));
 #pragma unroll
       for (int pr = 0; pr < 2; ++pr) {
         const u32x4 a = v[2 * pr], b = v[2 * pr + 1];
@@ -1080,8 +1111,8 @@ __global__ void __launch_bounds__(256) k_read_w(const bf16_t* __restrict__ x, co
     }
   }
   __syncthreads();
-  const int c0 = cs + lx * V;
-  if (c0 >= g.C) return;  // no barrier below
+  const int cb0 = cs + lx * V, c0 = lane_channel(cb0, V, g.C);
+  if (cb0 >= g.C) return;  // no barrier below
   for (int e = wave; e < E; e += 4) {
     const u32x4* ae = reinterpret_cast<const u32x4*>(ap + e * 2 * BC + lx * V);
     const u32x4 w00 = ae[0], w01 = ae[1];                       // pair 0, channels 0..3, 4..7
@@ -1157,8 +1188,8 @@ __global__ void __launch_bounds__(256) k_wgrad(const T* __restrict__ x, PtrPack 
   const int cg = threadIdx.x;
   // event lanes past E (padding to whole 4-wave blocks) only help stage the tile
   const int e = min(int(threadIdx.y), E - 1);
-  const int c0 = cs + cg * V;
-  const bool active = c0 < g.C && int(threadIdx.y) < E;
+  const int c0 = lane_channel(cs + cg * V, V, g.C);
+  const bool active = cs + cg * V < g.C && int(threadIdx.y) < E;
   const T* __restrict__ ze = static_cast<const T*>(z.p[e]);
   const int tid = threadIdx.y * BCG + threadIdx.x;
   const int nthr = BCG * blockDim.y;
@@ -1194,9 +1225,9 @@ __global__ void __launch_bounds__(256) k_wgrad(const T* __restrict__ x, PtrPack 
         const int t = row / S;
         const int ss = row - t * S;
         const int m = t0 + t;
-        const int ci = cs + cgi * V;
+        const int cbi = cs + cgi * V, ci = lane_channel(cbi, V, g.C);
         dst[q] = i < nvec ? row * BCG + cgi : -1;
-        if (m < m_end && ci < g.C) {
+        if (m < m_end && cbi < g.C) {
           int64_t off;
           if constexpr (CARRIER) {
             off = slot_offset<K>(cell_pixel0(m, g, index), ss, g, ci);
@@ -1284,30 +1315,29 @@ __global__ void __launch_bounds__(256) k_wgrad(const T* __restrict__ x, PtrPack 
 #ifndef SIHC_TRIB_MINB    // occupancy hint of k_trib_waves (blocks per CU)
 #define SIHC_TRIB_MINB 1
 #endif
-template <typename T, int V, bool ONE>
+template <typename T, int V, bool ONE, bool NT>
 __global__ void __launch_bounds__(256, SIHC_TRIB_MINB) k_trib_waves(const T* __restrict__ grad, PtrPack z, float* __restrict__ part,
                                                     int E, Geo g, int tpb, int nslices, PtrPack dout,
                                                     const void* __restrict__ gam, int gam_f32) {
   constexpr int LX = 16, RY = 4, BC = LX * V, RPL = TRIB_TT / RY;  // rows per lane per sub-tile
-  constexpr bool NTL = true, NTS = true;
+  constexpr bool NTL = NT, NTS = NT;
   extern __shared__ float lds[];
   float* gt = lds;                 // [TRIB_TT][BC] gradient rows
   float* gm = lds + TRIB_TT * BC;  // [E][BC] gamma slice
   const int NW = int(blockDim.x) / 64;
-  const int blk = int(blockIdx.x);
   int slice, chunk;
-  slice_chunk(blk, nslices, slice, chunk);
+  slice_chunk_row(int(gridDim.x), nslices, !NT, slice, chunk);
   const int cs = slice * BC;
   const int tid = int(threadIdx.x), wave = tid / 64, lane = tid % 64;
   const int lx = lane % LX, ly = lane / LX;
-  const int c0 = cs + lx * V;
-  const bool cok = c0 < g.C;  // the host guarantees C % V == 0: a lane is all in or all out
+  const int c0 = NT ? cs + lx * V : lane_channel(cs + lx * V, V, g.C);  // NT: V divides the width
+  const bool cok = cs + lx * V < g.C;
   const int m_begin = chunk * tpb;
   const int m_end = min(m_begin + tpb, g.M);
   // gamma slice, once per block
   for (int i = tid; i < E * BC; i += blockDim.x) {
-    const int e = i / BC, c = cs + (i - e * BC);
-    const int64_t gi = int64_t(e) * g.C + min(c, g.C - 1);
+    const int e = i / BC, cl = i - e * BC;
+    const int64_t gi = int64_t(e) * g.C + lane_channel(cs + cl / V * V, V, g.C) + cl % V;
     gm[i] = gam_f32 ? static_cast<const float*>(gam)[gi] : to_f32(static_cast<const bf16_t*>(gam)[gi]);
   }
   constexpr int NK = ONE ? 1 : TRIB_MAXK;  // accumulator sets held across sub-tiles
@@ -1340,9 +1370,9 @@ __global__ void __launch_bounds__(256, SIHC_TRIB_MINB) k_trib_waves(const T* __r
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int i = min(i0 + q * int(blockDim.x), tn * LX - 1);
-        const int row = i / LX, c = cs + (i - row * LX) * V;
-        if (c < g.C) {
-          load_vec<T, V, NTL>(grad + int64_t(s0 + row) * g.C + c, gv[q]);
+        const int row = i / LX, cb = cs + (i - row * LX) * V;
+        if (cb < g.C) {
+          load_vec<T, V, NTL>(grad + int64_t(s0 + row) * g.C + lane_channel(cb, V, g.C), gv[q]);
         } else {
 #pragma unroll
           for (int v = 0; v < V; ++v) gv[q][v] = 0.f;
@@ -1439,8 +1469,8 @@ __global__ void __launch_bounds__(256) k_wgrad_direct(const T* __restrict__ x, P
   // plain order: rotated, one event at D = 1152 ran 136.5 -> 139.9 us (1024: 130.9 -> 125.7)
   const int blk = logical_block<false>(), slice = blk % nslices, chunk = blk / nslices;
   const int e = threadIdx.y;
-  const int c0 = (slice * blockDim.x + threadIdx.x) * V;
-  if (c0 >= g.C) return;  // no barriers below
+  const int cb = (slice * blockDim.x + threadIdx.x) * V, c0 = lane_channel(cb, V, g.C);
+  if (cb >= g.C) return;  // no barriers below
   const T* __restrict__ ze = static_cast<const T*>(z.p[e]);
   float acc[S][V];
 #pragma unroll
@@ -1894,8 +1924,8 @@ __global__ void __launch_bounds__(512, SIHC_C16Z_MINW) k_wgradz_d2(const bf16_t*
 }
 
 // ----------------------------------------------------------------------------------
-// γ gradient partials on 16-byte row lanes (bf16, 3..32 updates, C % 8 == 0, 16-byte
-// aligned rows): part[chunk][j][c] = sum over the chunk's tokens m of g[m,c] * u_j[m,c].
+// γ gradient partials on 16-byte row lanes (bf16, 3..32 updates, and 2 where the rows are not
+// whole aligned vectors; at least 8 channels): part[chunk][j][c] = sum over the chunk's tokens m of g[m,c] * u_j[m,c].
 // A read-only mix of 1 + A workspace rows. A block is 16 lanes of 8 channels (a 128-channel
 // slice) x G update groups x 16 / G token rows (256 threads). Group y takes updates
 // y*NA .. y*NA + NA - 1 (past A: the last update again, never written). Every thread
@@ -1908,7 +1938,7 @@ __global__ void __launch_bounds__(512, SIHC_C16Z_MINW) k_wgradz_d2(const bf16_t*
 // ascending row order through LDS, one update at a time; each chunk's sum has a fixed
 // order, so the result is bitwise repeatable.
 // ----------------------------------------------------------------------------------
-template <int NA>
+template <int NA, bool NT>
 __global__ void __launch_bounds__(256) k_gamma_rows(const bf16_t* __restrict__ grad, PtrPack z,
                                                     float* __restrict__ part, int A, int M, int C, int tpb,
                                                     int nslices) {
@@ -1916,26 +1946,25 @@ __global__ void __launch_bounds__(256) k_gamma_rows(const bf16_t* __restrict__ g
   const int lx = int(threadIdx.x), gy = int(threadIdx.y), r = int(threadIdx.z);
   const int G = int(blockDim.y), TR = int(blockDim.z);
   int slice, chunk;
-  slice_chunk(int(blockIdx.x), nslices, slice, chunk);
-  const int c0 = slice * 128 + lx * 8;
+  slice_chunk_row(int(gridDim.x), nslices, !NT, slice, chunk);
+  const int cb = slice * 128 + lx * 8, c0 = lane_channel(cb, 8, C);
   const int j0 = gy * NA;
   float acc[NA][8];
 #pragma unroll
   for (int q = 0; q < NA; ++q)
 #pragma unroll
     for (int k = 0; k < 8; ++k) acc[q][k] = 0.f;
-  if (c0 < C) {
+  if (cb < C) {
     const int m_end = min(chunk * tpb + tpb, M);
-    const u32x4* up[NA];
+    const bf16_t* up[NA];
 #pragma unroll
-    for (int q = 0; q < NA; ++q) up[q] = static_cast<const u32x4*>(z.p[min(j0 + q, A - 1)]);
-    const u32x4* gp = reinterpret_cast<const u32x4*>(grad);
+    for (int q = 0; q < NA; ++q) up[q] = static_cast<const bf16_t*>(z.p[min(j0 + q, A - 1)]);
     for (int m = chunk * tpb + r; m < m_end; m += TR) {
-      const int64_t o = (int64_t(m) * C + c0) >> 3;  // 16-byte vector index
-      const u32x4 gv = ld<true>(gp + o);
+      const int64_t o = int64_t(m) * C + c0;
+      const u32x4 gv = ld_row<16, NT>(grad + o);
       u32x4 uv[NA];
 #pragma unroll
-      for (int q = 0; q < NA; ++q) uv[q] = ld<true>(up[q] + o);
+      for (int q = 0; q < NA; ++q) uv[q] = ld_row<16, NT>(up[q] + o);
       load_fence();
       // the gradient's 8 values first, then update by update (this order sets the register
       // allocation, and with it the occupancy the group table was measured at: 4 waves per
@@ -1966,8 +1995,8 @@ __global__ void __launch_bounds__(256) k_gamma_rows(const bf16_t* __restrict__ g
       const int gi = i >> 7, cl = i & 127;
       float sum = 0.f;
       for (int rr = 0; rr < TR; ++rr) sum += red[(rr * G + gi) * 128 + cl];
-      const int j = gi * NA + q, c = slice * 128 + cl;
-      if (j < A && c < C) part[(int64_t(chunk) * A + j) * C + c] = sum;
+      const int j = gi * NA + q, cbl = slice * 128 + (cl & ~7);
+      if (j < A && cbl < C) part[(int64_t(chunk) * A + j) * C + lane_channel(cbl, 8, C) + (cl & 7)] = sum;
     }
     __syncthreads();
   }
@@ -2021,12 +2050,10 @@ struct MMRow {  // VC channels of one row as the words a load returns
   static constexpr int NW = VC * int(sizeof(T)) / 4;
   uint32_t w[NW];
 };
-template <typename T, int VC>
+template <bool NT, typename T, int VC>
 __device__ __forceinline__ void mm_load(const T* p, MMRow<T, VC>& r) {
-  typedef typename RawT<VC * int(sizeof(T))>::type R;
-  typedef R RU __attribute__((aligned(sizeof(T))));  // any element alignment
-  const R v = __builtin_nontemporal_load(reinterpret_cast<const RU*>(p));
-  __builtin_memcpy(r.w, &v, sizeof(R));
+  const auto v = ld_row<VC * int(sizeof(T)), NT>(p);
+  __builtin_memcpy(r.w, &v, sizeof(v));
 }
 // acc[v] += the 4x4 products of rows a (tokens x the lane's slot) and b (tokens x its event)
 template <int VC>
@@ -2055,18 +2082,6 @@ __device__ __forceinline__ void mm_acc(const MMRow<float, VC> (&a)[4], const MMR
                                                   0, 0);
 }
 
-template <typename T, int VC>
-__device__ __forceinline__ void mm_store(T* p, const float (&v)[VC]) {
-  typedef typename RawT<VC * int(sizeof(T))>::type R;
-  typedef R RU __attribute__((aligned(sizeof(T))));
-  T e[VC];
-#pragma unroll
-  for (int i = 0; i < VC; ++i) e[i] = from_f32<T>(v[i]);
-  R r;
-  __builtin_memcpy(&r, e, sizeof(R));
-  asm volatile("" : "+v"(r));  // as in st(): keeps the non-temporal hint
-  __builtin_nontemporal_store(r, reinterpret_cast<RU*>(p));
-}
 // Transpose the 4 x 4 words that a quad of lanes holds (lane q, word t -> lane t, word q)
 // with two exchanges inside the quad (DPP quad permutes).
 __device__ __forceinline__ void quad_transpose(uint32_t& r0, uint32_t& r1, uint32_t& r2, uint32_t& r3, int q) {
@@ -2127,7 +2142,7 @@ constexpr int MM_WRITE = 2;  // backward of the write: also dz_e[m,c] = sum_s w[
 template <typename T, int VC>
 constexpr int MM_WG = 64 * VC * 4 * int(sizeof(T)) / 4;
 
-template <typename T, int K, int SGW, int EGW, int VC, int MODE>
+template <typename T, int K, int SGW, int EGW, int VC, int MODE, bool NT>
 __global__ void __launch_bounds__(256) k_wgrad_mm(const T* __restrict__ x, PtrPack z, float* __restrict__ part,
                                                   const int32_t* __restrict__ index, int E, Geo g, int gs,
                                                   int nchunks, int nslices, int wt, int segs,
@@ -2141,7 +2156,11 @@ __global__ void __launch_bounds__(256) k_wgrad_mm(const T* __restrict__ x, PtrPa
   const int tw = wave % wt, pw = wave / wt;                    // token wave, part
   const int sg0 = (pw % segs) * SGW, eg0 = (pw / segs) * EGW;  // this part's first slot / event group
   int slice, chunk;
-  slice_chunk_unless8(int(blockIdx.x), nslices, slice, chunk);
+  if constexpr (NT) {
+    slice_chunk_unless8(int(blockIdx.x), nslices, slice, chunk);
+  } else {
+    slice_chunk_row(int(gridDim.x), nslices, true, slice, chunk);
+  }
   const int cb = (slice * 16 + b) * VC;
   const int c0 = min(cb, g.C - VC);
   if constexpr (MODE != MM_GRAD) {
@@ -2202,11 +2221,11 @@ __global__ void __launch_bounds__(256) k_wgrad_mm(const T* __restrict__ x, PtrPa
 #pragma unroll
       for (int sg = 0; sg < SGW; ++sg)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) mm_load<T, VC>(xp[sg] + p1[t], xn[sg][t]);
+        for (int t = 0; t < 4; ++t) mm_load<NT, T, VC>(xp[sg] + p1[t], xn[sg][t]);
     };
     auto load_z = [&](int eg) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) mm_load<T, VC>(zp[eg] + z1[t], zr[eg][t]);
+      for (int t = 0; t < 4; ++t) mm_load<NT, T, VC>(zp[eg] + z1[t], zr[eg][t]);
     };
     // one iteration: the current 4 tokens (tn of them real); with MORE, the next ones' loads
     auto step = [&](int tn, auto more) {
@@ -2273,7 +2292,7 @@ __global__ void __launch_bounds__(256) k_wgrad_mm(const T* __restrict__ x, PtrPa
             float o[VC];
 #pragma unroll
             for (int v = 0; v < VC; ++v) o[v] = d[v][t];
-            if (real && t < tn) mm_store<T, VC>(dzp[eg] + zo[t], o);
+            if (real && t < tn) store_vec<T, VC, NT>(dzp[eg] + zo[t], o);
           }
         }
       }
@@ -2283,7 +2302,7 @@ __global__ void __launch_bounds__(256) k_wgrad_mm(const T* __restrict__ x, PtrPa
           float o[VC];
 #pragma unroll
           for (int v = 0; v < VC; ++v) o[v] = d[v][t];
-          if (t < tn) mm_store<T, VC>(dxp + p0[t], o);
+          if (t < tn) store_vec<T, VC, NT>(dxp + p0[t], o);
         }
       }
     };
@@ -2509,22 +2528,22 @@ __global__ void __launch_bounds__(256) k_triangular(const T* __restrict__ base, 
   extern __shared__ float lds[];
   const int BCG = blockDim.x, TL = blockDim.y;
   const int BC = BCG * V;
-  const int blk = logical_block<false>();
   int slice, chunk;
-  slice_chunk(blk, nslices, slice, chunk);
+  constexpr bool RAG = NTM == 0;  // only rows that V does not divide are launched without hints
+  slice_chunk_row(int(gridDim.x), nslices, RAG, slice, chunk);
   const int cs = slice * BC;
   const int A4 = (A + 3) & ~3;
   const int tid = threadIdx.y * BCG + threadIdx.x;
   for (int i = tid; i < A4 * BC; i += BCG * TL) {
     const int j = i / BC;
     const int cl = i - j * BC;
-    const int c = cs + cl;
-    const int cg = cl / V;
-    lds[lds_w<V>(j, cg, cl - cg * V, BCG)] = (j < A && c < C) ? to_f32(gamma[int64_t(j) * C + c]) : 0.f;
+    const int cg = cl / V, cbl = cs + cg * V;
+    const int c = lane_channel(cbl, V, C) + (cl - cg * V);
+    lds[lds_w<V>(j, cg, cl - cg * V, BCG)] = (j < A && cbl < C) ? to_f32(gamma[int64_t(j) * C + c]) : 0.f;
   }
   __syncthreads();
-  const int c0 = cs + threadIdx.x * V;
-  if (c0 >= C) return;
+  const int cb = cs + threadIdx.x * V, c0 = RAG ? lane_channel(cb, V, C) : cb;
+  if (cb >= C) return;
   // The block's tokens: groups of gs tokens (a multiple of U * TL), group `chunk` and
   // every nchunks-th one after it (the launchers pass gs = the block's whole run).
   for (int64_t m0 = int64_t(chunk) * gs; m0 < M; m0 += int64_t(nchunks) * gs) {
@@ -2594,11 +2613,10 @@ __global__ void __launch_bounds__(SIHC_EV_FWD_THREADS, SIHC_EV_MINW) k_event_fwd
   constexpr int S = K * K;
   constexpr int U = SIHC_EV_UNROLL;  // tokens per lane per iteration
   const int BCG = blockDim.x, TL = blockDim.y;
-  const int blk = logical_block<K == 4>();
   int slice, chunk;
-  slice_chunk(blk, nslices, slice, chunk);
-  const int c0 = (slice * BCG + threadIdx.x) * V;
-  if (c0 >= g.C) return;
+  slice_chunk_row(int(gridDim.x), nslices, K == 4 || !NTL, slice, chunk);
+  const int cb = (slice * BCG + threadIdx.x) * V, c0 = lane_channel(cb, V, g.C);
+  if (cb >= g.C) return;
   float bw[S][V], aw[S][V];
   load_weights<T, V, K>(beta, c0, bw);
   if constexpr (HAS_Z) load_weights<T, V, K>(alpha, c0, aw);
@@ -2658,9 +2676,9 @@ __global__ void __launch_bounds__(SIHC_EV_FWD_THREADS, SIHC_EV_MINW) k_event_fwd
   constexpr int U = SIHC_EV_UNROLL;  // tokens per lane per iteration
   const int BCG = blockDim.x, TL = blockDim.y;
   int slice, chunk;
-  slice_chunk(event16_block(BCG * V * 2, int(gridDim.x)), nslices, slice, chunk);
-  const int c0 = (slice * BCG + threadIdx.x) * V;
-  if (c0 >= g.C) return;
+  slice_chunk_row(int(gridDim.x), nslices, BCG * V * 2 < 128 || (g.C & 1) != 0, slice, chunk);
+  const int cb = (slice * BCG + threadIdx.x) * V, c0 = lane_channel(cb, V, g.C);
+  if (cb >= g.C) return;
   uint32_t bw[16], aw[16];  // word v * 8 + p: channel c0 + v, slots 2p, 2p + 1
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -2680,10 +2698,7 @@ __global__ void __launch_bounds__(SIHC_EV_FWD_THREADS, SIHC_EV_MINW) k_event_fwd
     const uint32_t u = w[v * 8 + (sl >> 1)];
     return __uint_as_float((sl & 1) ? (u & 0xffff0000u) : (u << 16));
   };
-  const int64_t row_w = int64_t(g.GK) * (g.C >> 1);  // words per carrier row (C even here)
-  const int pix_w = g.C >> 1;
-  const uint32_t* xw = reinterpret_cast<const uint32_t*>(x);
-  uint32_t* xow = reinterpret_cast<uint32_t*>(xo);
+  const int64_t row = int64_t(g.GK) * g.C, pix = g.C;  // elements of a carrier row and pixel
   const int m_begin = chunk * tpb;
   const int m_end = min(m_begin + tpb, g.M);
   for (int m = m_begin + threadIdx.y; m < m_end; m += U * TL) {
@@ -2694,13 +2709,13 @@ __global__ void __launch_bounds__(SIHC_EV_FWD_THREADS, SIHC_EV_MINW) k_event_fwd
     for (int u = 0; u < U; ++u) {
       ok[u] = m + u * TL < m_end;
       const int mu = ok[u] ? m + u * TL : m;  // tail: reload a valid token, store nothing
-      b0[u] = (cell_pixel0(mu, g, index) * g.C + c0) >> 1;
-      zw[u] = (int64_t(mu) * g.C + c0) >> 1;
-      dr[u] = ld<NTL>(reinterpret_cast<const uint32_t*>(dz) + zw[u]);
+      b0[u] = cell_pixel0(mu, g, index) * g.C + c0;
+      zw[u] = int64_t(mu) * g.C + c0;
+      dr[u] = ld_row<4, NTL>(dz + zw[u]);
 #pragma unroll
       for (int uy = 0; uy < K; ++uy)
 #pragma unroll
-        for (int ux = 0; ux < K; ++ux) xr[u][uy * K + ux] = ld<NTL>(xw + b0[u] + uy * row_w + ux * pix_w);
+        for (int ux = 0; ux < K; ++ux) xr[u][uy * K + ux] = ld_row<4, NTL>(x + b0[u] + uy * row + ux * pix);
     }
     load_fence();
 #pragma unroll
@@ -2716,10 +2731,10 @@ __global__ void __launch_bounds__(SIHC_EV_FWD_THREADS, SIHC_EV_MINW) k_event_fwd
           if constexpr (HAS_Z) zacc[v] = fmaf(wget(aw, sl, v), xv[v], zacc[v]);
         }
         if (ok[u])
-          store_vec<bf16_t, V, NTS>(reinterpret_cast<bf16_t*>(xow + b0[u] + (sl / K) * row_w + (sl % K) * pix_w), xv);
+          store_vec<bf16_t, V, NTS>(xo + b0[u] + (sl / K) * row + (sl % K) * pix, xv);
       }
       if constexpr (HAS_Z) {
-        if (ok[u]) store_vec<bf16_t, V, NTS>(zo + 2 * zw[u], zacc);
+        if (ok[u]) store_vec<bf16_t, V, NTS>(zo + zw[u], zacc);
       }
     }
   }
@@ -2739,7 +2754,7 @@ __global__ void __launch_bounds__(1024) k_event_fwd_rows(const T* __restrict__ x
                                                          const int32_t* __restrict__ index, Geo g) {
   constexpr int K = 2, S = 4;
   const int m = int(blockIdx.x) * int(blockDim.y) + int(threadIdx.y);
-  const int c0 = int(threadIdx.x) * V;
+  const int c0 = lane_channel(int(threadIdx.x) * V, V, g.C);
   if (m >= g.M) return;
   float bw[S][V], aw[S][V];
   load_weights<T, V, K>(beta, c0, bw);
@@ -2792,8 +2807,9 @@ __global__ void __launch_bounds__(256, SIHC_EV_MINW) k_event_bwd(const T* __rest
   const int BCG = blockDim.x, TL = blockDim.y;
   const int BC = BCG * V;
   int slice, chunk;
-  slice_chunk(K == 4 ? event16_block(BC * int(sizeof(T)), carry.nmain) : int(blockIdx.x), nslices, slice, chunk);
-  const int c0 = slice * BC + threadIdx.x * V;
+  constexpr bool RAG = !NTL;  // rows that V does not divide are launched without hints
+  slice_chunk_row(carry.nmain, nslices, (K == 4 && BC * int(sizeof(T)) < 128) || RAG, slice, chunk);
+  const int cb = slice * BC + threadIdx.x * V, c0 = RAG ? lane_channel(cb, V, g.C) : cb;
   float db[S][V], da[S][V];
 #pragma unroll
   for (int s = 0; s < S; ++s)
@@ -2802,7 +2818,7 @@ __global__ void __launch_bounds__(256, SIHC_EV_MINW) k_event_bwd(const T* __rest
       db[s][v] = 0.f;
       da[s][v] = 0.f;
     }
-  if (c0 < g.C) {
+  if (cb < g.C) {
     float bw[S][V], aw[S][V];
     if constexpr (HAS_W) load_weights<T, V, K>(beta, c0, bw);
     if constexpr (HAS_G) load_weights<T, V, K>(alpha, c0, aw);
@@ -2930,8 +2946,8 @@ __global__ void __launch_bounds__(256, SIHC_EV_MINW) k_event_bwd(const T* __rest
       const int r = i - lane * S * V;
       const int s = r / V;
       const int v = r - s * V;
-      const int c = cs + lane * V + v;
-      if (c < g.C) prow[(int64_t(w) * S + s) * g.C + c] = sum;
+      const int cbl = cs + lane * V;
+      if (cbl < g.C) prow[(int64_t(w) * S + s) * g.C + (RAG ? lane_channel(cbl, V, g.C) : cbl) + v] = sum;
     });
   }
 }
@@ -2961,8 +2977,8 @@ __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_
   const int BCG = blockDim.x, TL = blockDim.y;
   const int BC = BCG * V;
   int slice, chunk;
-  slice_chunk(event16_block(BC * 2, carry.nmain), nslices, slice, chunk);
-  const int c0 = slice * BC + threadIdx.x * V;
+  slice_chunk_row(carry.nmain, nslices, BC * 2 < 128 || (g.C & 1) != 0, slice, chunk);
+  const int cb = slice * BC + threadIdx.x * V, c0 = lane_channel(cb, V, g.C);
   float db[S][V], da[S][V];
 #pragma unroll
   for (int sl = 0; sl < S; ++sl)
@@ -2975,7 +2991,7 @@ __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_
   };
   auto lo_f = [](uint32_t u) { return __uint_as_float(u << 16); };
   auto hi_f = [](uint32_t u) { return __uint_as_float(u & 0xffff0000u); };
-  if (c0 < g.C) {
+  if (cb < g.C) {
     uint32_t bw[16], aw[16];
     if constexpr (HAS_W) {
 #pragma unroll
@@ -2994,29 +3010,25 @@ __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_
       }
     }
     const int64_t M = g.M;
-    const int64_t row_w = int64_t(g.GK) * (g.C >> 1);  // words per carrier row (C even here)
-    const int pix_w = g.C >> 1;
-    const uint32_t* gxw = reinterpret_cast<const uint32_t*>(gxo);
-    const uint32_t* xow = reinterpret_cast<const uint32_t*>(xo);
-    uint32_t* gxo_w = reinterpret_cast<uint32_t*>(gx);
+    const int64_t row = int64_t(g.GK) * g.C, pix = g.C;  // elements of a carrier row and pixel
     for (int64_t m0 = int64_t(chunk) * gs; m0 < M; m0 += int64_t(nchunks) * gs) {
       const int64_t m_end = min(m0 + gs, M);
       for (int64_t mi = m0; mi < m_end; mi += TL) {
         const int64_t mt = mi + threadIdx.y;
         const bool ok = mt < m_end;
         const int mu = int(ok ? mt : mi);  // tail: reload the iteration's first token
-        const int64_t b0 = (cell_pixel0(mu, g, index) * g.C + c0) >> 1;
-        const int64_t zw = (int64_t(mu) * g.C + c0) >> 1;
+        const int64_t b0 = cell_pixel0(mu, g, index) * g.C + c0;
+        const int64_t zw = int64_t(mu) * g.C + c0;
         uint32_t gzr = 0u, dr = 0u, tr[S], xr[S];
-        if constexpr (HAS_G) gzr = ld<NTL>(reinterpret_cast<const uint32_t*>(gzo) + zw);
-        if constexpr (HAS_W) dr = ld<NTL>(reinterpret_cast<const uint32_t*>(dz) + zw);
+        if constexpr (HAS_G) gzr = ld_row<4, NTL>(gzo + zw);
+        if constexpr (HAS_W) dr = ld_row<4, NTL>(dz + zw);
 #pragma unroll
         for (int uy = 0; uy < K; ++uy)
 #pragma unroll
           for (int ux = 0; ux < K; ++ux) {
-            const int64_t o = b0 + uy * row_w + ux * pix_w;
-            tr[uy * K + ux] = HAS_H ? ld<NTL>(gxw + o) : 0u;
-            if constexpr (HAS_G) xr[uy * K + ux] = ld<NTL>(xow + o);
+            const int64_t o = b0 + uy * row + ux * pix;
+            tr[uy * K + ux] = HAS_H ? ld_row<4, NTL>(gxo + o) : 0u;
+            if constexpr (HAS_G) xr[uy * K + ux] = ld_row<4, NTL>(xo + o);
           }
         load_fence();
         // a tail token adds exactly nothing: every loaded value is zeroed (a zero factor
@@ -3046,12 +3058,12 @@ __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_
           if constexpr (STORE_T) {
             if (ok) {
               const int uy = sl / K, ux = sl % K;
-              store_vec<bf16_t, V, NTS>(reinterpret_cast<bf16_t*>(gxo_w + b0 + uy * row_w + ux * pix_w), t);
+              store_vec<bf16_t, V, NTS>(gx + b0 + uy * row + ux * pix, t);
             }
           }
         }
         if constexpr (HAS_W) {
-          if (ok) store_vec<bf16_t, V, NTS>(gdz + (int64_t(mu) * g.C + c0), gd);
+          if (ok) store_vec<bf16_t, V, NTS>(gdz + zw, gd);
         }
       }
     }
@@ -3072,34 +3084,32 @@ __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_
       const int r = i - lane * S * V;
       const int sl = r / V;
       const int v = r - sl * V;
-      const int c = cs + lane * V + v;
-      if (c < g.C) prow[(int64_t(w) * S + sl) * g.C + c] = sum;
+      const int cbl = cs + lane * V;
+      if (cbl < g.C) prow[(int64_t(w) * S + sl) * g.C + lane_channel(cbl, V, g.C) + v] = sum;
     });
   }
 }
 
 // ----------------------------------------------------------------------------------
-// gather / scatter of whole cells (bit-exact copies of CH-byte chunks)
+// gather / scatter of whole cells (bit-exact copies of CH-byte pieces; the last piece of a
+// row that CH does not divide is moved back to end with it)
 // cells[m][s][:] <-> x[pixel(index(m), s)][:]
 // ----------------------------------------------------------------------------------
-template <typename R, int K, bool GATHER>
-__global__ void __launch_bounds__(256) k_cells(const R* __restrict__ src, R* __restrict__ dst,
-                                               const int32_t* __restrict__ index, Geo g, int row_chunks) {
-  constexpr int S = K * K;
+template <typename T, int CH, int K, bool GATHER>
+__global__ void __launch_bounds__(256) k_cells(const T* __restrict__ src, T* __restrict__ dst,
+                                               const int32_t* __restrict__ index, Geo g) {
+  constexpr int S = K * K, V = CH / int(sizeof(T));
   const int64_t row = int64_t(blockIdx.x) * blockDim.y + threadIdx.y;  // m*S + s
   if (row >= int64_t(g.M) * S) return;
   const int m = int(row / S);
   const int s = int(row - int64_t(m) * S);
   const int64_t pix = cell_pixel0(m, g, index) + int64_t(s / K) * g.GK + (s % K);
-  const int64_t xrow = pix * row_chunks;
-  const int64_t crow = row * row_chunks;
-  for (int i = threadIdx.x; i < row_chunks; i += blockDim.x) {
+  const int64_t xrow = pix * g.C;
+  const int64_t crow = row * g.C;
+  for (int c = int(threadIdx.x) * V; c < g.C; c += int(blockDim.x) * V) {
     constexpr bool NTL = (SIHC_CELLS_NTM & 1) != 0, NTS = (SIHC_CELLS_NTM & 2) != 0;
-    if constexpr (GATHER) {
-      st<NTS>(dst + crow + i, ld<NTL>(src + xrow + i));
-    } else {
-      st<NTS>(dst + xrow + i, ld<NTL>(src + crow + i));
-    }
+    const int64_t c0 = lane_channel(c, V, g.C), from = (GATHER ? xrow : crow) + c0, to = (GATHER ? crow : xrow) + c0;
+    st_row<CH, NTS>(dst + to, ld_row<CH, NTL>(src + from));
   }
 }
 
@@ -3151,8 +3161,20 @@ __global__ void __launch_bounds__(256) k_cells_add(const T* __restrict__ cells, 
   const int64_t pix0 = cell_pixel0(int(m), g, nullptr);
   const int64_t row = int64_t(S) * g.C;  // elements of one token's cell
   const T* __restrict__ src = cells + int64_t(b) * g.GG * row;
-  const int nvec = S * g.C / V;
+  const int per_slot = (g.C + V - 1) / V, nvec = S * per_slot;  // vectors of a slot row, of a cell
+  const bool whole = g.C % V == 0;
   for (int i0 = tid; i0 < nvec; i0 += CA_U * 256) {
+    int from[CA_U];  // past the last vector: that vector again, not stored
+#pragma unroll
+    for (int u = 0; u < CA_U; ++u) {
+      const int i = min(i0 + u * 256, nvec - 1);
+      if (whole) {
+        from[u] = i * V;
+      } else {
+        const int s = i / per_slot;
+        from[u] = s * g.C + lane_channel((i - s * per_slot) * V, V, g.C);
+      }
+    }
     float acc[CA_U][V];
 #pragma unroll
     for (int u = 0; u < CA_U; ++u)
@@ -3162,8 +3184,7 @@ __global__ void __launch_bounds__(256) k_cells_add(const T* __restrict__ cells, 
       const T* __restrict__ r = src + int64_t(hit[h]) * row;
       RawVec<T, V> val[CA_U];
 #pragma unroll
-      for (int u = 0; u < CA_U; ++u)  // past the last vector: that vector again, not stored
-        load_raw<T, V, NTL>(r + int64_t(min(i0 + u * 256, nvec - 1)) * V, val[u]);
+      for (int u = 0; u < CA_U; ++u) load_raw<T, V, NTL>(r + from[u], val[u]);
       load_fence();
 #pragma unroll
       for (int u = 0; u < CA_U; ++u) {
@@ -3175,9 +3196,8 @@ __global__ void __launch_bounds__(256) k_cells_add(const T* __restrict__ cells, 
     }
 #pragma unroll
     for (int u = 0; u < CA_U; ++u) {
-      const int i = i0 + u * 256;
-      if (i < nvec) {
-        const int s = i * V / g.C, c = i * V - s * g.C;
+      if (i0 + u * 256 < nvec) {
+        const int s = from[u] / g.C, c = from[u] - s * g.C;
         store_vec<T, V, NTS>(x + slot_offset<K>(pix0, s, g, c), acc[u]);
       }
     }
@@ -3351,6 +3371,28 @@ int pick_vec(int C, int elem, int max_v, const void* const* ptrs, int n) {
     if (ok) return v;
   }
   return 1;
+}
+
+// Vector width of a row of C channels: the largest V in {8, 4, 2, 1} with V <= max_v, V * elem
+// <= 16 and V <= C, whatever the alignment of the rows (ld_row, lane_channel). Against the
+// widest vector that divided the width and fitted every pointer, bf16, 4 slots: 16,384 tokens x
+// 1001 (1 element before), event forward 228 -> 61 us (5.4 TB/s), backward 335 -> 113,
+// triangular of 7 updates 243 -> 55, its backward 390 -> 136, gamma gradient 138 -> 47, weight
+// gradient of 8 events 261 -> 120, read 140 -> 97, write 178 -> 114, gather 117 -> 49; x 1154
+// (2 elements before), event backward 285 -> 144, read of 8 events 126 -> 112 (of 20: 277 ->
+// 280), write 160 -> 147; fp32, 8,192 x 627: event forward 105 -> 31, triangular 92 -> 27.
+// in_place: an output is one of the inputs, so every element has to be read and written by one
+// lane alone: then V divides C.
+int row_vec(int C, int elem, int max_v, bool in_place = false) {
+  for (int v : {8, 4, 2})
+    if (v <= max_v && v * elem <= 16 && v <= C && (!in_place || C % v == 0)) return v;
+  return 1;
+}
+bool any_equal(const void* const* a, int na, const void* const* b, int nb) {
+  for (int i = 0; i < na; ++i)
+    for (int j = 0; j < nb; ++j)
+      if (a[i] && a[i] == b[j]) return true;
+  return false;
 }
 
 struct Shape2D {
@@ -3676,34 +3718,32 @@ int cells_copy(const char* what, bool gather, const void* src, const int32_t* in
   if (!valid_dtype(dtype)) return fail(SIHC_ERR_INVALID, "%s: bad dtype %d", what, dtype);
   if (g.M == 0) return SIHC_OK;  // empty tensors may carry NULL data pointers
   if (!src || !dst) return fail(SIHC_ERR_INVALID, "%s: null pointer", what);
-  const int64_t row_bytes = int64_t(channels) * elem_size(dtype);
-  const int S = cell * cell;
-  const int64_t rows = int64_t(g.M) * S;
+  const int64_t rows = int64_t(g.M) * cell * cell;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  auto go = [&](auto r) {
-    using R = decltype(r);
-    const int row_chunks = int(row_bytes / int64_t(sizeof(R)));
+  auto go = [&](auto t, auto ch) {
+    using T = decltype(t);
+    constexpr int CH = decltype(ch)::value, V = CH / int(sizeof(T));
+    const int pieces = (channels + V - 1) / V;
     int bx = 64;
-    while (bx > 1 && bx / 2 >= row_chunks) bx /= 2;
+    while (bx > 1 && bx / 2 >= pieces) bx /= 2;
     const int by = 256 / bx;
     const int64_t gx = (rows + by - 1) / by;
     if (gx > 0x7fffffff) return fail(SIHC_ERR_INVALID, "%s: too many rows", what);
     auto launch = [&](auto kk) {
       constexpr int KK = decltype(kk)::value;
       if (gather) {
-        hipLaunchKernelGGL((k_cells<R, KK, true>), dim3(unsigned(gx)), dim3(bx, by), 0, st,
-                           static_cast<const R*>(src), static_cast<R*>(dst), index, g, row_chunks);
+        hipLaunchKernelGGL((k_cells<T, CH, KK, true>), dim3(unsigned(gx)), dim3(bx, by), 0, st,
+                           static_cast<const T*>(src), static_cast<T*>(dst), index, g);
       } else {
-        hipLaunchKernelGGL((k_cells<R, KK, false>), dim3(unsigned(gx)), dim3(bx, by), 0, st,
-                           static_cast<const R*>(src), static_cast<R*>(dst), index, g, row_chunks);
+        hipLaunchKernelGGL((k_cells<T, CH, KK, false>), dim3(unsigned(gx)), dim3(bx, by), 0, st,
+                           static_cast<const T*>(src), static_cast<T*>(dst), index, g);
       }
       return check_launch(what);
     };
     return with_cell(cell, launch);
   };
-  if (row_bytes % 16 == 0 && aligned(src, 16) && aligned(dst, 16)) return go(u32x4{});
-  if (row_bytes % 4 == 0 && aligned(src, 4) && aligned(dst, 4)) return go(uint32_t{});
-  return go(uint16_t{});
+  if (elem_size(dtype) == 4) return channels >= 4 ? go(uint32_t{}, IC<16>{}) : go(uint32_t{}, IC<4>{});
+  return channels >= 8 ? go(uint16_t{}, IC<16>{}) : go(uint16_t{}, IC<2>{});
 }
 
 // Adjoint of the gather (k_cells_add): one block per destination cell.
@@ -3716,8 +3756,7 @@ int cells_add(const char* what, const void* cells, const int32_t* index, void* x
   if (!cells || !x) return fail(SIHC_ERR_INVALID, "%s: null pointer", what);
   if (!index) return cells_copy(what, false, cells, nullptr, x, batch, grid, cell, channels, dtype, stream);
   if (g.GG > 16384) return fail(SIHC_ERR_INVALID, "%s: grid of %d cells exceeds 16384", what, g.GG);
-  const void* ptrs[] = {cells, x};
-  const int V = pick_vec(channels, elem_size(dtype), 8, ptrs, 2);
+  const int V = row_vec(channels, elem_size(dtype), 8);
   const size_t lds = size_t(g.GG) * sizeof(int32_t);
   hipStream_t st = static_cast<hipStream_t>(stream);
   return with_dtype(dtype, [&](auto t) {
@@ -3756,7 +3795,7 @@ int launch_mm(const char* what, const MMArgs& a, int max_chunks, int* chunks, hi
   constexpr int VC = 16 / int(sizeof(T));
   const int segs = K * K / 4 / SGW, parts = segs * (((a.events + 3) / 4 + EGW - 1) / EGW);
   const int slices = (a.g.C + 16 * VC - 1) / (16 * VC);
-  auto* kfn = &k_wgrad_mm<T, K, SGW, EGW, VC, MODE>;
+  auto* kfn = a.g.C % VC ? &k_wgrad_mm<T, K, SGW, EGW, VC, MODE, false> : &k_wgrad_mm<T, K, SGW, EGW, VC, MODE, true>;
   const size_t weights = MODE == MM_GRAD ? 0 : size_t((a.events + 3) / 4) * MM_WG<T, VC> * sizeof(float);
   auto lds_for = [&](int waves) { return std::max(size_t(waves) * 64 * VC * 4 * sizeof(float), weights); };
   // Chunks of a launch with wt token waves per block: whole rounds of resident blocks, so
@@ -3839,7 +3878,12 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
   if (dout)
     for (int i = 0; i < events; ++i) ptrs[nptr++] = dout[i];
   ptrs[nptr++] = x;
-  const int V = pick_vec(g.C, es, 8, ptrs, nptr);
+  bool in_place = false;
+  if (dout) {
+    const void* const* outs = const_cast<const void* const*>(dout);
+    in_place = any_equal(z, events, outs, events) || any_equal(&x, 1, outs, events);
+  }
+  const int V = row_vec(g.C, es, 8, in_place);
   int bcg, slices;
   wgrad_block(g.C, V, events, &bcg, &slices);
   const int tpb = int((int64_t(g.M) + chunks - 1) / chunks);
@@ -3926,7 +3970,7 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
           // 143), 9 and more events of aligned bf16 16-slot rows on the pipelined one (E = 12
           // 416 us, here 447; E = 8 355, here 295).
           if constexpr (CAR) {
-            const bool direct = KK == 2 && events == 1 && VV * int(sizeof(T)) == 16;
+            const bool direct = KK == 2 && events == 1 && VV * int(sizeof(T)) == 16 && g.C % VV == 0;
             if (g.C >= 16 / int(sizeof(T)) && !direct && !(KK == 4 && bf && events > 8)) {
               const MMArgs a{x, pk, part, index, events, g, nullptr, nullptr, PtrPack{}};
               if constexpr (KK == 2) return launch_mm_k2<T, MM_GRAD>(what, a, max_chunks, &chunks, st);
@@ -3951,21 +3995,24 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
             // gamma gradient of 2 updates: the pipelined kernel on one-slot rows (1 wave x 2
             // updates: 77 us at 65,536 rows x 1152 channels; row lanes 81)
             goz(IC<1>{}, IC<1>{}, IC<2>{}, 1);
-          } else if (!CAR && !SD && bf && events >= 3) {
+          } else if (!CAR && !SD && std::is_same<T, bf16_t>::value && VV == 8 && events >= 2) {
             // gamma gradient of 3..32 updates on row lanes (k_gamma_rows), update groups per
             // block measured per update count at 65,536 rows x 1152 channels: A = 3-4 in 4
             // groups (A = 4 124 -> 117 us), 5-10 in one (A = 9 262 -> 229), 11-22 in two (A =
             // 17 453 -> 407), 23-32 in four (A = 32 798 -> 767); against the previous kernels
-            const int G = events <= 4 ? 4 : events <= 10 ? 1 : events <= 22 ? 2 : 4;
+            const int G = events == 2 ? 2 : events <= 4 ? 4 : events <= 10 ? 1 : events <= 22 ? 2 : 4;
             const int slr = (g.C + 127) / 128;
             auto gorows = [&](auto na) {
               constexpr int NA = decltype(na)::value;
-              chunks = whole_rounds(slr, max_chunks,
-                                    resident_blocks(reinterpret_cast<const void*>(&k_gamma_rows<NA>), 256, 0));
-              const int tpr = int((int64_t(g.M) + chunks - 1) / chunks);
-              if (tpr > 0) chunks = int((int64_t(g.M) + tpr - 1) / tpr);  // no chunk past the last token
-              hipLaunchKernelGGL((k_gamma_rows<NA>), dim3(blocks1d(slr, chunks)), dim3(16, G, 16 / G), 0, st,
-                                 reinterpret_cast<const bf16_t*>(x), pk, part, events, int(g.M), g.C, tpr, slr);
+              with_bool(g.C % 8 == 0, [&](auto nt) {
+                auto* kfn = &k_gamma_rows<NA, decltype(nt)::value>;
+                chunks = whole_rounds(slr, max_chunks, resident_blocks(reinterpret_cast<const void*>(kfn), 256, 0));
+                const int tpr = int((int64_t(g.M) + chunks - 1) / chunks);
+                if (tpr > 0) chunks = int((int64_t(g.M) + tpr - 1) / tpr);  // no chunk past the last token
+                hipLaunchKernelGGL(kfn, dim3(blocks1d(slr, chunks)), dim3(16, G, 16 / G), 0, st,
+                                   reinterpret_cast<const bf16_t*>(x), pk, part, events, int(g.M), g.C, tpr, slr);
+                return 0;
+              });
             };
             switch ((events + G - 1) / G) {
               case 1: gorows(IC<1>{}); break;
@@ -3999,16 +4046,19 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
               bool waves = false;
               if constexpr (SD && VV * sizeof(T) == 16) {
                 // many updates: each wave streams one update at a time (k_trib_waves)
-                waves = SIHC_TRIB_WAVES > 0 && events >= SIHC_TRIB_WAVES && g.C % VV == 0;
+                waves = SIHC_TRIB_WAVES > 0 && events >= SIHC_TRIB_WAVES;
                 if (waves) {
                   const int slicesw = (g.C + 16 * VV - 1) / (16 * VV);
                   const size_t ldsw = size_t(TRIB_TT + events) * 16 * VV * sizeof(float);
-                  if (tpb <= TRIB_TT)
-                    hipLaunchKernelGGL((k_trib_waves<T, VV, true>), dim3(blocks1d(slicesw, chunks)), dim3(256), ldsw,
-                                       st, static_cast<const T*>(x), pk, part, events, g, tpb, slicesw, dk, gamma, gf32);
-                  else
-                    hipLaunchKernelGGL((k_trib_waves<T, VV, false>), dim3(blocks1d(slicesw, chunks)), dim3(256), ldsw,
-                                       st, static_cast<const T*>(x), pk, part, events, g, tpb, slicesw, dk, gamma, gf32);
+                  return with_bool(tpb <= TRIB_TT, [&](auto one) {
+                    return with_bool(g.C % VV == 0, [&](auto nt) {
+                      hipLaunchKernelGGL((k_trib_waves<T, VV, decltype(one)::value, decltype(nt)::value>),
+                                         dim3(blocks1d(slicesw, chunks)), dim3(256), ldsw, st,
+                                         static_cast<const T*>(x), pk, part, events, g, tpb, slicesw, dk, gamma,
+                                         gf32);
+                      return check_launch(what);
+                    });
+                  });
                 }
               }
               if (!waves)
@@ -4058,8 +4108,8 @@ int launch_stage_backward(const char* what, const void* x, const void* const* z,
 
 // Vector width of the per-event kernels: registers hold up to 2*S*V weights and 2*S*V
 // accumulators, so wide vectors are used only for the 4-slot cell.
-int event_vec(int C, int es, int cell, const void* const* ptrs, int n) {
-  return pick_vec(C, es, cell == 2 ? SIHC_EV_VEC : 2, ptrs, n);
+int event_vec(int C, int es, int cell, bool in_place) {
+  return row_vec(C, es, cell == 2 ? SIHC_EV_VEC : 2, in_place);
 }
 
 }  // namespace
@@ -4121,11 +4171,12 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
   if (!x || !alpha) return fail(SIHC_ERR_INVALID, "%s: null input", what);
   if (int rc = check_events(what, events, const_cast<const void* const*>(out))) return rc;
   const int es = elem_size(dtype);
-  const void* ptrs[SIHC_MAX_EVENTS + 1];
+  const void* ptrs[SIHC_MAX_EVENTS];
   for (int i = 0; i < events; ++i) ptrs[i] = out[i];
-  ptrs[events] = x;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int V = pick_vec(channels, es, cell == 2 ? 8 : SIHC_RW_VEC_K4, ptrs, events + 1);
+  // (16-slot fp32 keeps a dividing vector: 4,096 tokens x 627, E = 8, read 90 us with 1-channel
+  // lanes, 106 with 2; write 140 and 146)
+  const int V = row_vec(channels, es, cell == 2 ? 8 : SIHC_RW_VEC_K4, cell == 4 && es == 4);
   const int S = cell * cell;
   // 16 slots, bf16 weights, 2-channel lanes: weights packed as bf16 in LDS (half the
   // bytes, so twice the channels per block within the LDS budget)
@@ -4136,8 +4187,9 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
   // weights' pair words staged in the same LDS bytes as the packed bf16 weights)
   const bool d2 = SIHC_K4_DOT2 && wb && cell == 4 && aligned(alpha, 4);
   // 4 slots, bf16, 16-byte lanes, many events: one output array per wave at a time
-  if (SIHC_RDW_MINE > 0 && cell == 2 && dtype == SIHC_DTYPE_BF16 && V == 8 && events >= SIHC_RDW_MINE &&
-      aligned(alpha, 4)) {
+  // (whole vectors only: 16,384 tokens x 1154, E = 20, 342 us here, 277 with 2-channel lanes)
+  if (SIHC_RDW_MINE > 0 && cell == 2 && dtype == SIHC_DTYPE_BF16 && V == 8 && channels % 8 == 0 &&
+      events >= SIHC_RDW_MINE && aligned(alpha, 4)) {
     const int slicesw = (channels + 127) / 128;
     const int64_t chunksw = (int64_t(g.M) + RDW_TT - 1) / RDW_TT;
     const size_t ldsw = size_t(RDW_TT + events) * 2 * 128 * sizeof(uint32_t);
@@ -4150,7 +4202,11 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
       return check_launch(what);
     });
   }
-  const Shape2D sh = cell == 2 ? shape_for(channels, V, SIHC_RW_BCG, events * S * wbytes)
+  // ragged rows: 32 lanes where that covers the width with no more idle lanes than 16 (fewer
+  // lines shared between slices: 16,384 tokens x 1154, E = 8, 136 -> 112 us)
+  const int cg16 = ((channels + V - 1) / V + 15) / 16;
+  const int lanes2 = channels % V && cg16 % 2 == 0 ? 2 * SIHC_RW_BCG : SIHC_RW_BCG;
+  const Shape2D sh = cell == 2 ? shape_for(channels, V, lanes2, events * S * wbytes)
                                : shape_for(channels, V, events <= 8 ? 64 : SIHC_RW_BCG_K4, events * S * wbytes,
                                            SIHC_RW_LDS_K4);  // 64 lanes to 8 events: E = 4 569 -> 542 us
   const int unroll = d2 ? SIHC_RD2_U : cell == 2 ? SIHC_RW_UNROLL : SIHC_RW_UNROLL_K4;
@@ -4173,7 +4229,7 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
           } else {
             // non-temporal carrier loads: for 1-2 events (4 slots) or up to 12 (16 slots),
             // and only with slice rows of whole 128-byte lines
-            const int hints = read_hints(sh.bcg * VV * int(sizeof(T)) >= 128, cell, events);
+            const int hints = read_hints(sh.bcg * VV * int(sizeof(T)) >= 128 && channels % VV == 0, cell, events);
             return with_bcg<KK>(sh.bcg, [&](auto bb) {
               constexpr int BB = decltype(bb)::value;
               return with_hints<SIHC_RD_NTM>(hints, [&](auto nt) {
@@ -4220,13 +4276,9 @@ int sihc_write(const void* x, const void* const* updates, const void* beta, void
   if (g.M == 0) return SIHC_OK;  // empty tensors may carry NULL data pointers
   if ((add_x && !x) || !beta || !out) return fail(SIHC_ERR_INVALID, "%s: null input", what);
   if (int rc = check_events(what, events, updates)) return rc;
-  const void* ptrs[SIHC_MAX_EVENTS + 2];
-  for (int i = 0; i < events; ++i) ptrs[i] = updates[i];
-  ptrs[events] = add_x ? x : nullptr;
-  ptrs[events + 1] = out;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int es = std::max(elem_size(x_dtype), elem_size(w_dtype));
-  const int V = pick_vec(channels, es, cell == 2 ? 8 : SIHC_RW_VEC_K4, ptrs, events + 2);
+  const int V = row_vec(channels, es, cell == 2 ? 8 : SIHC_RW_VEC_K4, (add_x && x == out) || (cell == 4 && es == 4));
   const int S = cell * cell;
   const int E4 = (events + 3) & ~3;
   // 16 slots, bf16 weights, 2-channel lanes: weights packed as bf16 in LDS (as sihc_read)
@@ -4259,7 +4311,7 @@ int sihc_write(const void* x, const void* const* updates, const void* beta, void
             return fail(SIHC_ERR_INVALID, "%s: internal vector width", what);
           } else {
             // non-temporal loads with 8+ events and slice rows of whole 128-byte lines
-            const int hints = write_hints(sh.bcg * VV * int(sizeof(TX)) >= 128, events);
+            const int hints = write_hints(sh.bcg * VV * int(sizeof(TX)) >= 128 && channels % VV == 0, events);
             return with_bool(add_x != 0, [&](auto ax) {
               constexpr bool AX = decltype(ax)::value;
               return with_bcg<KK>(sh.bcg, [&](auto bb) {
@@ -4381,11 +4433,8 @@ int sihc_triangular(const void* base, const void* const* updates, const void* ga
   if (!base || !gamma || !out) return fail(SIHC_ERR_INVALID, "%s: null input", what);
   if (int rc = check_events(what, active, updates)) return rc;
   const int es = elem_size(dtype);
-  const void* ptrs[SIHC_MAX_EVENTS + 2];
-  for (int i = 0; i < active; ++i) ptrs[i] = updates[i];
-  ptrs[active] = base;
-  ptrs[active + 1] = out;
-  const int V = pick_vec(channels, es, 8, ptrs, active + 2);
+  const void* dst = out;
+  const int V = row_vec(channels, es, 8, base == out || any_equal(updates, active, &dst, 1));
   const int A4 = (active + 3) & ~3;
   const Shape2D sh = shape_for(channels, V, SIHC_RW_BCG, A4 * 4);
   // 32-token blocks (64 with one update): 3-5% faster than 128-token ones
@@ -4404,7 +4453,7 @@ int sihc_triangular(const void* base, const void* const* updates, const void* ga
         if constexpr (VV * sizeof(T) > 16) {
           return fail(SIHC_ERR_INVALID, "%s: internal vector width", what);
         } else {
-          return with_hints<SIHC_TRI_NTM>(triangular_hints(active), [&](auto nt) {
+          return with_hints<SIHC_TRI_NTM>(channels % VV ? 0 : triangular_hints(active), [&](auto nt) {
             constexpr int NT = decltype(nt)::value;
             hipLaunchKernelGGL((k_triangular<T, TG, VV, NT>), dim3(blocks1d(sh.slices, chunks)), dim3(sh.bcg, sh.tl),
                                lds, st, static_cast<const T*>(base), pk, static_cast<const TG*>(gamma),
@@ -4489,11 +4538,11 @@ int sihc_event_forward(const void* x, const void* dz, const void* beta, const vo
   const int S = cell * cell;
   if (!aligned(beta, std::min(16, S * es)) || (alpha_next && !aligned(alpha_next, std::min(16, S * es))))
     return fail(SIHC_ERR_INVALID, "%s: weights must be aligned to %d bytes", what, std::min(16, S * es));
-  const void* ptrs[] = {x, dz, x_out, z_out};
-  int V = event_vec(channels, es, cell, ptrs, 4);
+  const bool in_place = x == x_out || (z_out && z_out == dz);
+  int V = event_vec(channels, es, cell, in_place);
   // Weight rows are loaded as V*S contiguous elements: need min(16, V*S*es) alignment.
-  while (V > 1 && (!aligned(beta, std::min(16, V * S * es)) ||
-                   (alpha_next && !aligned(alpha_next, std::min(16, V * S * es)))))
+  while (cell == 4 && V > 1 && (!aligned(beta, std::min(16, V * S * es)) ||
+                                (alpha_next && !aligned(alpha_next, std::min(16, V * S * es)))))
     V /= 2;
   Shape2D sh = shape_for(channels, V, SIHC_EV_BCG, 0);
   sh.tl = SIHC_EV_FWD_THREADS / sh.bcg;  // one-shot blocks of SIHC_EV_FWD_THREADS threads
@@ -4511,19 +4560,19 @@ int sihc_event_forward(const void* x, const void* dz, const void* beta, const vo
         } else {
           return with_bool(alpha_next != nullptr, [&](auto hz) {
             constexpr bool HZ = decltype(hz)::value;
-            constexpr bool NTL = (SIHC_EV_FWD_NT & 1) != 0, NTS = (SIHC_EV_FWD_NT & 2) != 0;
+            return with_bool(channels % VV != 0, [&](auto rg) {
+            constexpr bool RAG = decltype(rg)::value;
+            constexpr bool NTL = !RAG && (SIHC_EV_FWD_NT & 1) != 0, NTS = !RAG && (SIHC_EV_FWD_NT & 2) != 0;
             if constexpr (SIHC_EV_FWD_ROWS && KK == 2 && HZ && std::is_same_v<T, bf16_t>) {
-              // whole rows of 16-byte lanes: every carrier, dz and z_out row and both weight
-              // arrays 16-byte aligned, C / 8 lanes of one token within one block. With a read
+              // whole rows of 16-byte lanes, C / 8 lanes of one token within one block. With a read
               // part only: the write-only forward (no alpha_next) ran 3% slower on whole rows
               // than on the general kernel (224 against 217 us at batch 256, C 1152).
               constexpr int VR = 8;
-              const int lanes = channels / VR;
-              if (channels % VR == 0 && lanes <= 1024 && aligned(x, 16) && aligned(dz, 16) && aligned(x_out, 16) &&
-                  aligned(z_out, 16) && aligned(beta, 16) && aligned(alpha_next, 16)) {
+              const int lanes = (channels + VR - 1) / VR;
+              if (channels >= VR && lanes <= 1024 && (!in_place || channels % VR == 0)) {
                 const int tr = std::max(1, SIHC_EV_ROW_THREADS / lanes);
                 const int64_t blocks = (int64_t(g.M) + tr - 1) / tr;
-                hipLaunchKernelGGL((k_event_fwd_rows<T, VR, HZ, NTL, NTS>), dim3(unsigned(blocks)), dim3(lanes, tr), 0,
+                hipLaunchKernelGGL((k_event_fwd_rows<T, VR, HZ, true, true>), dim3(unsigned(blocks)), dim3(lanes, tr), 0,
                                    st, static_cast<const T*>(x), static_cast<const T*>(dz),
                                    static_cast<const T*>(beta), static_cast<const T*>(alpha_next),
                                    static_cast<T*>(x_out), static_cast<T*>(z_out), index, g);
@@ -4542,6 +4591,7 @@ int sihc_event_forward(const void* x, const void* dz, const void* beta, const vo
                                static_cast<const T*>(alpha_next), static_cast<T*>(x_out), static_cast<T*>(z_out),
                                index, g, tpb, sh.slices);
             return check_launch(what);
+            });
           });
         }
       });
@@ -4615,9 +4665,10 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
   const int es = elem_size(dtype);
   if ((beta && !aligned(beta, std::min(16, S * es))) || (alpha_next && !aligned(alpha_next, std::min(16, S * es))))
     return fail(SIHC_ERR_INVALID, "%s: weights must be aligned to %d bytes", what, std::min(16, S * es));
-  const void* ptrs[] = {grad_x_out, grad_z_out, x_out, dz, grad_x, grad_dz};
-  int V = event_vec(channels, es, cell, ptrs, 6);
-  while (V > 1 && ((beta && !aligned(beta, std::min(16, V * S * es))) ||
+  const void* ins[] = {grad_x_out, grad_z_out, x_out, dz};
+  const void* outs[] = {grad_x, grad_dz};
+  int V = event_vec(channels, es, cell, any_equal(outs, 2, ins, 4));
+  while (cell == 4 && V > 1 && ((beta && !aligned(beta, std::min(16, V * S * es))) ||
                    (has_g && !aligned(alpha_next, std::min(16, V * S * es)))))
     V /= 2;
   // Channel lanes per block: 32; 16 for 16-byte fp32 lanes (256-byte rows, 65,536 tokens x
@@ -4652,7 +4703,9 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
             constexpr bool HH = decltype(hh)::value;
             auto go = [&](auto hg, auto hw, auto stt) {
               constexpr bool HG = decltype(hg)::value, HW = decltype(hw)::value, STT = decltype(stt)::value;
-              constexpr bool NTL = (SIHC_EV_BWD_NT & 1) != 0, NTS = (SIHC_EV_BWD_NT & 2) != 0;
+              return with_bool(channels % VV != 0, [&](auto rg) {
+              constexpr bool RAG = decltype(rg)::value;
+              constexpr bool NTL = !RAG && (SIHC_EV_BWD_NT & 1) != 0, NTS = !RAG && (SIHC_EV_BWD_NT & 2) != 0;
               // 16-slot bf16 cells with 2-channel lanes: the register-lean kernel
               constexpr bool B16 = SIHC_EV_BWD16 && KK == 4 && VV == 2 && std::is_same_v<T, bf16_t>;
               const void* kfn;
@@ -4686,6 +4739,7 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
                                  static_cast<T*>(grad_x), static_cast<T*>(grad_dz), part, index, g, gs, chunks,
                                  sh.slices, cy);
               return check_launch(what);
+              });
             };
             switch (mode) {
               case 0: return go(std::true_type{}, std::true_type{}, std::true_type{});
