@@ -25,6 +25,7 @@
 #include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -477,8 +478,10 @@ PyObject* to_list(const variable_list& ts) {
 }
 PyObject* not_implemented() { Py_RETURN_NOTIMPLEMENTED; }
 
-// Run `f`; a C-ABI error, or any C++ exception, hands the call to the Python op, which repeats
-// the checks and raises what it always raised.
+// Run `f`; a C-ABI error, or a C++ exception, hands the call to the Python op, which repeats
+// the checks and raises what it always raised. A Python exception comes from the caller's own
+// code (a saved-tensor hook) and goes on to the caller: checkpointing ends its recomputation
+// by raising from such a hook, which must not run again for the same call.
 template <typename F>
 PyObject* guarded(const char* name, F&& f) {
   try {
@@ -487,6 +490,9 @@ PyObject* guarded(const char* name, F&& f) {
     return f();
   } catch (const Failure&) {
     return not_implemented();
+  } catch (python_error& e) {
+    e.restore();
+    return nullptr;
   } catch (const std::exception&) {
     PyErr_Clear();
     return not_implemented();

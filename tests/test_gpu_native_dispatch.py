@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import pytest
 import torch
+import torch.utils.checkpoint
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from sihc_hip import indexed as ix
@@ -167,6 +168,28 @@ def test_saved_tensor_hooks_and_version_checks():
         w.add_(1.0)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         _grads(out, (x, w))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_an_error_of_a_saved_tensor_hook_reaches_the_caller_once(name):
+    """Checkpointing ends its recomputation by raising from the pack hook of the last tensor."""
+    op, args, _ = _calls(torch.float32)[name]
+    calls = []
+
+    def pack(t):
+        calls.append(t)
+        raise KeyError("stop")
+
+    with pytest.raises(KeyError, match="stop"), torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        op(*args)
+    assert len(calls) == 1
+
+    def region():
+        return _outs(op(*args))
+
+    again = torch.utils.checkpoint.checkpoint(region, use_reentrant=False)
+    assert _is_native(again[0])
+    assert all(torch.equal(a, b) for a, b in zip(_grads(again, args), _grads(region(), args)))
 
 
 def test_vmap_forward_mode_and_subclasses_take_the_registered_op():
