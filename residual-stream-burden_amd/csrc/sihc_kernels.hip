@@ -1135,7 +1135,9 @@ __global__ void __launch_bounds__(256) k_read_w(const bf16_t* __restrict__ x, co
 
 // ----------------------------------------------------------------------------------
 // Block reduction helper: sums W = (blockDim.x * NV) floats per thread over threadIdx.y
-// and hands each (lane-major) sum to `emit(i, value)`. red must hold TL * W floats.
+// and hands each (lane-major) sum to `emit(i, value)`. red must hold TL * W floats. More than 8
+// rows are summed as rows of 8: one chain over the 64 rows of a 4-lane slice left an fp32 weight
+// gradient of 256 tokens x 130 channels 1.6e-7 from the exact sum, 8-row blocks 0.9e-7.
 // ----------------------------------------------------------------------------------
 template <int NV, typename Emit>
 __device__ __forceinline__ void block_reduce_rows(const float* acc, float* red, Emit&& emit) {
@@ -1148,7 +1150,11 @@ __device__ __forceinline__ void block_reduce_rows(const float* acc, float* red, 
   __syncthreads();
   for (int i = tid; i < W; i += nthr) {
     float sum = 0.f;
-    for (int ty = 0; ty < TL; ++ty) sum += red[ty * W + i];
+    for (int t0 = 0; t0 < TL; t0 += 8) {
+      float eight = 0.f;
+      for (int ty = t0; ty < min(t0 + 8, TL); ++ty) eight += red[ty * W + i];
+      sum += eight;
+    }
     emit(i, sum);
   }
   __syncthreads();
