@@ -1150,10 +1150,14 @@ __device__ __forceinline__ void block_reduce_rows(const float* acc, float* red, 
   __syncthreads();
   for (int i = tid; i < W; i += nthr) {
     float sum = 0.f;
-    for (int t0 = 0; t0 < TL; t0 += 8) {
-      float eight = 0.f;
-      for (int ty = t0; ty < min(t0 + 8, TL); ++ty) eight += red[ty * W + i];
-      sum += eight;
+    if (TL <= 8) {
+      for (int ty = 0; ty < TL; ++ty) sum += red[ty * W + i];
+    } else {
+      for (int t0 = 0; t0 < TL; t0 += 8) {
+        float eight = 0.f;
+        for (int ty = t0; ty < min(t0 + 8, TL); ++ty) eight += red[ty * W + i];
+        sum += eight;
+      }
     }
     emit(i, sum);
   }
