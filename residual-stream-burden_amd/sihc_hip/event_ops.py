@@ -75,6 +75,12 @@ def _event_setup(ctx, inputs, output):
 @custom_op("sihc::event_write_read_backward", mutates_args=())
 def _event_backward(grad_x_out: Optional[Tensor], grad_z_out: Optional[Tensor], x_out: Tensor,
                     dz: Tensor, beta: Tensor, alpha_next: Tensor) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+    _validate_event(x_out, dz, beta, alpha_next)  # saved tensors come back through the caller's hooks
+    for grad, like in ((grad_x_out, x_out), (grad_z_out, dz)):
+        if grad is not None:
+            _require_packed("event write/read backward", grad=grad)
+            if grad.shape != like.shape or grad.dtype != like.dtype or grad.device != like.device:
+                raise ValueError("output gradients must match the outputs")
     gx, gdz, gb, ga = launch.event_backward(grad_x_out, grad_z_out, x_out, dz, beta, alpha_next)
     return gx, gdz, gb, ga
 

@@ -69,10 +69,25 @@ def _same_device(index: Tensor, x: Tensor) -> None:
         raise ValueError("index must live on the carrier's device")
 
 
+def _require_index(index: Tensor, x: Tensor, tokens: int) -> None:
+    """What the kernels read of an index: `tokens` packed int32 values on x's device."""
+    _same_device(index, x)
+    _require_packed("spatial index", index=index)
+    if index.dtype != torch.int32 or index.numel() != tokens:
+        raise ValueError(f"index must be int32 with {tokens} entries, got {index.dtype} {tuple(index.shape)}")
+
+
+def _require_cells(cells: Tensor, index: Tensor) -> None:
+    _require_packed("scatter_cells", cells=cells)
+    if cells.ndim != 4 or int(round(cells.shape[1] ** 0.5)) ** 2 != cells.shape[1]:
+        raise ValueError("expected [B, G*G, S, C] cells that cover a square workspace grid")
+    _require_index(index, cells, cells.shape[0] * cells.shape[1])
+
+
 @custom_op("sihc::indexed_read", mutates_args=())
 def _indexed_read(x: Tensor, alpha: Tensor, index: Tensor) -> list[Tensor]:
-    _geometry(x, alpha)
-    _same_device(index, x)
+    b, _, g, _ = _geometry(x, alpha)
+    _require_index(index, x, b * g * g)
     return launch.read(x, alpha, index=index)
 
 
@@ -86,8 +101,8 @@ def _indexed_read_fake(x, alpha, index):
 
 @custom_op("sihc::indexed_write_impl", mutates_args=())
 def _indexed_write_impl(x: Tensor, updates: list[Tensor], beta: Tensor, index: Tensor, add_x: bool) -> Tensor:
-    _validate_updates(x, beta, updates)
-    _same_device(index, x)
+    b, _, g, _ = _validate_updates(x, beta, updates)
+    _require_index(index, x, b * g * g)
     return launch.write(x, updates, beta, add_x=add_x, index=index)
 
 
@@ -98,7 +113,8 @@ def _indexed_write_impl_fake(x, updates, beta, index, add_x):
 
 @custom_op("sihc::indexed_weight_grad", mutates_args=())
 def _indexed_weight_grad(x: Tensor, updates: list[Tensor], weights: Tensor, index: Tensor) -> Tensor:
-    _validate_updates(x, weights, updates)
+    b, _, g, _ = _validate_updates(x, weights, updates)
+    _require_index(index, x, b * g * g)
     return launch.weight_grad(x, updates, weights, index=index)
 
 
@@ -109,8 +125,8 @@ def _indexed_weight_grad_fake(x, updates, weights, index):
 
 @custom_op("sihc::indexed_read_backward", mutates_args=())
 def _indexed_read_grads(x: Tensor, grads: list[Tensor], alpha: Tensor, index: Tensor) -> tuple[Tensor, Tensor]:
-    _validate_updates(x, alpha, grads)
-    _same_device(index, x)
+    b, _, g, _ = _validate_updates(x, alpha, grads)
+    _require_index(index, x, b * g * g)
     return launch.read_backward(x, grads, alpha, index=index)
 
 
@@ -122,8 +138,8 @@ def _indexed_read_grads_fake(x, grads, alpha, index):
 @custom_op("sihc::indexed_write_backward", mutates_args=())
 def _indexed_write_grads(grad: Tensor, updates: list[Tensor], beta: Tensor,
                          index: Tensor) -> tuple[list[Tensor], Tensor]:
-    _validate_updates(grad, beta, updates)
-    _same_device(index, grad)
+    b, _, g, _ = _validate_updates(grad, beta, updates)
+    _require_index(index, grad, b * g * g)
     return launch.write_backward(grad, updates, beta, index=index)
 
 
@@ -176,6 +192,8 @@ native(_indexed_write, "indexed_write")
 
 @custom_op("sihc::gather_cells", mutates_args=())
 def _gather_cells(x: Tensor, index: Tensor, slots: int) -> Tensor:
+    b, g = _carrier_grid(x, slots)
+    _require_index(index, x, b * g * g)
     return launch.gather_cells(x, index, slots)
 
 
@@ -189,6 +207,7 @@ def _gather_cells_fake(x, index, slots):
 
 @custom_op("sihc::scatter_cells", mutates_args=())
 def _scatter_cells(cells: Tensor, index: Tensor) -> Tensor:
+    _require_cells(cells, index)
     return launch.scatter_cells(cells, index)
 
 
@@ -202,6 +221,7 @@ def _scatter_cells_fake(cells, index):
 
 @custom_op("sihc::scatter_add_cells", mutates_args=())
 def _scatter_add_cells(cells: Tensor, index: Tensor) -> Tensor:
+    _require_cells(cells, index)
     return launch.scatter_add_cells(cells, index)
 
 

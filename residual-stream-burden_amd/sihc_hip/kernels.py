@@ -170,10 +170,19 @@ def _make_final_accumulate(tag: str):
                    schema=_schema(["x0", *dz_names, *beta_names], "Tensor"))
     fa.register_fake(lambda x0, *rest: torch.empty_like(x0))
 
+    def check_grad(what: str, grad_out: Tensor) -> tuple[int, int]:
+        _require_packed(what, grad_out=grad_out)
+        if grad_out.ndim != 4 or grad_out.shape[1] != edge or grad_out.shape[2] != edge:
+            raise ValueError(f"{what} expects grad_out [B,{edge},{edge},C], got {tuple(grad_out.shape)}")
+        return grad_out.shape[0], grad_out.shape[3]
+
     def grad_dz_impl(grad_out: Tensor, *betas: Tensor) -> Tensor:
         """[E,B,256,C] in grad_out's dtype: dz_e gradient = read of grad_out with beta_e."""
-        _require_packed(f"{name}_grad_dz_ptr", grad_out=grad_out)
-        b, c = grad_out.shape[0], grad_out.shape[3]
+        b, c = check_grad(f"{name}_grad_dz_ptr", grad_out)
+        _check_cuda(f"{name}_grad_dz_ptr", grad_out, *betas)
+        for i, beta in enumerate(betas):
+            if tuple(beta.shape) != (c, slots):
+                raise ValueError(f"{name} beta{i} must be [{c},{slots}], got {tuple(beta.shape)}")
         out = grad_out.new_empty((blocks, b, WORKSPACE_TOKENS, c))
         w = _upcast(torch.stack(betas), grad_out.dtype, name)
         launch.read(grad_out, w, out=out.unbind(0))
@@ -186,7 +195,12 @@ def _make_final_accumulate(tag: str):
 
     def grad_beta_impl(grad_out: Tensor, *dzs: Tensor) -> Tensor:
         """fp32 [E,C,S] = sum over tokens of grad_out[cell slot s] * dz_e (atomics-free)."""
-        _require_packed(f"{name}_grad_beta_ptr", grad_out=grad_out)
+        b, c = check_grad(f"{name}_grad_beta_ptr", grad_out)
+        _require_packed(f"{name}_grad_beta_ptr", **dict(zip(dz_names, dzs)))
+        _check_cuda(f"{name}_grad_beta_ptr", grad_out, *dzs)
+        for i, dz in enumerate(dzs):
+            if tuple(dz.shape) != (b, WORKSPACE_TOKENS, c):
+                raise ValueError(f"{name} dz{i} must be [{b},{WORKSPACE_TOKENS},{c}], got {tuple(dz.shape)}")
         ups = [_upcast(d, grad_out.dtype, name) for d in dzs]
         return launch.weight_grad(grad_out, ups, None, out_dtype=torch.float32, slots=slots)
 

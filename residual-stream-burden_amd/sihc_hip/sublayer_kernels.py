@@ -183,6 +183,7 @@ def sublayer_triangular(base: Tensor, updates: list[Tensor], gamma: Tensor) -> T
 @custom_op("sihc::sublayer_triangular_gamma_backward", mutates_args=())
 def _tri_gamma_backward(grad: Tensor, updates: list[Tensor], gamma: Tensor) -> Tensor:
     """dgamma_j = sum over rows of grad * dz_j, fp32 then cast (reference :355-361)."""
+    _validate_triangular(grad, updates, gamma)
     return launch.triangular_gamma_grad(grad, updates, gamma)
 
 
@@ -192,8 +193,9 @@ def _tri_backward(grad: Tensor, updates: list[Tensor], gamma: Tensor) -> tuple[T
 
     Same values as the reference's backward (:369-379: fp32 products cast to the
     workspace dtype, and `_tri_gamma_backward`), with grad read once instead of A + 1
-    times.
+    times. Saved tensors come back through the caller's hooks, so they are checked again.
     """
+    _validate_triangular(grad, updates, gamma)
     return launch.triangular_backward(grad, updates, gamma)
 
 
