@@ -218,7 +218,7 @@ def _make_final_accumulate(tag: str):
         saved = ctx.saved_tensors
         dzs, betas = saved[:blocks], saved[blocks:]
         grad_out = grad_out.contiguous()
-        if dzs[0].dtype == grad_out.dtype and not torch.is_grad_enabled():
+        if not torch.is_grad_enabled() and all(t.dtype == grad_out.dtype for t in saved):
             # one pass, the weight gradients reduced in fp32 and stored in the betas' dtype
             gdz, gbeta = _write_grads(grad_out, list(dzs), torch.stack(betas))
             return (grad_out, *gdz, *gbeta.unbind(0))

@@ -268,3 +268,22 @@ def test_few_event_reductions_direct_and_staged(events, c, dtype):
     for j in range(events):
         assert torch.equal(ddz[j].cpu(), rdz[j]), f"update gradient {j} not bit-exact"
     assert_parity(dg, rdg, torch.float32, what="gamma grad")
+
+
+@pytest.mark.parametrize("kept", ["updates", "weights", "both"])
+def test_final_accumulate_widens_bf16_copies_of_saved_tensors(kept):
+    """fp32 training whose saved-tensor hooks keep the updates, the weights or both as bf16
+    copies: the gradients of the widened values. The values here are bf16 ones, so the copies
+    lose nothing, and a sum of 512 fp32 products differs by its order alone (2^-24 x 512)."""
+    torch.manual_seed(7)
+    x = torch.randn(2, 32, 32, 24, device="cuda").requires_grad_()
+    dzs = [torch.randn(2, 256, 24, device="cuda").bfloat16().float().requires_grad_() for _ in range(12)]
+    betas = [torch.randn(24, 4, device="cuda").bfloat16().float().requires_grad_() for _ in range(12)]
+    up = torch.randn_like(x)
+    op = torch.ops.sihc.final_accumulate_p8_12_traceable
+    want = torch.autograd.grad(op(x, *dzs, *betas), (x, *dzs, *betas), up)
+    dims = {"updates": (3,), "weights": (2,), "both": (2, 3)}[kept]
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.bfloat16() if t.ndim in dims else t, lambda t: t):
+        out = op(x, *dzs, *betas)
+    for a, b in zip(torch.autograd.grad(out, (x, *dzs, *betas), up), want):
+        assert a.dtype == b.dtype and (a - b).norm() <= 512 * 2 ** -24 * b.norm()
