@@ -14,7 +14,9 @@
 // same holds in a backward: under create_graph, or where a mode or a wrapped tensor shows up
 // there, the node calls the registered ops through the dispatcher. Inputs are kept with
 // save_for_backward, so saved-tensor hooks and version checks apply, and undefined output
-// gradients are materialised as zeros, as for the Python ops.
+// gradients are materialised as zeros, as for the Python ops. An unpack hook may return another
+// type, shape, layout or device than was saved, so every backward repeats the forward's checks on
+// what it got, and leaves operands that do not fit to the registered ops, which raise.
 
 #include <Python.h>
 
@@ -31,6 +33,7 @@
 
 #include <algorithm>
 #include <optional>
+#include <string>
 #include <tuple>
 #include <vector>
 
@@ -109,6 +112,57 @@ bool token_shape(const Tensor& z, const Tensor& x, const Shape& s) {
 bool index_shape(const Tensor& index, const Tensor& x, const Shape& s) {
   return index.scalar_type() == at::kInt && index.dim() == 2 && index.size(0) == s.batch &&
          index.size(1) == s.grid * s.grid && index.device() == x.device();
+}
+
+// Everything the launches below take for granted about their operands: asked by the Python
+// entries of the arguments and by the backward nodes of the gradients and unpacked tensors.
+bool read_fits(const Tensor& x, const Tensor& alpha, const Tensor& index, Shape& s) {
+  return plain(x) && plain(alpha) && alpha.dim() == 3 && alpha.size(0) >= 1 && alpha.size(0) <= SIHC_MAX_EVENTS &&
+         carrier_shape(x, alpha, s) && (!index.defined() || (plain(index) && index_shape(index, x, s)));
+}
+// (also the adjoint of the read, whose gradients have the updates' shape)
+bool write_fits(const Tensor& x, TensorList updates, const Tensor& beta, const Tensor& index, Shape& s) {
+  if (!read_fits(x, beta, index, s) || beta.size(0) != int64_t(updates.size())) return false;
+  for (const Tensor& u : updates)
+    if (!plain(u) || !token_shape(u, x, s)) return false;
+  return true;
+}
+bool triangular_fits(const Tensor& base, TensorList updates, const Tensor& gamma) {
+  if (!plain(base) || !plain(gamma) || base.dim() < 1 || base.numel() == 0 || dtype_code(base) < 0 ||
+      updates.empty() || updates.size() > SIHC_MAX_EVENTS || gamma.dim() != 2 ||
+      gamma.size(0) != int64_t(updates.size()) || gamma.size(1) != base.size(-1) ||
+      gamma.device() != base.device() ||
+      (gamma.scalar_type() != base.scalar_type() && gamma.scalar_type() != at::kFloat))
+    return false;
+  for (const Tensor& u : updates)
+    if (!plain(u) || !u.sizes().equals(base.sizes()) || u.scalar_type() != base.scalar_type() ||
+        u.device() != base.device())
+      return false;
+  return true;
+}
+bool event_fits(const Tensor& x, const Tensor& dz, const Tensor& beta, const Tensor& alpha) {
+  Shape s{};
+  return plain(x) && plain(dz) && plain(beta) && plain(alpha) && beta.dim() == 2 && carrier_shape(x, beta, s) &&
+         token_shape(dz, x, s) && alpha.sizes().equals(beta.sizes()) && alpha.scalar_type() == x.scalar_type() &&
+         alpha.device() == x.device();
+}
+bool gather_fits(const Tensor& x, const Tensor& index, int64_t slots) {
+  if (!plain(x) || !plain(index)) return false;
+  const int64_t k = slots == 4 ? 2 : 4;
+  if (x.dim() != 4 || x.numel() == 0 || dtype_code(x) < 0 || (slots != 4 && slots != 16) ||
+      x.size(1) != x.size(2) || x.size(1) % k != 0 || x.size(3) >= (int64_t(1) << 31))
+    return false;
+  const Shape s{x.size(0), x.size(1) / k, k, x.size(3), slots};
+  // (the adjoint holds a batch row of the index in LDS: 16384 cells)
+  return index_shape(index, x, s) && s.grid <= 128;
+}
+bool scatter_fits(const Tensor& cells, const Tensor& index) {
+  if (!plain(cells) || !plain(index) || cells.dim() != 4 || cells.numel() == 0 || dtype_code(cells) < 0 ||
+      (cells.size(2) != 4 && cells.size(2) != 16) || cells.size(1) > 16384 || cells.size(3) >= (int64_t(1) << 31))
+    return false;
+  Shape s{cells.size(0), 1, cells.size(2) == 4 ? 2 : 4, cells.size(3), cells.size(2)};
+  while (s.grid * s.grid < cells.size(1)) ++s.grid;
+  return s.grid * s.grid == cells.size(1) && index_shape(index, cells, s);
 }
 
 // ----------------------------------------------------------------------- the C-ABI calls
@@ -198,12 +252,8 @@ template <typename Sig>
 auto registered(const char* name) {
   return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Sig>();
 }
-bool plain_all(TensorList ts) {
-  if (at::GradMode::is_enabled() || !plain_mode()) return false;
-  for (const Tensor& t : ts)
-    if (!plain(t)) return false;
-  return true;
-}
+// A backward may launch directly: nothing recorded or in force (its operands are asked apart).
+bool direct() { return !at::GradMode::is_enabled() && plain_mode(); }
 
 // ------------------------------------------------------------------------ autograd nodes
 struct ReadFn : torch::autograd::Function<ReadFn> {
@@ -218,11 +268,9 @@ struct ReadFn : torch::autograd::Function<ReadFn> {
     const auto saved = ctx->get_saved_variables();
     const Tensor &x = saved[0], &alpha = saved[1], &index = saved[2];
     for (Tensor& g : grads) g = g.contiguous();
-    variable_list all = grads;
-    all.push_back(x);
-    all.push_back(alpha);
     std::tuple<Tensor, Tensor> r;
-    if (plain_all(all)) {
+    Shape s{};
+    if (direct() && write_fits(x, grads, alpha, index, s)) {
       r = run_read_backward(x, grads, alpha, index);
     } else if (index.defined()) {
       static auto op = registered<std::tuple<Tensor, Tensor>(const Tensor&, TensorList, const Tensor&,
@@ -252,12 +300,10 @@ struct WriteFn : torch::autograd::Function<WriteFn> {
     const Tensor &beta = saved[0], &index = saved[1];
     const variable_list updates(saved.begin() + 2, saved.end());
     const Tensor grad = grads[0].contiguous();
-    variable_list all = updates;
-    all.push_back(grad);
-    all.push_back(beta);
     variable_list dz;
     Tensor db;
-    if (plain_all(all)) {
+    Shape s{};
+    if (direct() && write_fits(grad, updates, beta, index, s)) {
       std::tie(dz, db) = run_write_backward(grad, updates, beta, index);
     } else if (index.defined()) {
       static auto read =
@@ -304,11 +350,8 @@ struct TriangularFn : torch::autograd::Function<TriangularFn> {
     const Tensor& gamma = saved[0];
     const variable_list updates(saved.begin() + 1, saved.end());
     const Tensor grad = grads[0].contiguous();
-    variable_list all = updates;
-    all.push_back(grad);
-    all.push_back(gamma);
     variable_list out{grad};
-    if (plain_all(all)) {
+    if (direct() && triangular_fits(grad, updates, gamma)) {
       const c10::DeviceGuard guard(grad.device());
       const int64_t c = grad.size(-1), rows = grad.numel() / c;
       const int active = int(updates.size());
@@ -362,7 +405,8 @@ struct EventFn : torch::autograd::Function<EventFn> {
     const auto saved = ctx->get_saved_variables();
     const Tensor &xo = saved[0], &dz = saved[1], &beta = saved[2], &alpha = saved[3];
     const Tensor gx = grads[0].contiguous(), gz = grads[1].contiguous();
-    if (!plain_all({gx, gz, xo, dz, beta, alpha})) {
+    if (!direct() || !event_fits(xo, dz, beta, alpha) || !event_fits(gx, gz, beta, alpha) ||
+        !gx.sizes().equals(xo.sizes()) || gx.scalar_type() != xo.scalar_type()) {
       static auto op = registered<std::tuple<Tensor, Tensor, Tensor, Tensor>(
           const std::optional<Tensor>&, const std::optional<Tensor>&, const Tensor&, const Tensor&, const Tensor&,
           const Tensor&)>("sihc::event_write_read_backward");
@@ -388,35 +432,56 @@ struct EventFn : torch::autograd::Function<EventFn> {
 // gradients are rows of one [E, C, S] result in the weights' type.
 struct BlockWriteFn : torch::autograd::Function<BlockWriteFn> {
   static constexpr bool is_traceable = true;
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, TensorList updates, TensorList betas) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, TensorList updates, TensorList betas,
+                        const std::string& name) {
+    ctx->saved_data["name"] = name;
     variable_list keep(updates.begin(), updates.end());
     keep.insert(keep.end(), betas.begin(), betas.end());
     ctx->save_for_backward(keep);
     return run_write(x, updates, at::stack(betas), Tensor());
   }
+  // Updates and one [C, S] weight tensor each, of one type, for a carrier of 16 x 16 cells.
+  static bool fits(const Tensor& x, const variable_list& updates, const variable_list& betas) {
+    Shape s{};
+    if (!plain(x)) return false;
+    for (size_t i = 0; i < updates.size(); ++i) {
+      const Tensor &u = updates[i], &w = betas[i];
+      if (!plain(u) || !plain(w) || w.dim() != 2 || w.size(1) != betas[0].size(1) || !carrier_shape(x, w, s) ||
+          s.grid != 16 || !token_shape(u, x, s))
+        return false;
+    }
+    return true;
+  }
+  static variable_list finish(variable_list out) {
+    out.emplace_back();  // the op's name
+    return out;
+  }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
     const size_t n = saved.size() / 2;
     const variable_list updates(saved.begin(), saved.begin() + long(n)), betas(saved.begin() + long(n), saved.end());
-    const Tensor grad = grads[0].contiguous(), beta = at::stack(betas);
-    variable_list all = updates;
-    all.push_back(grad);
-    all.push_back(beta);
-    variable_list dz;
-    Tensor db;
-    if (plain_all(all)) {
-      std::tie(dz, db) = run_write_backward(grad, updates, beta, Tensor());
-    } else {
-      static auto read = registered<std::vector<Tensor>(const Tensor&, const Tensor&)>("sihc::sublayer_read");
-      static auto wgrad =
-          registered<Tensor(const Tensor&, TensorList, const Tensor&)>("sihc::sublayer_weight_grad");
-      dz = read.call(grad, beta);
-      db = wgrad.call(grad, updates, beta);
+    const Tensor grad = grads[0].contiguous();
+    if (direct() && fits(grad, updates, betas)) {
+      const auto [dz, db] = run_write_backward(grad, updates, at::stack(betas), Tensor());
+      variable_list out{grad};
+      out.insert(out.end(), dz.begin(), dz.end());
+      for (const Tensor& t : db.unbind(0)) out.push_back(t);
+      return finish(std::move(out));
     }
+    // the gradient ops of the legacy family, which widen bf16 updates and weights to fp32
+    const std::string name = ctx->saved_data["name"].toStringRef();
+    auto gradient_op = [&](const char* which, const variable_list& rest) {
+      const auto op = c10::Dispatcher::singleton().findSchemaOrThrow((name + which).c_str(), "");
+      torch::jit::Stack stack{grad};
+      for (const Tensor& t : rest) stack.emplace_back(t);
+      op.callBoxed(stack);
+      return stack.back().toTensor();
+    };
     variable_list out{grad};
-    out.insert(out.end(), dz.begin(), dz.end());
-    for (const Tensor& t : db.unbind(0)) out.push_back(t);
-    return out;
+    for (const Tensor& t : gradient_op("_grad_dz_ptr", betas).unbind(0)) out.push_back(t);
+    const variable_list db = gradient_op("_grad_beta_ptr", updates).unbind(0);
+    for (size_t i = 0; i < n; ++i) out.push_back(db[i].to(betas[i].scalar_type()));
+    return finish(std::move(out));
   }
 };
 
@@ -449,7 +514,7 @@ struct GatherFn : torch::autograd::Function<GatherFn> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const Tensor index = ctx->get_saved_variables()[0], grad = grads[0].contiguous();
-    if (plain_all({grad, index})) return {run_scatter(sihc_scatter_add_cells, grad, index, false), Tensor(), Tensor()};
+    if (direct() && scatter_fits(grad, index)) return {run_scatter(sihc_scatter_add_cells, grad, index, false), Tensor(), Tensor()};
     static auto op = registered<Tensor(const Tensor&, const Tensor&)>("sihc::scatter_add_cells");
     return {op.call(grad, index), Tensor(), Tensor()};
   }
@@ -464,7 +529,7 @@ struct ScatterFn : torch::autograd::Function<ScatterFn> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const Tensor index = ctx->get_saved_variables()[0], grad = grads[0].contiguous();
     const int64_t slots = ctx->saved_data["slots"].toInt();
-    if (plain_all({grad, index})) return {run_gather(grad, index, slots), Tensor()};
+    if (direct() && gather_fits(grad, index, slots)) return {run_gather(grad, index, slots), Tensor()};
     static auto op = registered<Tensor(const Tensor&, const Tensor&, int64_t)>("sihc::gather_cells");
     return {op.call(grad, index, slots), Tensor()};
   }
@@ -507,9 +572,7 @@ PyObject* read_impl(const char* name, PyObject* const* args, bool indexed) {
     Tensor x, alpha, index;
     Shape s{};
     if (!unwrap(args[0], x) || !unwrap(args[1], alpha) || (indexed && !unwrap(args[2], index))) return not_implemented();
-    if (!plain(x) || !plain(alpha) || alpha.dim() != 3 || alpha.size(0) < 1 || alpha.size(0) > SIHC_MAX_EVENTS ||
-        !carrier_shape(x, alpha, s) || (indexed && (!plain(index) || !index_shape(index, x, s))))
-      return not_implemented();
+    if ((indexed && !index.defined()) || !read_fits(x, alpha, index, s)) return not_implemented();
     return to_list(unrecorded() ? run_read(x, alpha, index) : ReadFn::apply(x, alpha, maybe(index)));
   });
 }
@@ -521,12 +584,7 @@ PyObject* write_impl(const char* name, PyObject* const* args, bool indexed) {
     if (!unwrap(args[0], x) || !unwrap_list(args[1], updates) || !unwrap(args[2], beta) ||
         (indexed && !unwrap(args[3], index)))
       return not_implemented();
-    if (!plain(x) || !plain(beta) || beta.dim() != 3 || updates.empty() || updates.size() > SIHC_MAX_EVENTS ||
-        beta.size(0) != int64_t(updates.size()) || !carrier_shape(x, beta, s) ||
-        (indexed && (!plain(index) || !index_shape(index, x, s))))
-      return not_implemented();
-    for (const Tensor& u : updates)
-      if (!plain(u) || !token_shape(u, x, s)) return not_implemented();
+    if ((indexed && !index.defined()) || !write_fits(x, updates, beta, index, s)) return not_implemented();
     return THPVariable_Wrap(unrecorded() ? run_write(x, updates, beta, index)
                                          : WriteFn::apply(x, TensorList(updates), beta, maybe(index)));
   });
@@ -550,16 +608,7 @@ PyObject* py_triangular(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Tensor base, gamma;
     std::vector<Tensor> updates;
     if (!unwrap(args[0], base) || !unwrap_list(args[1], updates) || !unwrap(args[2], gamma)) return not_implemented();
-    if (!plain(base) || !plain(gamma) || base.dim() < 1 || base.numel() == 0 || dtype_code(base) < 0 ||
-        updates.empty() || updates.size() > SIHC_MAX_EVENTS || gamma.dim() != 2 ||
-        gamma.size(0) != int64_t(updates.size()) || gamma.size(1) != base.size(-1) ||
-        gamma.device() != base.device() ||
-        (gamma.scalar_type() != base.scalar_type() && gamma.scalar_type() != at::kFloat))
-      return not_implemented();
-    for (const Tensor& u : updates)
-      if (!plain(u) || !u.sizes().equals(base.sizes()) || u.scalar_type() != base.scalar_type() ||
-          u.device() != base.device())
-        return not_implemented();
+    if (!triangular_fits(base, updates, gamma)) return not_implemented();
     return THPVariable_Wrap(unrecorded() ? run_triangular(base, updates, gamma)
                                          : TriangularFn::apply(base, TensorList(updates), gamma));
   });
@@ -568,13 +617,9 @@ PyObject* py_event(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 4) return not_implemented();
   return guarded("sihc::event_write_read", [&]() -> PyObject* {
     Tensor x, dz, beta, alpha;
-    Shape s{};
     if (!unwrap(args[0], x) || !unwrap(args[1], dz) || !unwrap(args[2], beta) || !unwrap(args[3], alpha))
       return not_implemented();
-    if (!plain(x) || !plain(dz) || !plain(beta) || !plain(alpha) || beta.dim() != 2 ||
-        !carrier_shape(x, beta, s) || !token_shape(dz, x, s) || !alpha.sizes().equals(beta.sizes()) ||
-        alpha.scalar_type() != x.scalar_type() || alpha.device() != x.device())
-      return not_implemented();
+    if (!event_fits(x, dz, beta, alpha)) return not_implemented();
     const variable_list out = unrecorded() ? run_event(x, dz, beta, alpha) : EventFn::apply(x, dz, beta, alpha);
     PyObject* pair = PyTuple_New(2);
     for (int i = 0; pair && i < 2; ++i) PyTuple_SET_ITEM(pair, i, THPVariable_Wrap(out[size_t(i)]));
@@ -582,24 +627,25 @@ PyObject* py_event(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
-// (carrier edge, blocks, slots, x0, dz_0.., beta_0..)
+// (op name without its suffix, carrier edge, blocks, slots, x0, dz_0.., beta_0..)
 PyObject* py_block_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n < 4) return not_implemented();
-  const long edge = PyLong_AsLong(args[0]), blocks = PyLong_AsLong(args[1]), slots = PyLong_AsLong(args[2]);
-  if (n != 4 + 2 * blocks) return not_implemented();
+  if (n < 5) return not_implemented();
+  const char* name = PyUnicode_AsUTF8(args[0]);
+  if (!name) return nullptr;
+  const long edge = PyLong_AsLong(args[1]), blocks = PyLong_AsLong(args[2]), slots = PyLong_AsLong(args[3]);
+  if (n != 5 + 2 * blocks) return not_implemented();
   return guarded("sihc::final_accumulate", [&]() -> PyObject* {
     Tensor x;
     std::vector<Tensor> updates(static_cast<size_t>(blocks)), betas(static_cast<size_t>(blocks));
-    if (!unwrap(args[3], x) || !plain(x) || x.dim() != 4 || x.size(1) != edge) return not_implemented();
-    Shape s{};
-    for (long i = 0; i < blocks; ++i) {
-      Tensor &u = updates[size_t(i)], &w = betas[size_t(i)];
-      if (!unwrap(args[4 + i], u) || !unwrap(args[4 + blocks + i], w) || !plain(u) || !plain(w) || w.dim() != 2 ||
-          w.size(1) != slots || !carrier_shape(x, w, s) || s.grid != 16 || !token_shape(u, x, s))
+    if (!unwrap(args[4], x)) return not_implemented();
+    for (long i = 0; i < blocks; ++i)
+      if (!unwrap(args[5 + i], updates[size_t(i)]) || !unwrap(args[5 + blocks + i], betas[size_t(i)]))
         return not_implemented();
-    }
-    return THPVariable_Wrap(unrecorded() ? run_write(x, updates, at::stack(betas), Tensor())
-                                         : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas)));
+    if (!BlockWriteFn::fits(x, updates, betas) || x.size(1) != edge || betas[0].size(1) != slots)
+      return not_implemented();
+    return THPVariable_Wrap(unrecorded()
+                                ? run_write(x, updates, at::stack(betas), Tensor())
+                                : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas), std::string(name)));
   });
 }
 PyObject* py_gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -607,14 +653,7 @@ PyObject* py_gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const long slots = PyLong_AsLong(args[2]);
   return guarded("sihc::gather_cells", [&]() -> PyObject* {
     Tensor x, index;
-    if (!unwrap(args[0], x) || !unwrap(args[1], index) || !plain(x) || !plain(index)) return not_implemented();
-    const int64_t k = slots == 4 ? 2 : 4;
-    if (x.dim() != 4 || x.numel() == 0 || dtype_code(x) < 0 || (slots != 4 && slots != 16) ||
-        x.size(1) != x.size(2) || x.size(1) % k != 0 || x.size(3) >= (int64_t(1) << 31))
-      return not_implemented();
-    const Shape s{x.size(0), x.size(1) / k, k, x.size(3), slots};
-    // (the adjoint holds a batch row of the index in LDS: 16384 cells)
-    if (!index_shape(index, x, s) || s.grid > 128) return not_implemented();
+    if (!unwrap(args[0], x) || !unwrap(args[1], index) || !gather_fits(x, index, slots)) return not_implemented();
     return THPVariable_Wrap(unrecorded() ? run_gather(x, index, slots) : GatherFn::apply(x, index, int64_t(slots)));
   });
 }
@@ -622,13 +661,7 @@ PyObject* py_scatter(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 2) return not_implemented();
   return guarded("sihc::scatter_cells", [&]() -> PyObject* {
     Tensor cells, index;
-    if (!unwrap(args[0], cells) || !unwrap(args[1], index) || !plain(cells) || !plain(index)) return not_implemented();
-    if (cells.dim() != 4 || cells.numel() == 0 || dtype_code(cells) < 0 ||
-        (cells.size(2) != 4 && cells.size(2) != 16) || cells.size(1) > 16384 || cells.size(3) >= (int64_t(1) << 31))
-      return not_implemented();
-    Shape s{cells.size(0), 1, cells.size(2) == 4 ? 2 : 4, cells.size(3), cells.size(2)};
-    while (s.grid * s.grid < cells.size(1)) ++s.grid;
-    if (s.grid * s.grid != cells.size(1) || !index_shape(index, cells, s)) return not_implemented();
+    if (!unwrap(args[0], cells) || !unwrap(args[1], index) || !scatter_fits(cells, index)) return not_implemented();
     return THPVariable_Wrap(unrecorded() ? run_scatter(sihc_scatter_cells, cells, index, true)
                                          : ScatterFn::apply(cells, index));
   });

@@ -274,7 +274,8 @@ def test_few_event_reductions_direct_and_staged(events, c, dtype):
 def test_final_accumulate_widens_bf16_copies_of_saved_tensors(kept):
     """fp32 training whose saved-tensor hooks keep the updates, the weights or both as bf16
     copies: the gradients of the widened values. The values here are bf16 ones, so the copies
-    lose nothing, and a sum of 512 fp32 products differs by its order alone (2^-24 x 512)."""
+    lose nothing, and a sum of 512 fp32 products differs by its order alone (2^-24 x 512). A
+    weight gradient is stored in the kept weights' type (one rounding, 2^-9 in bf16)."""
     torch.manual_seed(7)
     x = torch.randn(2, 32, 32, 24, device="cuda").requires_grad_()
     dzs = [torch.randn(2, 256, 24, device="cuda").bfloat16().float().requires_grad_() for _ in range(12)]
@@ -286,4 +287,5 @@ def test_final_accumulate_widens_bf16_copies_of_saved_tensors(kept):
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t.bfloat16() if t.ndim in dims else t, lambda t: t):
         out = op(x, *dzs, *betas)
     for a, b in zip(torch.autograd.grad(out, (x, *dzs, *betas), up), want):
-        assert a.dtype == b.dtype and (a - b).norm() <= 512 * 2 ** -24 * b.norm()
+        bound = 2 ** -9 if a.ndim == 2 and 2 in dims else 512 * 2 ** -24
+        assert a.dtype == b.dtype and (a - b).norm() <= bound * b.norm()

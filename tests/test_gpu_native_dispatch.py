@@ -170,6 +170,59 @@ def test_saved_tensor_hooks_and_version_checks():
         _grads(out, (x, w))
 
 
+def _with_one_changed(op, args, place, change):
+    """op(*args) whose backward gets change(t) in place of the saved tensor number `place`."""
+    packed = []
+
+    def pack(t):
+        packed.append(t)
+        return len(packed) - 1, t
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda v: change(v[1]) if v[0] == place else v[1]):
+        return _outs(op(*args)), packed
+
+
+CHANGES = {"cast": lambda t: t.long() if t.dtype == torch.int32 else
+           t.to(torch.bfloat16 if t.dtype == torch.float32 else torch.float32),
+           "narrowed": lambda t: t[..., :-1].contiguous(),
+           "strided": lambda t: t.repeat_interleave(2, -1)[..., ::2],
+           "on the host": lambda t: t.cpu()}
+
+
+@pytest.mark.parametrize("change", list(CHANGES))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("name", NAMES)
+def test_unpacked_tensors_that_do_not_fit_are_refused(name, dtype, change):
+    """An unpack hook may return anything: the backward checks what it got, tensor by tensor,
+    before it launches. (Widening bf16 weights or updates is the legacy write's own contract, and
+    a gamma may be of either type.)"""
+    op, args, _ = _calls(dtype)[name]
+    _, saved = _with_one_changed(op, args, None, None)
+    for place in range(len(saved)):
+        if change == "cast" and (name == "final_accumulate" and dtype == torch.float32
+                                 or name == "triangular" and dtype == torch.bfloat16 and place == 0):
+            continue
+        if change == "strided" and name == "final_accumulate" and place >= 12:
+            continue  # its weights are stacked, and so packed, first
+        out, _ = _with_one_changed(op, args, place, CHANGES[change])
+        assert _is_native(out[0])
+        with pytest.raises((ValueError, RuntimeError)):
+            _grads(out, args)
+
+
+@pytest.mark.parametrize("dims", [(2, 3), (2,), (3,)], ids=["both", "weights", "updates"])
+def test_bf16_copies_of_the_legacy_write_are_widened(dims):
+    """fp32 training whose hooks keep the updates or weights as bf16 copies: the registered op's
+    gradients bit for bit (it widens the copies)."""
+    op, args, registered = _calls(torch.float32)["final_accumulate"]
+    both = []
+    for f in (op, registered):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.bfloat16() if t.ndim in dims else t, lambda t: t):
+            out = _outs(f(*args))
+        both.append(_grads(out, args))
+    assert all(a.dtype == b.dtype and torch.equal(a, b) for a, b in zip(*both))
+
+
 @pytest.mark.parametrize("name", NAMES)
 def test_an_error_of_a_saved_tensor_hook_reaches_the_caller_once(name):
     """Checkpointing ends its recomputation by raising from the pack hook of the last tensor."""
