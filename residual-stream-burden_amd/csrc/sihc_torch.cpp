@@ -563,6 +563,17 @@ PyObject* guarded(const char* name, F&& f) {
     return not_implemented();
   }
 }
+// f() with the GIL released: a launch waits where the queue is full, and an allocation may wait for
+// the device. (The registered ops release it around every dispatch and launch.) Saved-tensor hooks
+// take it again for their own calls.
+template <typename F>
+auto without_gil(F&& f) {
+  struct Released {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  return f();
+}
 // Below autograd (a custom op's own body, inference mode) and under no_grad nothing is recorded.
 bool unrecorded() { return !at::GradMode::is_enabled() || below_autograd(); }
 std::optional<Tensor> maybe(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
@@ -573,7 +584,8 @@ PyObject* read_impl(const char* name, PyObject* const* args, bool indexed) {
     Shape s{};
     if (!unwrap(args[0], x) || !unwrap(args[1], alpha) || (indexed && !unwrap(args[2], index))) return not_implemented();
     if ((indexed && !index.defined()) || !read_fits(x, alpha, index, s)) return not_implemented();
-    return to_list(unrecorded() ? run_read(x, alpha, index) : ReadFn::apply(x, alpha, maybe(index)));
+    return to_list(without_gil(
+        [&] { return unrecorded() ? run_read(x, alpha, index) : ReadFn::apply(x, alpha, maybe(index)); }));
   });
 }
 PyObject* write_impl(const char* name, PyObject* const* args, bool indexed) {
@@ -585,8 +597,10 @@ PyObject* write_impl(const char* name, PyObject* const* args, bool indexed) {
         (indexed && !unwrap(args[3], index)))
       return not_implemented();
     if ((indexed && !index.defined()) || !write_fits(x, updates, beta, index, s)) return not_implemented();
-    return THPVariable_Wrap(unrecorded() ? run_write(x, updates, beta, index)
-                                         : WriteFn::apply(x, TensorList(updates), beta, maybe(index)));
+    return THPVariable_Wrap(without_gil([&] {
+      return unrecorded() ? run_write(x, updates, beta, index)
+                          : WriteFn::apply(x, TensorList(updates), beta, maybe(index));
+    }));
   });
 }
 
@@ -609,8 +623,10 @@ PyObject* py_triangular(PyObject*, PyObject* const* args, Py_ssize_t n) {
     std::vector<Tensor> updates;
     if (!unwrap(args[0], base) || !unwrap_list(args[1], updates) || !unwrap(args[2], gamma)) return not_implemented();
     if (!triangular_fits(base, updates, gamma)) return not_implemented();
-    return THPVariable_Wrap(unrecorded() ? run_triangular(base, updates, gamma)
-                                         : TriangularFn::apply(base, TensorList(updates), gamma));
+    return THPVariable_Wrap(without_gil([&] {
+      return unrecorded() ? run_triangular(base, updates, gamma)
+                          : TriangularFn::apply(base, TensorList(updates), gamma);
+    }));
   });
 }
 PyObject* py_event(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -620,7 +636,8 @@ PyObject* py_event(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!unwrap(args[0], x) || !unwrap(args[1], dz) || !unwrap(args[2], beta) || !unwrap(args[3], alpha))
       return not_implemented();
     if (!event_fits(x, dz, beta, alpha)) return not_implemented();
-    const variable_list out = unrecorded() ? run_event(x, dz, beta, alpha) : EventFn::apply(x, dz, beta, alpha);
+    const variable_list out = without_gil(
+        [&] { return unrecorded() ? run_event(x, dz, beta, alpha) : EventFn::apply(x, dz, beta, alpha); });
     PyObject* pair = PyTuple_New(2);
     for (int i = 0; pair && i < 2; ++i) PyTuple_SET_ITEM(pair, i, THPVariable_Wrap(out[size_t(i)]));
     return pair;
@@ -643,9 +660,10 @@ PyObject* py_block_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
         return not_implemented();
     if (!BlockWriteFn::fits(x, updates, betas) || x.size(1) != edge || betas[0].size(1) != slots)
       return not_implemented();
-    return THPVariable_Wrap(unrecorded()
-                                ? run_write(x, updates, at::stack(betas), Tensor())
-                                : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas), std::string(name)));
+    return THPVariable_Wrap(without_gil([&] {
+      return unrecorded() ? run_write(x, updates, at::stack(betas), Tensor())
+                          : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas), std::string(name));
+    }));
   });
 }
 PyObject* py_gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -654,7 +672,8 @@ PyObject* py_gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded("sihc::gather_cells", [&]() -> PyObject* {
     Tensor x, index;
     if (!unwrap(args[0], x) || !unwrap(args[1], index) || !gather_fits(x, index, slots)) return not_implemented();
-    return THPVariable_Wrap(unrecorded() ? run_gather(x, index, slots) : GatherFn::apply(x, index, int64_t(slots)));
+    return THPVariable_Wrap(without_gil(
+        [&] { return unrecorded() ? run_gather(x, index, slots) : GatherFn::apply(x, index, int64_t(slots)); }));
   });
 }
 PyObject* py_scatter(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -662,8 +681,9 @@ PyObject* py_scatter(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded("sihc::scatter_cells", [&]() -> PyObject* {
     Tensor cells, index;
     if (!unwrap(args[0], cells) || !unwrap(args[1], index) || !scatter_fits(cells, index)) return not_implemented();
-    return THPVariable_Wrap(unrecorded() ? run_scatter(sihc_scatter_cells, cells, index, true)
-                                         : ScatterFn::apply(cells, index));
+    return THPVariable_Wrap(without_gil([&] {
+      return unrecorded() ? run_scatter(sihc_scatter_cells, cells, index, true) : ScatterFn::apply(cells, index);
+    }));
   });
 }
 

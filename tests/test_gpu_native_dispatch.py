@@ -7,6 +7,10 @@ subclasses, no_grad and inference mode, version checks; what it refuses is still
 """
 from __future__ import annotations
 
+import sys
+import threading
+import time
+
 import pytest
 import torch
 import torch.utils.checkpoint
@@ -243,6 +247,38 @@ def test_an_error_of_a_saved_tensor_hook_reaches_the_caller_once(name):
     again = torch.utils.checkpoint.checkpoint(region, use_reentrant=False)
     assert _is_native(again[0])
     assert all(torch.equal(a, b) for a, b in zip(_grads(again, args), _grads(region(), args)))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_other_threads_run_during_a_native_call(name):
+    """The GIL is free while a call allocates and launches. With a switch interval that no thread
+    outlives, another thread runs only where this one gives the GIL up: inside a call."""
+    op, args, _ = _calls(torch.float32)[name]
+    op(*args)
+    entry, inside, stop, seen = op._sihc_entry, [False], [False], []
+
+    def watch():
+        while not stop[0]:
+            if inside[0]:
+                seen.append(1)
+            time.sleep(0)
+
+    other, interval = threading.Thread(target=watch), sys.getswitchinterval()
+    try:
+        sys.setswitchinterval(20.0)
+        other.start()
+        for _ in range(5000):
+            inside[0] = True
+            out = entry(*args)
+            inside[0] = False
+            del out
+            if seen:
+                break
+    finally:
+        stop[0] = True
+        sys.setswitchinterval(interval)
+        other.join()
+    assert seen
 
 
 def test_vmap_forward_mode_and_subclasses_take_the_registered_op():
