@@ -9,7 +9,8 @@
 // Plain means: exactly the tensors and shapes that the op accepts, all packed, dense, on one
 // GPU and not empty, of type torch.Tensor or torch.nn.Parameter, and nothing in force that has
 // to see the op: no dispatch or function mode (tracing, fake tensors, selective checkpointing),
-// no functorch transform, no forward-mode tangent. Anything else returns NotImplemented and
+// no functorch transform, no forward-mode tangent, and no kernel or autocast rule that the
+// program registered for the op itself. Anything else returns NotImplemented and
 // the caller runs the Python op, which validates, raises and composes as it always did. The
 // same holds in a backward: under create_graph, or where a mode or a wrapped tensor shows up
 // there, the node calls the registered ops through the dispatcher. Inputs are kept with
@@ -32,6 +33,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
+#include <cstring>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -469,7 +471,8 @@ struct BlockWriteFn : torch::autograd::Function<BlockWriteFn> {
       return finish(std::move(out));
     }
     // the gradient ops of the legacy family, which widen bf16 updates and weights to fp32
-    const std::string name = ctx->saved_data["name"].toStringRef();
+    std::string name = ctx->saved_data["name"].toStringRef();  // sihc::final_accumulate_<tag>_traceable
+    name.resize(name.rfind("_traceable"));
     auto gradient_op = [&](const char* which, const variable_list& rest) {
       const auto op = c10::Dispatcher::singleton().findSchemaOrThrow((name + which).c_str(), "");
       torch::jit::Stack stack{grad};
@@ -543,15 +546,30 @@ PyObject* to_list(const variable_list& ts) {
 }
 PyObject* not_implemented() { Py_RETURN_NOTIMPLEMENTED; }
 
+// One Python entry: the op that it stands for.
+struct Entry {
+  c10::OperatorHandle op;
+  const char* name() const { return op.operator_name().name.c_str(); }
+  // A custom op has kernels under alias keys only: one under these is the program's own.
+  bool overridden() const {
+    return op.hasKernelForDispatchKey(c10::DispatchKey::CUDA) ||
+           op.hasKernelForDispatchKey(c10::DispatchKey::AutogradCUDA) ||
+           op.hasKernelForDispatchKey(c10::DispatchKey::AutocastCUDA);
+  }
+};
+constexpr const char* ENTRY = "sihc_entry";
+const Entry& entry_of(PyObject* self) { return *static_cast<Entry*>(PyCapsule_GetPointer(self, ENTRY)); }
+
 // Run `f`; a C-ABI error, or a C++ exception, hands the call to the Python op, which repeats
 // the checks and raises what it always raised. A Python exception comes from the caller's own
 // code (a saved-tensor hook) and goes on to the caller: checkpointing ends its recomputation
 // by raising from such a hook, which must not run again for the same call.
 template <typename F>
-PyObject* guarded(const char* name, F&& f) {
+PyObject* guarded(PyObject* self, F&& f) {
   try {
-    if (!plain_mode()) return not_implemented();
-    RECORD_FUNCTION(name, std::vector<c10::IValue>());
+    const Entry& entry = entry_of(self);
+    if (!plain_mode() || entry.overridden()) return not_implemented();
+    RECORD_FUNCTION(entry.name(), std::vector<c10::IValue>());
     return f();
   } catch (const Failure&) {
     return not_implemented();
@@ -578,8 +596,8 @@ auto without_gil(F&& f) {
 bool unrecorded() { return !at::GradMode::is_enabled() || below_autograd(); }
 std::optional<Tensor> maybe(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 
-PyObject* read_impl(const char* name, PyObject* const* args, bool indexed) {
-  return guarded(name, [&]() -> PyObject* {
+PyObject* read_impl(PyObject* self, PyObject* const* args, bool indexed) {
+  return guarded(self, [&]() -> PyObject* {
     Tensor x, alpha, index;
     Shape s{};
     if (!unwrap(args[0], x) || !unwrap(args[1], alpha) || (indexed && !unwrap(args[2], index))) return not_implemented();
@@ -588,8 +606,8 @@ PyObject* read_impl(const char* name, PyObject* const* args, bool indexed) {
         [&] { return unrecorded() ? run_read(x, alpha, index) : ReadFn::apply(x, alpha, maybe(index)); }));
   });
 }
-PyObject* write_impl(const char* name, PyObject* const* args, bool indexed) {
-  return guarded(name, [&]() -> PyObject* {
+PyObject* write_impl(PyObject* self, PyObject* const* args, bool indexed) {
+  return guarded(self, [&]() -> PyObject* {
     Tensor x, beta, index;
     std::vector<Tensor> updates;
     Shape s{};
@@ -604,21 +622,21 @@ PyObject* write_impl(const char* name, PyObject* const* args, bool indexed) {
   });
 }
 
-PyObject* py_read(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  return n == 2 ? read_impl("sihc::sublayer_read", args, false) : not_implemented();
+PyObject* py_read(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+  return n == 2 ? read_impl(self, args, false) : not_implemented();
 }
-PyObject* py_indexed_read(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  return n == 3 ? read_impl("sihc::indexed_read", args, true) : not_implemented();
+PyObject* py_indexed_read(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+  return n == 3 ? read_impl(self, args, true) : not_implemented();
 }
-PyObject* py_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  return n == 3 ? write_impl("sihc::sublayer_write", args, false) : not_implemented();
+PyObject* py_write(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+  return n == 3 ? write_impl(self, args, false) : not_implemented();
 }
-PyObject* py_indexed_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  return n == 4 ? write_impl("sihc::indexed_write", args, true) : not_implemented();
+PyObject* py_indexed_write(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+  return n == 4 ? write_impl(self, args, true) : not_implemented();
 }
-PyObject* py_triangular(PyObject*, PyObject* const* args, Py_ssize_t n) {
+PyObject* py_triangular(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   if (n != 3) return not_implemented();
-  return guarded("sihc::sublayer_triangular", [&]() -> PyObject* {
+  return guarded(self, [&]() -> PyObject* {
     Tensor base, gamma;
     std::vector<Tensor> updates;
     if (!unwrap(args[0], base) || !unwrap_list(args[1], updates) || !unwrap(args[2], gamma)) return not_implemented();
@@ -629,9 +647,9 @@ PyObject* py_triangular(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }));
   });
 }
-PyObject* py_event(PyObject*, PyObject* const* args, Py_ssize_t n) {
+PyObject* py_event(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   if (n != 4) return not_implemented();
-  return guarded("sihc::event_write_read", [&]() -> PyObject* {
+  return guarded(self, [&]() -> PyObject* {
     Tensor x, dz, beta, alpha;
     if (!unwrap(args[0], x) || !unwrap(args[1], dz) || !unwrap(args[2], beta) || !unwrap(args[3], alpha))
       return not_implemented();
@@ -644,41 +662,39 @@ PyObject* py_event(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
-// (op name without its suffix, carrier edge, blocks, slots, x0, dz_0.., beta_0..)
-PyObject* py_block_write(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n < 5) return not_implemented();
-  const char* name = PyUnicode_AsUTF8(args[0]);
-  if (!name) return nullptr;
-  const long edge = PyLong_AsLong(args[1]), blocks = PyLong_AsLong(args[2]), slots = PyLong_AsLong(args[3]);
-  if (n != 5 + 2 * blocks) return not_implemented();
-  return guarded("sihc::final_accumulate", [&]() -> PyObject* {
+// (carrier edge, blocks, slots, x0, dz_0.., beta_0..)
+PyObject* py_block_write(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+  if (n < 4) return not_implemented();
+  const long edge = PyLong_AsLong(args[0]), blocks = PyLong_AsLong(args[1]), slots = PyLong_AsLong(args[2]);
+  if (n != 4 + 2 * blocks) return not_implemented();
+  return guarded(self, [&]() -> PyObject* {
     Tensor x;
     std::vector<Tensor> updates(static_cast<size_t>(blocks)), betas(static_cast<size_t>(blocks));
-    if (!unwrap(args[4], x)) return not_implemented();
+    if (!unwrap(args[3], x)) return not_implemented();
     for (long i = 0; i < blocks; ++i)
-      if (!unwrap(args[5 + i], updates[size_t(i)]) || !unwrap(args[5 + blocks + i], betas[size_t(i)]))
+      if (!unwrap(args[4 + i], updates[size_t(i)]) || !unwrap(args[4 + blocks + i], betas[size_t(i)]))
         return not_implemented();
     if (!BlockWriteFn::fits(x, updates, betas) || x.size(1) != edge || betas[0].size(1) != slots)
       return not_implemented();
     return THPVariable_Wrap(without_gil([&] {
       return unrecorded() ? run_write(x, updates, at::stack(betas), Tensor())
-                          : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas), std::string(name));
+                          : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas), std::string(entry_of(self).name()));
     }));
   });
 }
-PyObject* py_gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
+PyObject* py_gather(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   if (n != 3 || !PyLong_CheckExact(args[2])) return not_implemented();
   const long slots = PyLong_AsLong(args[2]);
-  return guarded("sihc::gather_cells", [&]() -> PyObject* {
+  return guarded(self, [&]() -> PyObject* {
     Tensor x, index;
     if (!unwrap(args[0], x) || !unwrap(args[1], index) || !gather_fits(x, index, slots)) return not_implemented();
     return THPVariable_Wrap(without_gil(
         [&] { return unrecorded() ? run_gather(x, index, slots) : GatherFn::apply(x, index, int64_t(slots)); }));
   });
 }
-PyObject* py_scatter(PyObject*, PyObject* const* args, Py_ssize_t n) {
+PyObject* py_scatter(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   if (n != 2) return not_implemented();
-  return guarded("sihc::scatter_cells", [&]() -> PyObject* {
+  return guarded(self, [&]() -> PyObject* {
     Tensor cells, index;
     if (!unwrap(args[0], cells) || !unwrap(args[1], index) || !scatter_fits(cells, index)) return not_implemented();
     return THPVariable_Wrap(without_gil([&] {
@@ -688,17 +704,35 @@ PyObject* py_scatter(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
-PyMethodDef entry(const char* name) {
+PyMethodDef define(const char* name) {
   return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(F)), METH_FASTCALL, nullptr};
 }
-PyMethodDef methods[] = {
-    entry<py_read>("sublayer_read"),        entry<py_write>("sublayer_write"),
-    entry<py_triangular>("sublayer_triangular"), entry<py_event>("event_write_read"),
-    entry<py_indexed_read>("indexed_read"), entry<py_indexed_write>("indexed_write"),
-    entry<py_block_write>("block_write"),   entry<py_gather>("gather_cells"),
-    entry<py_scatter>("scatter_cells"),
-    {nullptr, nullptr, 0, nullptr},
+PyMethodDef entries[] = {
+    define<py_read>("sublayer_read"),        define<py_write>("sublayer_write"),
+    define<py_triangular>("sublayer_triangular"), define<py_event>("event_write_read"),
+    define<py_indexed_read>("indexed_read"), define<py_indexed_write>("indexed_write"),
+    define<py_block_write>("block_write"),   define<py_gather>("gather_cells"),
+    define<py_scatter>("scatter_cells"),
 };
+// entry(name, op): the native entry `name` for the registered op `op` ("namespace::name")
+PyObject* py_entry(PyObject*, PyObject* args) {
+  const char *name, *op;
+  if (!PyArg_ParseTuple(args, "ss", &name, &op)) return nullptr;
+  for (PyMethodDef& def : entries) {
+    if (std::strcmp(def.ml_name, name) != 0) continue;
+    const auto handle = c10::Dispatcher::singleton().findSchema({op, ""});
+    if (!handle) return PyErr_Format(PyExc_ValueError, "no registered op %s", op);
+    PyObject* self = PyCapsule_New(new Entry{*handle}, ENTRY, [](PyObject* capsule) {
+      delete static_cast<Entry*>(PyCapsule_GetPointer(capsule, ENTRY));
+    });
+    if (!self) return nullptr;
+    PyObject* function = PyCFunction_New(&def, self);
+    Py_DECREF(self);
+    return function;
+  }
+  return PyErr_Format(PyExc_AttributeError, "no native entry %s", name);
+}
+PyMethodDef methods[] = {{"entry", py_entry, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_sihc_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

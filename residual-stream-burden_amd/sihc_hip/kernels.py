@@ -227,7 +227,7 @@ def _make_final_accumulate(tag: str):
         return (grad_out, *gdz.unbind(0), *(g.to(b.dtype) for g, b in zip(gbeta.unbind(0), betas)))
 
     register_autograd(fa, backward, setup_context=setup)
-    native(fa, "block_write", lambda entry: lambda *args: entry(f"sihc::{name}", edge, blocks, slots, *args))
+    native(fa, "block_write", lambda entry: lambda *args: entry(edge, blocks, slots, *args))
     return fa, grad_dz, grad_beta
 
 

@@ -19,6 +19,7 @@ from torch.utils._python_dispatch import TorchDispatchMode
 from sihc_hip import indexed as ix
 from sihc_hip import kernels as legacy
 from sihc_hip import sublayer_kernels as sk
+from sihc_hip._native import native
 from sihc_hip.event_ops import event_write_read
 
 pytestmark = pytest.mark.gpu
@@ -247,6 +248,54 @@ def test_an_error_of_a_saved_tensor_hook_reaches_the_caller_once(name):
     again = torch.utils.checkpoint.checkpoint(region, use_reentrant=False)
     assert _is_native(again[0])
     assert all(torch.equal(a, b) for a, b in zip(_grads(again, args), _grads(region(), args)))
+
+
+def _read_op(name):
+    """An op like sublayer_read with a native entry, for one test's registrations."""
+    @torch.library.custom_op(f"sihc_test::{name}", mutates_args=())
+    def read(x: torch.Tensor, alpha: torch.Tensor) -> list[torch.Tensor]:
+        return sk.sublayer_read(x, alpha)
+
+    torch.library.register_autograd(read, sk._read_backward, setup_context=sk._read_setup)
+    return native(read, "sublayer_read")
+
+
+def test_what_a_program_registers_for_an_op_is_honoured():
+    _, (x, w), _ = _calls(torch.float32)["read"]
+    want = sk.sublayer_read(x, w)
+
+    def again(op, register, expected):
+        assert _is_native(op(x, w)[0])
+        register(op)
+        got = op(x, w)
+        assert not _is_native(got[0])
+        assert torch.equal(got[0], expected)
+
+    def kernel(x, alpha):
+        return [2 * t for t in sk.sublayer_read(x, alpha)]
+
+    again(_read_op("kernel"), lambda op: op.register_kernel(None, kernel), 2 * want[0])
+    again(_read_op("cuda_kernel"), lambda op: op.register_kernel("cuda", kernel), 2 * want[0])
+    lib = torch.library.Library("sihc_test", "FRAGMENT")
+    again(_read_op("dispatcher_kernel"), lambda op: lib.impl("dispatcher_kernel", kernel, "CUDA"), 2 * want[0])
+    again(_read_op("by_name"), lambda op: torch.library.register_kernel("sihc_test::by_name", "cuda", kernel),
+          2 * want[0])
+
+    def backward(ctx, grads):
+        return torch.full_like(x, 3.0), None
+
+    op = _read_op("rule")
+    again(op, lambda op: torch.library.register_autograd("sihc_test::rule", backward), want[0])
+    assert (torch.autograd.grad(op(x, w)[0].sum(), x)[0] == 3.0).all()
+
+    op = _read_op("autocast")
+    again(op, lambda op: torch.library.register_autocast("sihc_test::autocast", "cuda", torch.bfloat16), want[0])
+    with torch.autocast("cuda", torch.bfloat16):
+        assert op(x, w)[0].dtype == torch.bfloat16
+
+    op = _read_op("host_kernel")
+    op.register_kernel("cpu", kernel)
+    assert _is_native(op(x, w)[0])
 
 
 @pytest.mark.parametrize("name", NAMES)
