@@ -1135,11 +1135,13 @@ __global__ void __launch_bounds__(256) k_read_w(const bf16_t* __restrict__ x, co
 
 // ----------------------------------------------------------------------------------
 // Block reduction helper: sums W = (blockDim.x * NV) floats per thread over threadIdx.y
-// and hands each (lane-major) sum to `emit(i, value)`. red must hold TL * W floats. More than 8
-// rows are summed as rows of 8: one chain over the 64 rows of a 4-lane slice left an fp32 weight
-// gradient of 256 tokens x 130 channels 1.6e-7 from the exact sum, 8-row blocks 0.9e-7.
+// and hands each (lane-major) sum to `emit(i, value)`. red must hold TL * W floats. ROWS8: more
+// than 8 rows (a power of two) are summed as rows of 8, 8 loads at a time: one chain over the 64
+// rows of a 4-lane slice left an fp32 weight gradient of 256 tokens x 130 channels 1.6e-7 from
+// the exact sum, 8-row blocks 0.9e-7. A kernel of up to 8 rows is compiled without it: beside the
+// plain loop it cost the wide launches 2% (event backward, 16,384 tokens x 1152 bf16: 109.6 us with both, 107.8 without).
 // ----------------------------------------------------------------------------------
-template <int NV, typename Emit>
+template <int NV, bool ROWS8, typename Emit>
 __device__ __forceinline__ void block_reduce_rows(const float* acc, float* red, Emit&& emit) {
   const int W = blockDim.x * NV;
   const int TL = blockDim.y;
@@ -1150,14 +1152,15 @@ __device__ __forceinline__ void block_reduce_rows(const float* acc, float* red, 
   __syncthreads();
   for (int i = tid; i < W; i += nthr) {
     float sum = 0.f;
-    if (TL <= 8) {
-      for (int ty = 0; ty < TL; ++ty) sum += red[ty * W + i];
-    } else {
+    if (ROWS8 && TL > 8) {
       for (int t0 = 0; t0 < TL; t0 += 8) {
         float eight = 0.f;
-        for (int ty = t0; ty < min(t0 + 8, TL); ++ty) eight += red[ty * W + i];
+#pragma unroll
+        for (int ty = 0; ty < 8; ++ty) eight += red[(t0 + ty) * W + i];
         sum += eight;
       }
+    } else {
+      for (int ty = 0; ty < TL; ++ty) sum += red[ty * W + i];
     }
     emit(i, sum);
   }
@@ -2802,7 +2805,8 @@ __global__ void __launch_bounds__(1024) k_event_fwd_rows(const T* __restrict__ x
 //   HAS_W: write part (dz, beta)  STORE_T: store t as grad_x (else the caller aliases)
 // part[chunk][0][s][c] = partial grad_beta, part[chunk][1][s][c] = partial grad_alpha_next
 // ----------------------------------------------------------------------------------
-template <typename T, int V, int K, bool HAS_H, bool HAS_G, bool HAS_W, bool STORE_T, bool NTL, bool NTS>
+//   RAG: rows that V does not divide       NARROW: more than 8 lane rows per block
+template <typename T, int V, int K, bool HAS_H, bool HAS_G, bool HAS_W, bool STORE_T, bool RAG, bool NARROW>
 __global__ void __launch_bounds__(256, SIHC_EV_MINW) k_event_bwd(const T* __restrict__ gxo, const T* __restrict__ gzo,
                                                    const T* __restrict__ xo, const T* __restrict__ dz,
                                                    const T* __restrict__ beta,
@@ -2812,12 +2816,12 @@ __global__ void __launch_bounds__(256, SIHC_EV_MINW) k_event_bwd(const T* __rest
                                                    int nslices, EvCarry carry) {
   constexpr int S = K * K;
   constexpr int U = SIHC_EV_UNROLL;  // tokens per lane per iteration
+  constexpr bool NTL = !RAG && (SIHC_EV_BWD_NT & 1) != 0, NTS = !RAG && (SIHC_EV_BWD_NT & 2) != 0;
   extern __shared__ float red[];  // TL x BCG x S x V floats (>= FINALIZE_LDS(4): 256 x 4)
   if (run_carry<T>(carry, S, g.C, red)) return;
   const int BCG = blockDim.x, TL = blockDim.y;
   const int BC = BCG * V;
   int slice, chunk;
-  constexpr bool RAG = !NTL;  // rows that V does not divide are launched without hints
   slice_chunk_row(carry.nmain, nslices, (K == 4 && BC * int(sizeof(T)) < 128) || RAG, slice, chunk);
   const int cb = slice * BC + threadIdx.x * V, c0 = RAG ? lane_channel(cb, V, g.C) : cb;
   float db[S][V], da[S][V];
@@ -2951,7 +2955,7 @@ __global__ void __launch_bounds__(256, SIHC_EV_MINW) k_event_bwd(const T* __rest
 #pragma unroll
       for (int v = 0; v < V; ++v) flat[s * V + v] = w == 0 ? db[s][v] : da[s][v];
     // lane-major layout in `red`: [ty][lane][s][v]; remap to [s][c] on emit.
-    block_reduce_rows<S * V>(flat, red, [&](int i, float sum) {
+    block_reduce_rows<S * V, NARROW>(flat, red, [&](int i, float sum) {
       const int lane = i / (S * V);
       const int r = i - lane * S * V;
       const int s = r / V;
@@ -2972,7 +2976,7 @@ __global__ void __launch_bounds__(256, SIHC_EV_MINW) k_event_bwd(const T* __rest
 // word p = slots 2p, 2p + 1) with four 16-byte loads. The token order per thread equals
 // k_event_bwd's (tokens ty, ty + TL, ... of each group), so the partial rows are the same.
 // ----------------------------------------------------------------------------------
-template <bool HAS_H, bool HAS_G, bool HAS_W, bool STORE_T, bool NTL, bool NTS>
+template <bool HAS_H, bool HAS_G, bool HAS_W, bool STORE_T, bool RAG, bool NARROW>
 __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_t* __restrict__ gxo,
                                                      const bf16_t* __restrict__ gzo,
                                                      const bf16_t* __restrict__ xo, const bf16_t* __restrict__ dz,
@@ -2982,13 +2986,14 @@ __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_
                                                      const int32_t* __restrict__ index, Geo g, int gs, int nchunks,
                                                      int nslices, EvCarry carry) {
   constexpr int K = 4, S = 16, V = 2;
+  constexpr bool NTL = !RAG && (SIHC_EV_BWD_NT & 1) != 0, NTS = !RAG && (SIHC_EV_BWD_NT & 2) != 0;
   extern __shared__ float red[];  // TL x BCG x S x V floats (>= FINALIZE_LDS(4))
   if (run_carry<bf16_t>(carry, S, g.C, red)) return;
   const int BCG = blockDim.x, TL = blockDim.y;
   const int BC = BCG * V;
   int slice, chunk;
-  slice_chunk_row(carry.nmain, nslices, BC * 2 < 128 || (g.C & 1) != 0, slice, chunk);
-  const int cb = slice * BC + threadIdx.x * V, c0 = lane_channel(cb, V, g.C);
+  slice_chunk_row(carry.nmain, nslices, BC * 2 < 128 || RAG, slice, chunk);
+  const int cb = slice * BC + threadIdx.x * V, c0 = RAG ? lane_channel(cb, V, g.C) : cb;
   float db[S][V], da[S][V];
 #pragma unroll
   for (int sl = 0; sl < S; ++sl)
@@ -3089,13 +3094,13 @@ __global__ void __launch_bounds__(256, SIHC_EV16_MINW) k_event_bwd16(const bf16_
     for (int sl = 0; sl < S; ++sl)
 #pragma unroll
       for (int v = 0; v < V; ++v) flat[sl * V + v] = w == 0 ? db[sl][v] : da[sl][v];
-    block_reduce_rows<S * V>(flat, red, [&](int i, float sum) {
+    block_reduce_rows<S * V, NARROW>(flat, red, [&](int i, float sum) {
       const int lane = i / (S * V);
       const int r = i - lane * S * V;
       const int sl = r / V;
       const int v = r - sl * V;
       const int cbl = cs + lane * V;
-      if (cbl < g.C) prow[(int64_t(w) * S + sl) * g.C + lane_channel(cbl, V, g.C) + v] = sum;
+      if (cbl < g.C) prow[(int64_t(w) * S + sl) * g.C + (RAG ? lane_channel(cbl, V, g.C) : cbl) + v] = sum;
     });
   }
 }
@@ -4714,15 +4719,17 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
             auto go = [&](auto hg, auto hw, auto stt) {
               constexpr bool HG = decltype(hg)::value, HW = decltype(hw)::value, STT = decltype(stt)::value;
               return with_bool(channels % VV != 0, [&](auto rg) {
-              constexpr bool RAG = decltype(rg)::value;
-              constexpr bool NTL = !RAG && (SIHC_EV_BWD_NT & 1) != 0, NTS = !RAG && (SIHC_EV_BWD_NT & 2) != 0;
+              return with_bool(sh.tl > 8, [&](auto nr) {
+              // blocks of up to 8 lane rows: 32 and more lanes of the widest bf16 and 16-slot vectors
+              constexpr bool WIDE = KK == 4 ? VV == 2 : VV == 4 && std::is_same_v<T, bf16_t>;
+              constexpr bool RAG = decltype(rg)::value, NR = RAG || !WIDE || decltype(nr)::value;
               // 16-slot bf16 cells with 2-channel lanes: the register-lean kernel
               constexpr bool B16 = SIHC_EV_BWD16 && KK == 4 && VV == 2 && std::is_same_v<T, bf16_t>;
               const void* kfn;
               if constexpr (B16) {
-                kfn = reinterpret_cast<const void*>(&k_event_bwd16<HH, HG, HW, STT, NTL, NTS>);
+                kfn = reinterpret_cast<const void*>(&k_event_bwd16<HH, HG, HW, STT, RAG, NR>);
               } else {
-                kfn = reinterpret_cast<const void*>(&k_event_bwd<T, VV, KK, HH, HG, HW, STT, NTL, NTS>);
+                kfn = reinterpret_cast<const void*>(&k_event_bwd<T, VV, KK, HH, HG, HW, STT, RAG, NR>);
               }
               chunks = whole_rounds(sh.slices, max_chunks, resident_blocks(kfn, sh.bcg * sh.tl, lds));
               // token groups: a multiple of one loop iteration (SIHC_EV_UNROLL x TL tokens);
@@ -4734,7 +4741,7 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
               cy.nmain = int(blocks1d(sh.slices, chunks));
               const dim3 grid_blocks(blocks1d(sh.slices, chunks) + carry_blocks);
               if constexpr (B16) {
-                hipLaunchKernelGGL((k_event_bwd16<HH, HG, HW, STT, NTL, NTS>), grid_blocks, dim3(sh.bcg, sh.tl), lds,
+                hipLaunchKernelGGL((k_event_bwd16<HH, HG, HW, STT, RAG, NR>), grid_blocks, dim3(sh.bcg, sh.tl), lds,
                                    st, static_cast<const T*>(grad_x_out), static_cast<const T*>(grad_z_out),
                                    static_cast<const T*>(x_out), static_cast<const T*>(dz),
                                    static_cast<const T*>(beta), static_cast<const T*>(alpha_next),
@@ -4742,13 +4749,14 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
                                    sh.slices, cy);
                 return check_launch(what);
               }
-              hipLaunchKernelGGL((k_event_bwd<T, VV, KK, HH, HG, HW, STT, NTL, NTS>), grid_blocks, dim3(sh.bcg, sh.tl),
+              hipLaunchKernelGGL((k_event_bwd<T, VV, KK, HH, HG, HW, STT, RAG, NR>), grid_blocks, dim3(sh.bcg, sh.tl),
                                  lds, st, static_cast<const T*>(grad_x_out), static_cast<const T*>(grad_z_out),
                                  static_cast<const T*>(x_out), static_cast<const T*>(dz),
                                  static_cast<const T*>(beta), static_cast<const T*>(alpha_next),
                                  static_cast<T*>(grad_x), static_cast<T*>(grad_dz), part, index, g, gs, chunks,
                                  sh.slices, cy);
               return check_launch(what);
+              });
               });
             };
             switch (mode) {
