@@ -2760,14 +2760,15 @@ __global__ void __launch_bounds__(SIHC_EV_FWD_THREADS, SIHC_EV_MINW) k_event_fwd
 // the dz / z_out rows. k_event_fwd's arithmetic per element (same bits); one-shot, no
 // loop: token blockIdx.x * TR + threadIdx.y.
 // ----------------------------------------------------------------------------------
-template <typename T, int V, bool HAS_Z, bool NTL, bool NTS>
+template <typename T, int V, bool HAS_Z, bool RAG>
 __global__ void __launch_bounds__(1024) k_event_fwd_rows(const T* __restrict__ x, const T* __restrict__ dz,
                                                          const T* __restrict__ beta, const T* __restrict__ alpha,
                                                          T* __restrict__ xo, T* __restrict__ zo,
                                                          const int32_t* __restrict__ index, Geo g) {
   constexpr int K = 2, S = 4;
+  constexpr bool NTL = (SIHC_EV_FWD_NT & 1) != 0, NTS = (SIHC_EV_FWD_NT & 2) != 0;
   const int m = int(blockIdx.x) * int(blockDim.y) + int(threadIdx.y);
-  const int c0 = lane_channel(int(threadIdx.x) * V, V, g.C);
+  const int c0 = RAG ? lane_channel(int(threadIdx.x) * V, V, g.C) : int(threadIdx.x) * V;
   if (m >= g.M) return;
   float bw[S][V], aw[S][V];
   load_weights<T, V, K>(beta, c0, bw);
@@ -4587,11 +4588,13 @@ int sihc_event_forward(const void* x, const void* dz, const void* beta, const vo
               if (channels >= VR && lanes <= 1024 && (!in_place || channels % VR == 0)) {
                 const int tr = std::max(1, SIHC_EV_ROW_THREADS / lanes);
                 const int64_t blocks = (int64_t(g.M) + tr - 1) / tr;
-                hipLaunchKernelGGL((k_event_fwd_rows<T, VR, HZ, true, true>), dim3(unsigned(blocks)), dim3(lanes, tr), 0,
-                                   st, static_cast<const T*>(x), static_cast<const T*>(dz),
-                                   static_cast<const T*>(beta), static_cast<const T*>(alpha_next),
-                                   static_cast<T*>(x_out), static_cast<T*>(z_out), index, g);
-                return check_launch(what);
+                return with_bool(channels % VR != 0, [&](auto rr) {
+                  hipLaunchKernelGGL((k_event_fwd_rows<T, VR, HZ, decltype(rr)::value>), dim3(unsigned(blocks)),
+                                     dim3(lanes, tr), 0, st, static_cast<const T*>(x), static_cast<const T*>(dz),
+                                     static_cast<const T*>(beta), static_cast<const T*>(alpha_next),
+                                     static_cast<T*>(x_out), static_cast<T*>(z_out), index, g);
+                  return check_launch(what);
+                });
               }
             }
             if constexpr (SIHC_EV_FWD16 && KK == 4 && VV == 2 && std::is_same_v<T, bf16_t>) {
