@@ -257,6 +257,13 @@ auto registered(const char* name) {
 // A backward may launch directly: nothing recorded or in force (its operands are asked apart).
 bool direct() { return !at::GradMode::is_enabled() && plain_mode(); }
 
+// What a profiler sees of a call: the op's name and its arguments (made only if one looks).
+using Args = std::vector<c10::IValue>;
+Args listed(const Tensor& x, TensorList ts, const Tensor& w, const Tensor& index) {
+  Args args{x, ts.vec(), w};
+  if (index.defined()) args.emplace_back(index);
+  return args;
+}
 // ------------------------------------------------------------------------ autograd nodes
 struct ReadFn : torch::autograd::Function<ReadFn> {
   static constexpr bool is_traceable = true;
@@ -273,6 +280,8 @@ struct ReadFn : torch::autograd::Function<ReadFn> {
     std::tuple<Tensor, Tensor> r;
     Shape s{};
     if (direct() && write_fits(x, grads, alpha, index, s)) {
+      RECORD_FUNCTION(index.defined() ? "sihc::indexed_read_backward" : "sihc::sublayer_read_backward",
+                      listed(x, grads, alpha, index));
       r = run_read_backward(x, grads, alpha, index);
     } else if (index.defined()) {
       static auto op = registered<std::tuple<Tensor, Tensor>(const Tensor&, TensorList, const Tensor&,
@@ -306,6 +315,8 @@ struct WriteFn : torch::autograd::Function<WriteFn> {
     Tensor db;
     Shape s{};
     if (direct() && write_fits(grad, updates, beta, index, s)) {
+      RECORD_FUNCTION(index.defined() ? "sihc::indexed_write_backward" : "sihc::sublayer_write_backward",
+                      listed(grad, updates, beta, index));
       std::tie(dz, db) = run_write_backward(grad, updates, beta, index);
     } else if (index.defined()) {
       static auto read =
@@ -354,7 +365,8 @@ struct TriangularFn : torch::autograd::Function<TriangularFn> {
     const Tensor grad = grads[0].contiguous();
     variable_list out{grad};
     if (direct() && triangular_fits(grad, updates, gamma)) {
-      const c10::DeviceGuard guard(grad.device());
+      RECORD_FUNCTION("sihc::sublayer_triangular_backward", listed(grad, updates, gamma, Tensor()));
+      const c10::DeviceGuard device(grad.device());
       const int64_t c = grad.size(-1), rows = grad.numel() / c;
       const int active = int(updates.size());
       // one allocation, as the Python op's stacked result
@@ -415,7 +427,8 @@ struct EventFn : torch::autograd::Function<EventFn> {
       const auto [a, b, c, d] = op.call(gx, gz, xo, dz, beta, alpha);
       return {a, b, c, d};
     }
-    const c10::DeviceGuard guard(xo.device());
+    RECORD_FUNCTION("sihc::event_write_read_backward", (Args{gx, gz, xo, dz, beta, alpha}));
+    const c10::DeviceGuard device(xo.device());
     const Shape s = shape_of(xo, beta);
     Tensor dx = at::empty_like(xo), ddz = at::empty_like(dz), db = at::empty_like(beta), da = at::empty_like(alpha);
     const Tensor ws = workspace(
@@ -464,7 +477,9 @@ struct BlockWriteFn : torch::autograd::Function<BlockWriteFn> {
     const variable_list updates(saved.begin(), saved.begin() + long(n)), betas(saved.begin() + long(n), saved.end());
     const Tensor grad = grads[0].contiguous();
     if (direct() && fits(grad, updates, betas)) {
-      const auto [dz, db] = run_write_backward(grad, updates, at::stack(betas), Tensor());
+      const Tensor beta = at::stack(betas);
+      RECORD_FUNCTION("sihc::sublayer_write_backward", listed(grad, updates, beta, Tensor()));
+      const auto [dz, db] = run_write_backward(grad, updates, beta, Tensor());
       variable_list out{grad};
       out.insert(out.end(), dz.begin(), dz.end());
       for (const Tensor& t : db.unbind(0)) out.push_back(t);
@@ -517,7 +532,10 @@ struct GatherFn : torch::autograd::Function<GatherFn> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const Tensor index = ctx->get_saved_variables()[0], grad = grads[0].contiguous();
-    if (direct() && scatter_fits(grad, index)) return {run_scatter(sihc_scatter_add_cells, grad, index, false), Tensor(), Tensor()};
+    if (direct() && scatter_fits(grad, index)) {
+      RECORD_FUNCTION("sihc::scatter_add_cells", (Args{grad, index}));
+      return {run_scatter(sihc_scatter_add_cells, grad, index, false), Tensor(), Tensor()};
+    }
     static auto op = registered<Tensor(const Tensor&, const Tensor&)>("sihc::scatter_add_cells");
     return {op.call(grad, index), Tensor(), Tensor()};
   }
@@ -532,7 +550,10 @@ struct ScatterFn : torch::autograd::Function<ScatterFn> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const Tensor index = ctx->get_saved_variables()[0], grad = grads[0].contiguous();
     const int64_t slots = ctx->saved_data["slots"].toInt();
-    if (direct() && gather_fits(grad, index, slots)) return {run_gather(grad, index, slots), Tensor()};
+    if (direct() && gather_fits(grad, index, slots)) {
+      RECORD_FUNCTION("sihc::gather_cells", (Args{grad, index, slots}));
+      return {run_gather(grad, index, slots), Tensor()};
+    }
     static auto op = registered<Tensor(const Tensor&, const Tensor&, int64_t)>("sihc::gather_cells");
     return {op.call(grad, index, slots), Tensor()};
   }
@@ -569,7 +590,6 @@ PyObject* guarded(PyObject* self, F&& f) {
   try {
     const Entry& entry = entry_of(self);
     if (!plain_mode() || entry.overridden()) return not_implemented();
-    RECORD_FUNCTION(entry.name(), std::vector<c10::IValue>());
     return f();
   } catch (const Failure&) {
     return not_implemented();
@@ -581,11 +601,12 @@ PyObject* guarded(PyObject* self, F&& f) {
     return not_implemented();
   }
 }
-// f() with the GIL released: a launch waits where the queue is full, and an allocation may wait for
+// f() as a call of the op of `self`, with the GIL released: a launch waits where the queue is full, and an allocation may wait for
 // the device. (The registered ops release it around every dispatch and launch.) Saved-tensor hooks
 // take it again for their own calls.
-template <typename F>
-auto without_gil(F&& f) {
+template <typename A, typename F>
+auto call(PyObject* self, A&& args, F&& f) {
+  RECORD_FUNCTION(entry_of(self).name(), args());
   struct Released {
     PyThreadState* state = PyEval_SaveThread();
     ~Released() { PyEval_RestoreThread(state); }
@@ -602,7 +623,8 @@ PyObject* read_impl(PyObject* self, PyObject* const* args, bool indexed) {
     Shape s{};
     if (!unwrap(args[0], x) || !unwrap(args[1], alpha) || (indexed && !unwrap(args[2], index))) return not_implemented();
     if ((indexed && !index.defined()) || !read_fits(x, alpha, index, s)) return not_implemented();
-    return to_list(without_gil(
+    return to_list(call(
+        self, [&] { return index.defined() ? Args{x, alpha, index} : Args{x, alpha}; },
         [&] { return unrecorded() ? run_read(x, alpha, index) : ReadFn::apply(x, alpha, maybe(index)); }));
   });
 }
@@ -615,7 +637,7 @@ PyObject* write_impl(PyObject* self, PyObject* const* args, bool indexed) {
         (indexed && !unwrap(args[3], index)))
       return not_implemented();
     if ((indexed && !index.defined()) || !write_fits(x, updates, beta, index, s)) return not_implemented();
-    return THPVariable_Wrap(without_gil([&] {
+    return THPVariable_Wrap(call(self, [&] { return listed(x, updates, beta, index); }, [&] {
       return unrecorded() ? run_write(x, updates, beta, index)
                           : WriteFn::apply(x, TensorList(updates), beta, maybe(index));
     }));
@@ -641,7 +663,7 @@ PyObject* py_triangular(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     std::vector<Tensor> updates;
     if (!unwrap(args[0], base) || !unwrap_list(args[1], updates) || !unwrap(args[2], gamma)) return not_implemented();
     if (!triangular_fits(base, updates, gamma)) return not_implemented();
-    return THPVariable_Wrap(without_gil([&] {
+    return THPVariable_Wrap(call(self, [&] { return listed(base, updates, gamma, Tensor()); }, [&] {
       return unrecorded() ? run_triangular(base, updates, gamma)
                           : TriangularFn::apply(base, TensorList(updates), gamma);
     }));
@@ -654,7 +676,8 @@ PyObject* py_event(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     if (!unwrap(args[0], x) || !unwrap(args[1], dz) || !unwrap(args[2], beta) || !unwrap(args[3], alpha))
       return not_implemented();
     if (!event_fits(x, dz, beta, alpha)) return not_implemented();
-    const variable_list out = without_gil(
+    const variable_list out = call(
+        self, [&] { return Args{x, dz, beta, alpha}; },
         [&] { return unrecorded() ? run_event(x, dz, beta, alpha) : EventFn::apply(x, dz, beta, alpha); });
     PyObject* pair = PyTuple_New(2);
     for (int i = 0; pair && i < 2; ++i) PyTuple_SET_ITEM(pair, i, THPVariable_Wrap(out[size_t(i)]));
@@ -676,7 +699,13 @@ PyObject* py_block_write(PyObject* self, PyObject* const* args, Py_ssize_t n) {
         return not_implemented();
     if (!BlockWriteFn::fits(x, updates, betas) || x.size(1) != edge || betas[0].size(1) != slots)
       return not_implemented();
-    return THPVariable_Wrap(without_gil([&] {
+    auto listing = [&] {
+      Args all{x};
+      for (const auto* ts : {&updates, &betas})
+        for (const Tensor& t : *ts) all.emplace_back(t);
+      return all;
+    };
+    return THPVariable_Wrap(call(self, listing, [&] {
       return unrecorded() ? run_write(x, updates, at::stack(betas), Tensor())
                           : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas), std::string(entry_of(self).name()));
     }));
@@ -688,7 +717,8 @@ PyObject* py_gather(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   return guarded(self, [&]() -> PyObject* {
     Tensor x, index;
     if (!unwrap(args[0], x) || !unwrap(args[1], index) || !gather_fits(x, index, slots)) return not_implemented();
-    return THPVariable_Wrap(without_gil(
+    return THPVariable_Wrap(call(
+        self, [&] { return Args{x, index, int64_t(slots)}; },
         [&] { return unrecorded() ? run_gather(x, index, slots) : GatherFn::apply(x, index, int64_t(slots)); }));
   });
 }
@@ -697,7 +727,7 @@ PyObject* py_scatter(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   return guarded(self, [&]() -> PyObject* {
     Tensor cells, index;
     if (!unwrap(args[0], cells) || !unwrap(args[1], index) || !scatter_fits(cells, index)) return not_implemented();
-    return THPVariable_Wrap(without_gil([&] {
+    return THPVariable_Wrap(call(self, [&] { return Args{cells, index}; }, [&] {
       return unrecorded() ? run_scatter(sihc_scatter_cells, cells, index, true) : ScatterFn::apply(cells, index);
     }));
   });

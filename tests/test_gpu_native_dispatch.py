@@ -250,6 +250,19 @@ def test_an_error_of_a_saved_tensor_hook_reaches_the_caller_once(name):
     assert all(torch.equal(a, b) for a, b in zip(_grads(again, args), _grads(region(), args)))
 
 
+@pytest.mark.parametrize("name", NAMES)
+def test_profiles_show_the_ops_with_their_shapes(name):
+    op, args, registered = _calls(torch.float32)[name]
+    seen = []
+    for f in (op, registered):
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=True) as prof:
+            _grads(_outs(f(*args)), args)
+        ours = {e.name: e.input_shapes for e in prof.events() if e.name.startswith("sihc::")}
+        forward = registered._qualified_op_name
+        seen.append((ours[forward], sorted(n for n in ours if "backward" in n or "_add_" in n)))
+    assert seen[0] == seen[1] and seen[0][0]
+
+
 def _read_op(name):
     """An op like sublayer_read with a native entry, for one test's registrations."""
     @torch.library.custom_op(f"sihc_test::{name}", mutates_args=())
