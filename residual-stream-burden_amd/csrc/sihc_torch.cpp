@@ -768,6 +768,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_sihc_torch", nullptr, -1, methods
 }  // namespace
 
 PyMODINIT_FUNC PyInit__sihc_torch(void) {
+  if (sihc_abi_version() != SIHC_ABI_VERSION)
+    return PyErr_Format(PyExc_ImportError, "libsihc_hip.so has ABI %d, expected %d: rebuild it", sihc_abi_version(),
+                        SIHC_ABI_VERSION);
   PyObject* nn = PyImport_ImportModule("torch.nn");
   if (!nn) return nullptr;
   parameter_type = PyObject_GetAttrString(nn, "Parameter");

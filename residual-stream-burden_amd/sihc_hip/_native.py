@@ -19,6 +19,8 @@ from typing import Callable, Optional
 from torch.compiler import is_compiling
 from torch.library import CustomOpDef
 
+from ._lib import lib
+
 NATIVE_PATH = Path(__file__).resolve().with_name("_sihc_torch.so")
 _module = None
 
@@ -30,6 +32,7 @@ def module():
         if not NATIVE_PATH.exists():
             raise RuntimeError(f"{NATIVE_PATH} is missing: build it with "
                                "`python residual-stream-burden_amd/build.py`")
+        lib()  # the library that the extension calls, its version checked
         spec = importlib.util.spec_from_file_location("_sihc_torch", NATIVE_PATH)
         loaded = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(loaded)
