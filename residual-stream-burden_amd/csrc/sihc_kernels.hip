@@ -2337,7 +2337,7 @@ __global__ void __launch_bounds__(256) k_wgrad_mm(const T* __restrict__ x, PtrPa
         m0 = nchunks * gs < g.M - m0 ? m0 + nchunks * gs : g.M;  // the last chunk's sum stays below 2^31
       }
       const bool last = m0 + mi >= g.M;
-      if constexpr (SGW * EGW * VC <= 32) {
+      if constexpr (SGW * EGW * VC <= 32) {  // fp32 holds twice the row words, but at most 28 sums here
         if (last) {
           step(tn, std::false_type{});
           break;
@@ -3844,23 +3844,35 @@ int launch_mm(const char* what, const MMArgs& a, int max_chunks, int* chunks, hi
   *chunks = n;
   return check_launch(what);
 }
-// 4-slot cells: one part with all event groups.
+// 4-slot cells: one part with all event groups; the plain gradient of 17 and more events in two
+// parts below the sizes where the carrier rows that the second part loads again cost more than
+// the sums that a wave no longer holds (bf16, E = 20, 16,384 tokens x 768: 116 us one part, 112
+// two; 65,536 x 768: 379 and 409; E = 32, 16,384 x 1152: 290 and 239; 65,536 x 1152: 821 and
+// 895). fp32 of 29-32 events always takes two: beside 128 sums a lane its rows spill (16,384 x
+// 1152: 598 us one part, 455 two).
 template <typename T, int MODE>
 int launch_mm_k2(const char* what, const MMArgs& a, int max_chunks, int* chunks, hipStream_t st) {
   if (a.events <= 4) return launch_mm<T, 2, 1, 1, MODE>(what, a, max_chunks, chunks, st);
   if (a.events <= 8) return launch_mm<T, 2, 1, 2, MODE>(what, a, max_chunks, chunks, st);
-  if constexpr (MODE == MM_WRITE) return fail(SIHC_ERR_INVALID, "%s: internal weight-gradient shape", what);
-  switch ((a.events + 3) / 4) {
-    case 3: return launch_mm<T, 2, 1, 3, MODE>(what, a, max_chunks, chunks, st);
-    case 4: return launch_mm<T, 2, 1, 4, MODE>(what, a, max_chunks, chunks, st);
-    case 5: return launch_mm<T, 2, 1, 5, MODE>(what, a, max_chunks, chunks, st);
-    case 6: return launch_mm<T, 2, 1, 6, MODE>(what, a, max_chunks, chunks, st);
-    default: break;
-  }
-  if constexpr (MODE == MM_GRAD) {
-    if (a.events <= 32)
-      return a.events <= 28 ? launch_mm<T, 2, 1, 7, MODE>(what, a, max_chunks, chunks, st)
-                            : launch_mm<T, 2, 1, 8, MODE>(what, a, max_chunks, chunks, st);
+  if constexpr (MODE != MM_WRITE) {
+    if constexpr (MODE == MM_GRAD) {
+      constexpr bool bf = sizeof(T) == 2;
+      const int64_t work = int64_t(a.g.M) * a.g.C;
+      if (a.events > 28 ? !bf || work < (48 << 20) : bf && a.events > 16 && work < ((a.events <= 18 ? 24 : 48) << 20))
+        return a.events <= 24 ? launch_mm<T, 2, 1, 3, MODE>(what, a, max_chunks, chunks, st)
+                              : launch_mm<T, 2, 1, 4, MODE>(what, a, max_chunks, chunks, st);
+      if (a.events > 24 && a.events <= 28) return launch_mm<T, 2, 1, 7, MODE>(what, a, max_chunks, chunks, st);
+      if constexpr (bf) {
+        if (a.events > 28) return launch_mm<T, 2, 1, 8, MODE>(what, a, max_chunks, chunks, st);
+      }
+    }
+    switch ((a.events + 3) / 4) {
+      case 3: return launch_mm<T, 2, 1, 3, MODE>(what, a, max_chunks, chunks, st);
+      case 4: return launch_mm<T, 2, 1, 4, MODE>(what, a, max_chunks, chunks, st);
+      case 5: return launch_mm<T, 2, 1, 5, MODE>(what, a, max_chunks, chunks, st);
+      case 6: return launch_mm<T, 2, 1, 6, MODE>(what, a, max_chunks, chunks, st);
+      default: break;
+    }
   }
   return fail(SIHC_ERR_INVALID, "%s: internal weight-gradient shape", what);
 }
@@ -3985,13 +3997,38 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
           // events per lane >= E) and covers the carrier tile (64 x waves x vectors per
           // thread >= 1024 vectors at 16 slots).
           // Carriers of at least one 16-byte vector of channels: the matrix-core kernel, except
-          // where another one measured faster (65,536 tokens x 1152 channels, bf16, and 32,768
-          // for 16 slots): one event of aligned 4-slot rows on the direct kernel (136 us, here
-          // 143), 9 and more events of aligned bf16 16-slot rows on the pipelined one (E = 12
-          // 416 us, here 447; E = 8 355, here 295).
+          // where another one measured faster. Its waves hold all events of a row, so few tokens
+          // leave it few waves, and then the kernels that split the events over waves win. The
+          // lines lie where the two sides crossed, in tokens x channels (`work`):
+          //   4 slots, one event of aligned rows: the direct kernel (65,536 x 1152 bf16 136 us,
+          //     here 143)
+          //   4 slots, 17-24 events of aligned bf16 rows below 4 Mi: the pipelined one (4,096 x
+          //     768, E = 17 37 us, here 44; 8,192 x 768 62 and 60)
+          //   4 slots, 21-32 events of fp32 below 1.25 Mi: k_wgrad (1,024 x 768, E = 24 25 us,
+          //     here 29; 2,048 x 768 46 and 44)
+          //   16 slots of aligned bf16 rows: the pipelined one, but to 4 events from 24 Mi (32,768
+          //     x 768, E = 4 223 us, here 209; 16,384 x 768 120 and 128) and for 5-8 events from 6
+          //     Mi, or 16 Mi up to 512 channels (8,192 x 768, E = 8 90 us, here 82; 4,096 x
+          //     768 44 and 51; 16,384 x 512 121 and 137; 32,768 x 1152 355 and 295)
+          //   16 slots of other rows: k_wgrad16 for fp32 of 17 and more events or bf16 of 21 and
+          //     more below 1.125 Mi (1,024 x 768 fp32, E = 24 44 us, here 54; 2,048 x 768 96 and
+          //     81) and fp32 of 13-16 events from 0.5 to 2.25 Mi (2,048 x 768 48 and 55; 256 x 768
+          //     32 and 29; 4,096 x 768 117 and 92)
           if constexpr (CAR) {
-            const bool direct = KK == 2 && events == 1 && VV * int(sizeof(T)) == 16 && g.C % VV == 0;
-            if (g.C >= 16 / int(sizeof(T)) && !direct && !(KK == 4 && bf && events > 8)) {
+            const int64_t work = int64_t(g.M) * g.C, Mi = 1 << 20;
+            constexpr bool f32 = sizeof(T) == 4;
+            bool mm = g.C >= 16 / int(sizeof(T));
+            if constexpr (KK == 2) {
+              if (events == 1) mm = mm && !(VV * int(sizeof(T)) == 16 && g.C % VV == 0);
+              if (bf && events >= 17 && events <= 24) mm = mm && work >= 4 * Mi;
+              if (f32 && events >= 21) mm = mm && work >= 5 * Mi / 4;
+            } else if (bf) {
+              mm = mm && events <= 8 && work >= (events <= 4 ? 24 : g.C > 512 ? 6 : 16) * Mi;
+            } else {
+              if (events >= (f32 ? 17 : 21)) mm = mm && work >= 9 * Mi / 8;
+              else if (f32 && events >= 13) mm = mm && (work < Mi / 2 || work >= 9 * Mi / 4);
+            }
+            if (mm) {
               const MMArgs a{x, pk, part, index, events, g, nullptr, nullptr, PtrPack{}};
               if constexpr (KK == 2) return launch_mm_k2<T, MM_GRAD>(what, a, max_chunks, &chunks, st);
               else return launch_mm_k4<T>(what, a, max_chunks, &chunks, st);
@@ -4001,7 +4038,9 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
             if (bf) {
               // 16 slots: E = 9 3 x 3 730 us (2 x 5 of 4: 907), E = 17-21 8 x 3 1095-1142 us
               // (5-6 x 4: 1320-1429), E = 28 / 32 8 x 4 1405 / 1421 us (k_wgrad16: 2290 / 2089)
-              if (events == 9) goz(IC<4>{}, IC<6>{}, IC<3>{}, 3);
+              if (events <= 4) goz(IC<4>{}, IC<4>{}, IC<1>{}, 4);  // idle waves only stage
+              else if (events <= 8) goz(IC<4>{}, IC<8>{}, IC<4>{}, 2);
+              else if (events == 9) goz(IC<4>{}, IC<6>{}, IC<3>{}, 3);
               else if (events <= 12) goz(IC<4>{}, IC<4>{}, IC<3>{}, 4);
               else if (events <= 16) goz(IC<4>{}, IC<4>{}, IC<4>{}, 4);
               else if (events <= 24) goz(IC<4>{}, IC<2>{}, IC<3>{}, 8);
@@ -4011,6 +4050,9 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
               hipLaunchKernelGGL((k_wgrad16<T>), dim3(blocks1d(slices16, chunks)), dim3(C16_LANES, nw), 0, st,
                                  static_cast<const T*>(x), pk, part, index, events, g, tpb, slices16, vs16);
             }
+          } else if (CAR && bf && events >= 17 && events <= 24) {
+            // 4 slots: 6-8 waves x 3 events
+            goz(IC<2>{}, IC<1>{}, IC<3>{}, (events + 2) / 3);
           } else if (!CAR && !SD && bf && events == 2) {
             // gamma gradient of 2 updates: the pipelined kernel on one-slot rows (1 wave x 2
             // updates: 77 us at 65,536 rows x 1152 channels; row lanes 81)
@@ -4081,10 +4123,14 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
                   });
                 }
               }
-              if (!waves)
-                hipLaunchKernelGGL((k_wgrad<T, VV, KK, CAR, SD>), dim3(blocks1d(slices, chunks)), dim3(bcg, lanes),
-                                   lds, st, static_cast<const T*>(x), pk, part, index, events, g, tpb, slices, tt, dk,
-                                   gamma, gf32);
+              if constexpr (CAR && VV * int(sizeof(T)) == 16 && sizeof(T) == 2) {
+                return fail(SIHC_ERR_INVALID, "%s: internal weight-gradient shape", what);  // never left to k_wgrad
+              } else {
+                if (!waves)
+                  hipLaunchKernelGGL((k_wgrad<T, VV, KK, CAR, SD>), dim3(blocks1d(slices, chunks)), dim3(bcg, lanes),
+                                     lds, st, static_cast<const T*>(x), pk, part, index, events, g, tpb, slices, tt,
+                                     dk, gamma, gf32);
+              }
             }
           }
           return check_launch(what);
