@@ -3459,14 +3459,44 @@ int rw_tokens_per_lane(int cell, int events, bool read, bool dot2) {
   if (!read && events > 8 && events <= 12) return 32;
   return events <= 4 ? SIHC_RW_TPT : events <= 16 ? 16 : 64;
 }
-// The same for a launch of M tokens in blocks of tl token lanes x `slices` slices: halved, down
-// to one iteration of `unroll` tokens, while the grid holds fewer than three blocks per CU
-// (1,024 tokens x 768, 16 slots, E = 12: read 58 -> 32 us, write 88 -> 26).
+// The same for a launch of M tokens in blocks of tl token lanes x `slices` slices: fewer tokens,
+// down to one iteration of `unroll`, where the grid is small.
+//   4 slots: halved while the grid holds under three blocks per CU.
+//   16 slots: the run of least cost, a CU's share of the blocks times what one of them takes. A
+//     block's time is its tokens per lane, one more, and half of `stage` (its staged weights in
+//     units of a lane's token); of the k blocks of a CU, r run together (what `lds` allows, at most
+//     6), at 0.7 of the rate of two if alone, 1.05 for three and 1.1 for more. The five numbers
+//     are the best of a grid search over 765 measured launches (1-32 events, 512-32,768 tokens x
+//     128-1152 channels, bf16 and fp32): 3% faster on average than halving to three blocks per CU,
+//     17 of them 6-16% slower. 16,384 x 128 bf16, E = 1, read 12 us with 512
+//     blocks of 8 tokens, 15 with 1,024; fp32 2,048 x 1152, E = 8, write without carry 76 us with
+//     288, two of them per CU, 89 with 1,152; 1,024 x 768, E = 12: read 58 -> 32 us, write 88 -> 26
+//     against the longest run.
+//   16-slot bf16 writes of 9-12 and past 16 events: twice the tokens where that grid is two to
+//     three blocks per CU (16,384 x 768, E = 12, without carry: 154 us with 768 blocks, 177 with
+//     1,536; 16,384 x 1152, E = 17: 400 and 445).
 int device_cus();
-int rw_tokens(int cell, int events, bool read, bool dot2, int unroll, int64_t M, int tl, int slices) {
-  int t = rw_tokens_per_lane(cell, events, read, dot2);
-  const int64_t blocks = 3 * int64_t(std::max(device_cus(), 1));
-  while (t / 2 >= unroll && ((M + tl * t - 1) / (tl * t)) * slices < blocks) t /= 2;
+int rw_tokens(int cell, int events, bool read, bool dot2, int unroll, int64_t M, int tl, int slices, size_t lds,
+              double stage) {
+  const int longest = rw_tokens_per_lane(cell, events, read, dot2);
+  const int64_t cus = std::max(device_cus(), 1);
+  auto blocks = [&](int n) { return ((M + int64_t(tl) * n - 1) / (int64_t(tl) * n)) * slices; };
+  int t = longest;
+  if (cell == 2) {
+    while (t / 2 >= unroll && blocks(t) < 3 * cus) t /= 2;
+    return t;
+  }
+  if (dot2 && !read && (events > 16 || (events > 8 && events <= 12)) && blocks(2 * t) >= 2 * cus &&
+      blocks(2 * t) <= 3 * cus)
+    return 2 * t;
+  const int64_t r = std::min<int64_t>(6, std::max<int64_t>(1, 160 * 1024 / int64_t(std::max<size_t>(lds, 1))));
+  auto share = [](int64_t n) { return n == 1 ? 1 / 0.7 : n == 2 ? 2. : n == 3 ? 3 / 1.05 : n / 1.1; };
+  auto cost = [&](int n) {
+    const int64_t k = (blocks(n) + cus - 1) / cus;
+    return (n + 1 + 0.5 * stage) * (double(k / r) * share(r) + (k % r ? share(k % r) : 0.));
+  };
+  for (int n = longest / 2; n >= unroll; n /= 2)
+    if (cost(n) < 0.985 * cost(t)) t = n;
   return t;
 }
 
@@ -4276,10 +4306,11 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
                                : shape_for(channels, V, events <= 8 ? 64 : SIHC_RW_BCG_K4, events * S * wbytes,
                                            SIHC_RW_LDS_K4);  // 64 lanes to 8 events: E = 4 569 -> 542 us
   const int unroll = d2 ? SIHC_RD2_U : cell == 2 ? SIHC_RW_UNROLL : SIHC_RW_UNROLL_K4;
-  const int tpb = sh.tl * rw_tokens(cell, events, true, d2, unroll, g.M, sh.tl, sh.slices);
+  const size_t lds = size_t(events) * S * sh.bcg * V * wbytes;
+  const double stage = double(events) * S * wbytes / (double(S + events) * es * sh.tl);
+  const int tpb = sh.tl * rw_tokens(cell, events, true, d2, unroll, g.M, sh.tl, sh.slices, lds, stage);
   const int64_t chunks = (int64_t(g.M) + tpb - 1) / tpb;
   const int gs = tpb;  // one contiguous run per block (interleaved groups measured no faster)
-  const size_t lds = size_t(events) * S * sh.bcg * V * wbytes;
   const PtrPack pk = pack(ptrs, events);
   return with_dtype(dtype, [&](auto t) {
     using T = decltype(t);
@@ -4358,10 +4389,11 @@ int sihc_write(const void* x, const void* const* updates, const void* beta, void
                                : shape_for(channels, V, E4 <= 8 ? 64 : SIHC_RW_BCG_K4, E4 * S * wbytes,
                                            SIHC_RW_LDS_K4);  // 64 lanes to 8 events: E = 4 1010 -> 964 us
   const int unroll = d2 ? SIHC_WR2_U : cell == 2 ? SIHC_RW_UNROLL : SIHC_RW_UNROLL_K4;
-  const int tpb = sh.tl * rw_tokens(cell, E4, false, d2, unroll, g.M, sh.tl, sh.slices);
+  const size_t lds = size_t(E4) * S * sh.bcg * V * wbytes;
+  const double stage = double(E4) * S * wbytes / (double((add_x ? 2 : 1) * S + events) * es * sh.tl);
+  const int tpb = sh.tl * rw_tokens(cell, E4, false, d2, unroll, g.M, sh.tl, sh.slices, lds, stage);
   const int64_t chunks = (int64_t(g.M) + tpb - 1) / tpb;
   const int gs = tpb;  // one contiguous run per block (interleaved groups measured no faster)
-  const size_t lds = size_t(E4) * S * sh.bcg * V * wbytes;
   const PtrPack pk = pack(updates, events);
   auto launch = [&](auto tx, auto tw) {
     using TX = decltype(tx);
