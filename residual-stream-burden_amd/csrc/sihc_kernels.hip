@@ -3408,6 +3408,17 @@ int row_vec(int C, int elem, int max_v, bool in_place = false) {
     if (v <= max_v && v * elem <= 16 && v <= C && (!in_place || C % v == 0)) return v;
   return 1;
 }
+// The width for a launch of blocks(V) blocks: a vector that does not divide the row only for
+// rows of at least 24 channels and grids of more than one block per CU. Narrower rows and
+// smaller grids leave its few lanes idle (4,096 tokens x 130 bf16, 4 slots: read of 5 events 5.0
+// us with 2-element vectors, 6.9 with 8, write 7.2 and 12.8; 65,536 x 17 fp32: event backward 28
+// and 31).
+int device_cus();
+template <typename Blocks>
+int ragged_vec(int C, int elem, int max_v, bool in_place, Blocks&& blocks) {
+  const int whole = row_vec(C, elem, max_v, true), v = row_vec(C, elem, max_v, in_place);
+  return v == whole || (C >= 24 && blocks(v) > device_cus()) ? v : whole;
+}
 bool any_equal(const void* const* a, int na, const void* const* b, int nb) {
   for (int i = 0; i < na; ++i)
     for (int j = 0; j < nb; ++j)
@@ -3498,6 +3509,29 @@ int rw_tokens(int cell, int events, bool read, bool dot2, int unroll, int64_t M,
   for (int n = longest / 2; n >= unroll; n /= 2)
     if (cost(n) < 0.985 * cost(t)) t = n;
   return t;
+}
+
+// 4-slot reads of ragged rows: 32 lanes where that covers the width with no more idle lanes than
+// 16 (fewer lines shared between slices: 16,384 tokens x 1154, E = 8, 136 -> 112 us).
+int read_lanes(int C, int V) {
+  const int cg16 = ((C + V - 1) / V + 15) / 16;
+  return C % V && cg16 % 2 == 0 ? 2 * SIHC_RW_BCG : SIHC_RW_BCG;
+}
+// Vector width of the 4-slot read and write. A dividing vector of at least 4 bytes also where the
+// wider one would leave over 40% of its lanes idle: 65,536 tokens x 130 bf16 (17 of 32 lanes), read
+// of 5 events 29 us with 2-element vectors, 38 with 8; write of 5 39 and 49; fp32 x 67 (17 of 32),
+// write of 3 31 us with one element, 39 with 4, but read of 12 20% slower.
+int stage_vec(int C, int es, int events, bool read, bool in_place, int64_t M) {
+  auto shape = [&](int v) { return shape_for(C, v, read ? read_lanes(C, v) : SIHC_RW_BCG, 0); };
+  const int t = rw_tokens_per_lane(2, read ? events : (events + 3) & ~3, read, false);
+  const int V = ragged_vec(C, es, 8, in_place, [&](int v) {
+    const Shape2D sh = shape(v);
+    return (M + sh.tl * t - 1) / (sh.tl * t) * sh.slices;
+  });
+  const int whole = row_vec(C, es, 8, true);
+  if (C % V == 0 || whole * es < 4 || (read && es == 4)) return V;
+  const Shape2D sh = shape(V);
+  return 5 * ((C + V - 1) / V) < 3 * sh.bcg * sh.slices ? whole : V;
 }
 
 int chunk_count(int64_t M, int tokens_per_chunk, int max_chunks) {
@@ -3945,7 +3979,15 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
     const void* const* outs = const_cast<const void* const*>(dout);
     in_place = any_equal(z, events, outs, events) || any_equal(&x, 1, outs, events);
   }
-  const int V = row_vec(g.C, es, 8, in_place);
+  // Rows too narrow for a vector that does not divide them (65,536 x 9 bf16: fused backward of 5
+  // updates 25 us with one element, 37 with 8; gamma gradient of 5 24 and 20), and one or two
+  // updates where the launch has no lanes to spare (4,096 x 130 bf16, one update: fused backward
+  // 8.4 us with 2-element vectors, 10.4 with 8, alone 6.4 and 8.7; alone also up to 256 channels,
+  // 65,536 x 99 22 and 26).
+  const bool few = !carrier && events <= 2 &&
+                   (int64_t(g.M) * g.C < (1 << 20) || (!dout && events == 1 && es == 2 && g.C < 256));
+  const int narrow = carrier ? 24 : dout ? (es == 2 ? 24 : 12) : events <= 2 ? 24 : 8;
+  const int V = row_vec(g.C, es, 8, in_place || g.C < narrow || few);
   int bcg, slices;
   wgrad_block(g.C, V, events, &bcg, &slices);
   const int tpb = int((int64_t(g.M) + chunks - 1) / chunks);
@@ -4272,8 +4314,9 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
   hipStream_t st = static_cast<hipStream_t>(stream);
   // (16-slot fp32 keeps a dividing vector: 4,096 tokens x 627, E = 8, read 90 us with 1-channel
   // lanes, 106 with 2; write 140 and 146)
-  const int V = row_vec(channels, es, cell == 2 ? 8 : SIHC_RW_VEC_K4, cell == 4 && es == 4);
+  int V = row_vec(channels, es, cell == 2 ? 8 : SIHC_RW_VEC_K4, cell == 4 && es == 4);
   const int S = cell * cell;
+  if (cell == 2) V = stage_vec(channels, es, events, true, false, g.M);
   // 16 slots, bf16 weights, 2-channel lanes: weights packed as bf16 in LDS (half the
   // bytes, so twice the channels per block within the LDS budget)
   const bool wb = dtype == SIHC_DTYPE_BF16 &&
@@ -4298,11 +4341,7 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
       return check_launch(what);
     });
   }
-  // ragged rows: 32 lanes where that covers the width with no more idle lanes than 16 (fewer
-  // lines shared between slices: 16,384 tokens x 1154, E = 8, 136 -> 112 us)
-  const int cg16 = ((channels + V - 1) / V + 15) / 16;
-  const int lanes2 = channels % V && cg16 % 2 == 0 ? 2 * SIHC_RW_BCG : SIHC_RW_BCG;
-  const Shape2D sh = cell == 2 ? shape_for(channels, V, lanes2, events * S * wbytes)
+  const Shape2D sh = cell == 2 ? shape_for(channels, V, read_lanes(channels, V), events * S * wbytes)
                                : shape_for(channels, V, events <= 8 ? 64 : SIHC_RW_BCG_K4, events * S * wbytes,
                                            SIHC_RW_LDS_K4);  // 64 lanes to 8 events: E = 4 569 -> 542 us
   const int unroll = d2 ? SIHC_RD2_U : cell == 2 ? SIHC_RW_UNROLL : SIHC_RW_UNROLL_K4;
@@ -4375,8 +4414,9 @@ int sihc_write(const void* x, const void* const* updates, const void* beta, void
   if (int rc = check_events(what, events, updates)) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int es = std::max(elem_size(x_dtype), elem_size(w_dtype));
-  const int V = row_vec(channels, es, cell == 2 ? 8 : SIHC_RW_VEC_K4, (add_x && x == out) || (cell == 4 && es == 4));
+  int V = row_vec(channels, es, cell == 2 ? 8 : SIHC_RW_VEC_K4, (add_x && x == out) || (cell == 4 && es == 4));
   const int S = cell * cell;
+  if (cell == 2) V = stage_vec(channels, es, events, false, add_x && x == out, g.M);
   const int E4 = (events + 3) & ~3;
   // 16 slots, bf16 weights, 2-channel lanes: weights packed as bf16 in LDS (as sihc_read)
   const bool wb = w_dtype == SIHC_DTYPE_BF16 &&
@@ -4532,8 +4572,14 @@ int sihc_triangular(const void* base, const void* const* updates, const void* ga
   if (int rc = check_events(what, active, updates)) return rc;
   const int es = elem_size(dtype);
   const void* dst = out;
-  const int V = row_vec(channels, es, 8, base == out || any_equal(updates, active, &dst, 1));
   const int A4 = (active + 3) & ~3;
+  const bool in_place = base == out || any_equal(updates, active, &dst, 1);
+  int V = row_vec(channels, es, 8, in_place);
+  if (active == 1 && es == 2)  // (4,096 x 130: 4.3 us with 2-element vectors, 5.6 with 8; fp32 and more updates gain)
+    V = ragged_vec(channels, es, 8, in_place, [&](int v) {
+      const Shape2D s = shape_for(channels, v, SIHC_RW_BCG, A4 * 4);
+      return (rows + s.tl * 4 - 1) / (s.tl * 4) * s.slices;
+    });
   const Shape2D sh = shape_for(channels, V, SIHC_RW_BCG, A4 * 4);
   // 32-token blocks (64 with one update): 3-5% faster than 128-token ones
   const int tpb = sh.tl * (active == 1 ? 4 : 2);
@@ -4767,7 +4813,12 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
     return fail(SIHC_ERR_INVALID, "%s: weights must be aligned to %d bytes", what, std::min(16, S * es));
   const void* ins[] = {grad_x_out, grad_z_out, x_out, dz};
   const void* outs[] = {grad_x, grad_dz};
-  int V = event_vec(channels, es, cell, any_equal(outs, 2, ins, 4));
+  const bool in_place = any_equal(outs, 2, ins, 4);
+  int V = event_vec(channels, es, cell, in_place);
+  if (cell == 2)  // (4,096 x 130 bf16: 14 us with 2-element vectors, 19 with 4; fp32 17 and 14)
+    V = ragged_vec(channels, es, SIHC_EV_VEC, in_place, [&](int v) {
+      return es == 2 ? int64_t(max_chunks) * shape_for(channels, v, SIHC_EV_BCG, 0).slices : INT64_MAX;
+    });
   while (cell == 4 && V > 1 && ((beta && !aligned(beta, std::min(16, V * S * es))) ||
                    (has_g && !aligned(alpha_next, std::min(16, V * S * es)))))
     V /= 2;
