@@ -14,6 +14,7 @@ import torch
 from helpers import announce, assert_parity
 from oracle import sihc_oracle as O
 from sihc_hip import launch
+from sihc_hip._lib import check, lib, ptr_array
 
 pytestmark = pytest.mark.gpu
 
@@ -105,3 +106,99 @@ def test_ragged_rows(dtype, slots, channels):
     back = Out(x.shape, dtype)
     launch.scatter_add_cells(_off(cells), index.cuda(), out=back.t)
     assert torch.equal(back.check(), x.cuda())
+
+
+# Tokens for which the launches hold more blocks than a device has CUs, so that rows a vector does
+# not divide take it all the same (smaller grids keep a dividing one).
+MANY = (64, 16)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("channels", [24, 67, 130, 259])
+def test_ragged_rows_of_large_grids(dtype, channels):
+    """Reads, writes, triangular and the per-event backward at 16,384 tokens: the oracle's values,
+    and the bits of whole rows one element off alignment."""
+    announce(f"ragged rows, large grid C={channels} {dtype}")
+    gen = torch.Generator().manual_seed(channels)
+    (b, g), c, events = MANY, channels, 3
+
+    def draw(*shape, scale=1.0):
+        return (scale * torch.randn(*shape, generator=gen)).to(dtype)
+
+    x, z = draw(b, 2 * g, 2 * g, c), [draw(b, g * g, c) for _ in range(events)]
+    w, gamma = (0.25 + 0.1 * draw(events, c, 4).float()).to(dtype), draw(events, c).float()
+    xd, zd, wd, gd = x.cuda(), [t.cuda() for t in z], w.cuda(), gamma.cuda()
+    outs = [Out((b, g * g, c), dtype) for _ in range(events)]
+    launch.read(_off(xd), wd, out=[o.t for o in outs])
+    for o, want, a in zip(outs, O.read(x, w), launch.read(xd, wd)):
+        assert_parity(o.check(), want, dtype, what="read")
+        assert torch.equal(o.t, a)
+    out = Out(x.shape, dtype)
+    launch.write(_off(xd), [_off(t) for t in zd], wd, out=out.t)
+    assert_parity(out.check(), O.write(x, z, w), dtype, what="write")
+    assert torch.equal(out.t, launch.write(xd, zd, wd))
+    for active in (1, 3):
+        got = launch.triangular(_off(zd[2]), [_off(t) for t in zd[:active]], gd[:active].contiguous())
+        assert_parity(got, O.triangular_torch(z[2], z[:active], gamma[:active]), dtype, what="triangular")
+    got = launch.event_backward(_off(xd), _off(zd[1]), xd, zd[0], wd[0], wd[1])
+    want = O.event_backward(x, z[1], x, z[0], w[0], w[1])
+    for name, a, e, kind in zip(("dX", "ddz", "dbeta", "dalpha"), got, want, ("elementwise",) * 2 + ("reduced",) * 2):
+        assert_parity(a, e.to(dtype), dtype, what=name, kind=kind)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("channels", [67, 130, 259])
+def test_outputs_that_are_inputs(dtype, channels):
+    """Every entry point that lets an output be one of its inputs, at widths whose last lane
+    overlaps its neighbour where it is not: the bits of the call with its own output."""
+    announce(f"in place C={channels} {dtype}")
+    gen = torch.Generator(device="cuda").manual_seed(channels)
+    (b, g), c, L = MANY, channels, lib()
+    code, m, st = launch.dtype_code(dtype), b * g * g, launch._stream(torch.device("cuda"))
+
+    def draw(*shape):
+        return torch.empty(*shape, device="cuda").normal_(generator=gen).to(dtype)
+
+    x, y, z = draw(b, 2 * g, 2 * g, c), draw(b, 2 * g, 2 * g, c), [draw(b, g * g, c) for _ in range(5)]
+    w = draw(2, c, 4)
+    p = torch.Tensor.data_ptr
+
+    gammas = {a: torch.empty(a, c, device="cuda").normal_(generator=gen) for a in (1, 2, 3, 5)}
+    for active, gamma in gammas.items():
+        want = launch.triangular(z[0], z[:active], gamma)
+        for over in (0, active - 1, None):  # over an update (the base is z[0] too), or over a base of its own
+            base, ups = z[0].clone(), [t.clone() for t in z[:active]]
+            out = base if over is None else ups[over]
+            check(L.sihc_triangular(p(base), ptr_array(map(p, ups)), p(gamma), p(out), active, m, c, code, 0, st))
+            assert torch.equal(out, want)
+        wdz, wdg = launch.triangular_backward(z[4], z[:active], gamma, out_dtype=torch.float32)
+        ws = launch._workspace(L.sihc_triangular_gamma_grad_workspace_size(active, m, c), x.device)
+        for over in ("updates", "gradient") if active == 1 else ("updates",):
+            grad, ups, dg = z[4].clone(), [t.clone() for t in z[:active]], torch.empty_like(wdg)
+            outs = ups if over == "updates" else [grad]
+            check(L.sihc_triangular_backward(p(grad), ptr_array(map(p, ups)), p(gamma), ptr_array(map(p, outs)), p(dg),
+                                             active, m, c, code, 0, 0, p(ws), ws.numel() * 4, st))
+            assert all(torch.equal(a, e) for a, e in zip(outs, wdz))
+            # narrower lanes sum other rows together: 64 roundings of a random chain
+            bound = 64 * 2 ** -24 * torch.stack([(z[4].float() * t.float()).abs().sum((0, 1)) for t in z[:active]])
+            assert ((dg - wdg).abs() <= bound).all()
+
+    want_x, want_z = launch.event_forward(x, z[0], w[0], w[1])
+    for over_x, over_z in ((True, False), (False, True), (True, True)):
+        xi, zi = x.clone(), z[0].clone()
+        xo, zo = xi if over_x else torch.empty_like(x), zi if over_z else torch.empty_like(zi)
+        check(L.sihc_event_forward(p(xi), p(zi), p(w[0]), p(w[1]), p(xo), p(zo), b, g, 2, c, None, code, st))
+        assert torch.equal(xo, want_x) and torch.equal(zo, want_z)
+
+    want = launch.event_backward(y, z[1], x, z[0], w[0], w[1])
+    ws = launch._workspace(L.sihc_event_backward_workspace_size(b, g, 2, c), x.device)
+    for over in ("gx", "x", "dz", "gz"):
+        gx, gz, xi, dz = y.clone(), z[1].clone(), x.clone(), z[0].clone()
+        ox = {"gx": gx, "x": xi}.get(over, torch.empty_like(x))
+        oz = {"dz": dz, "gz": gz}.get(over, torch.empty_like(dz))
+        ob, oa = torch.empty_like(w[0]), torch.empty_like(w[1])
+        check(L.sihc_event_backward(p(gx), p(gz), p(xi), p(dz), p(w[0]), p(w[1]), p(ox), p(oz), p(ob), p(oa), b, g, 2, c,
+                                    None, code, code, p(ws), ws.numel() * 4, st))
+        assert torch.equal(ox, want[0]) and torch.equal(oz, want[1])
+        assert_parity(ob, want[2].cpu(), dtype, what="dbeta", kind="reduced")
+        assert_parity(oa, want[3].cpu(), dtype, what="dalpha", kind="reduced")
