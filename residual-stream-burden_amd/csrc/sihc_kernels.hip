@@ -2532,7 +2532,7 @@ __global__ void __launch_bounds__(256) k_fill_zero(TO* __restrict__ out, int64_t
 // triangular: out[m,c] = base[m,c] + sum_j gamma[j,c] * upd_j[m,c]
 // (active count padded to a multiple of 4 with zero gamma rows, as in k_write)
 // ----------------------------------------------------------------------------------
-template <typename T, typename TG, int V, int NTM>
+template <typename T, typename TG, int V, int NTM, bool RAG>
 __global__ void __launch_bounds__(256) k_triangular(const T* __restrict__ base, PtrPack upd,
                                                     const TG* __restrict__ gamma, T* __restrict__ out,
                                                     int A, int M, int C, int gs, int nchunks, int nslices) {
@@ -2542,7 +2542,6 @@ __global__ void __launch_bounds__(256) k_triangular(const T* __restrict__ base, 
   const int BCG = blockDim.x, TL = blockDim.y;
   const int BC = BCG * V;
   int slice, chunk;
-  constexpr bool RAG = NTM == 0;  // only rows that V does not divide are launched without hints
   slice_chunk_row(int(gridDim.x), nslices, RAG, slice, chunk);
   const int cs = slice * BC;
   const int A4 = (A + 3) & ~3;
@@ -4597,12 +4596,20 @@ int sihc_triangular(const void* base, const void* const* updates, const void* ga
         if constexpr (VV * sizeof(T) > 16) {
           return fail(SIHC_ERR_INVALID, "%s: internal vector width", what);
         } else {
-          return with_hints<SIHC_TRI_NTM>(channels % VV ? 0 : triangular_hints(active), [&](auto nt) {
-            constexpr int NT = decltype(nt)::value;
-            hipLaunchKernelGGL((k_triangular<T, TG, VV, NT>), dim3(blocks1d(sh.slices, chunks)), dim3(sh.bcg, sh.tl),
-                               lds, st, static_cast<const T*>(base), pk, static_cast<const TG*>(gamma),
-                               static_cast<T*>(out), active, int(rows), channels, gs, int(chunks), sh.slices);
-            return check_launch(what);
+          return with_bool(channels % VV != 0, [&](auto rg) {
+            constexpr bool RAG = decltype(rg)::value;
+            auto go = [&](auto nt) {
+              hipLaunchKernelGGL((k_triangular<T, TG, VV, decltype(nt)::value, RAG>), dim3(blocks1d(sh.slices, chunks)),
+                                 dim3(sh.bcg, sh.tl), lds, st, static_cast<const T*>(base), pk,
+                                 static_cast<const TG*>(gamma), static_cast<T*>(out), active, int(rows), channels, gs,
+                                 int(chunks), sh.slices);
+              return check_launch(what);
+            };
+            if constexpr (RAG) {
+              return go(IC<(SIHC_TRI_NTM < 0 ? 0 : SIHC_TRI_NTM)>{});
+            } else {
+              return with_hints<SIHC_TRI_NTM>(triangular_hints(active), go);
+            }
           });
         }
       });
