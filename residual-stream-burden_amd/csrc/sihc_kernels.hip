@@ -4836,10 +4836,24 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
   // every other CU narrower slices, whose blocks take more tokens at a time (16 slots, 2,048 x
   // 768: 76 -> 63 us, 256 x 768: 57 -> 37; 4,096 x 768, 192 blocks: 84 -> 118).
   const int64_t cus = std::max(device_cus(), 1);
-  auto blocks_with = [&](int bcg) { return int64_t(max_chunks) * shape_for(channels, V, bcg, 0).slices; };
+  // Tokens per interleaved group: a multiple of one loop iteration (SIHC_EV_UNROLL x TL tokens);
+  // group 0 means one contiguous run of tokens per chunk. Narrow slices take more tokens an
+  // iteration, so they have fewer groups than chunks at few tokens: blocks past the last group
+  // would own no token, and their partial rows would be written and summed for nothing.
+  auto group = [&](int tl, int n) {
+    return group_tokens(cell == 2 ? SIHC_EV_GROUP : SIHC_EV_GROUP_K4, g.M, n, SIHC_EV_UNROLL * tl);
+  };
+  auto live_chunks = [&](int tl, int n) {
+    const int gs = group(tl, n);
+    return int(std::min<int64_t>(n, (int64_t(g.M) + gs - 1) / gs));
+  };
+  auto blocks_with = [&](int bcg) {
+    const Shape2D s = shape_for(channels, V, bcg, 0);
+    return int64_t(live_chunks(s.tl, max_chunks)) * s.slices;
+  };
   int lanes = cell == 2 && V * es == 16 ? 16 : SIHC_EV_BCG;
   if (cell == 4 && es == 2 && V == 2 && blocks_with(64) >= cus) lanes = 64;
-  while (lanes > 4 && blocks_with(lanes) < cus / 2) lanes /= 2;
+  while (lanes > 4 && blocks_with(lanes) < cus / 2 && blocks_with(lanes / 2) > blocks_with(lanes)) lanes /= 2;
   const Shape2D sh = shape_for(channels, V, lanes, 0);
   const size_t lds = size_t(sh.tl) * sh.bcg * S * V * sizeof(float);  // TL x (BCG*S*V) floats
   if (carry && (sh.tl * sh.bcg != 256 || lds < FINALIZE_LDS(4) * sizeof(float)))
@@ -4875,10 +4889,8 @@ static int event_backward_impl(const char* what, const void* grad_x_out, const v
                 kfn = reinterpret_cast<const void*>(&k_event_bwd<T, VV, KK, HH, HG, HW, STT, RAG, NR>);
               }
               chunks = whole_rounds(sh.slices, max_chunks, resident_blocks(kfn, sh.bcg * sh.tl, lds));
-              // token groups: a multiple of one loop iteration (SIHC_EV_UNROLL x TL tokens);
-              // group 0 means one contiguous run of tokens per chunk
-              const int gs = group_tokens(KK == 2 ? SIHC_EV_GROUP : SIHC_EV_GROUP_K4, g.M, chunks,
-                                          SIHC_EV_UNROLL * sh.tl);
+              chunks = live_chunks(sh.tl, chunks);
+              const int gs = group(sh.tl, chunks);
               EvCarry cy{};
               if (carry) cy = *prev;
               cy.nmain = int(blocks1d(sh.slices, chunks));

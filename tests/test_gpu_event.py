@@ -7,6 +7,7 @@ import torch
 from helpers import announce, assert_parity
 from oracle import sihc_oracle as O
 from sihc_hip import launch
+from sihc_hip._lib import check, lib
 from sihc_hip.event_ops import event_write_read, literal_stage
 
 pytestmark = pytest.mark.gpu
@@ -351,3 +352,33 @@ def test_event_backward_launch_shapes(slots, dtype, batch, grid, channels):
     index = torch.arange(grid * grid, dtype=torch.int32).repeat(batch, 1).cuda()
     again = launch.event_backward(*(t.cuda() for t in (gx, gz, xo, dz, beta, alpha)), index=index)
     assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+@pytest.mark.parametrize("slots,dtype,batch,grid,channels", [(4, torch.bfloat16, 1, 16, 264), (4, torch.float32, 1, 16, 130),
+                                                             (4, torch.bfloat16, 1, 5, 64), (16, torch.bfloat16, 1, 16, 136),
+                                                             (16, torch.float32, 3, 13, 40)])
+def test_event_backward_writes_no_partial_row_without_tokens(slots, dtype, batch, grid, channels):
+    """At few tokens narrow slices take more tokens an iteration than a chunk holds: only chunks with
+    tokens are launched and summed. Random gradients leave no such row at zero."""
+    announce(f"event live rows slots={slots} {dtype} b={batch} g={grid} C={channels}")
+    gen = torch.Generator(device="cuda").manual_seed(channels)
+    k, L = O.cell_edge(slots), lib()
+
+    def draw(*shape):
+        return torch.empty(*shape, device="cuda").normal_(generator=gen).to(dtype)
+
+    x, y = draw(batch, k * grid, k * grid, channels), draw(batch, k * grid, k * grid, channels)
+    dz, gz, w = draw(batch, grid * grid, channels), draw(batch, grid * grid, channels), draw(2, channels, slots)
+    rows = 2 * slots * channels
+    ws = torch.full((L.sihc_event_backward_workspace_size(batch, grid, k, channels) // 4,), float("nan"), device="cuda")
+    outs = [torch.empty_like(x), torch.empty_like(dz), torch.empty_like(w[0]), torch.empty_like(w[1])]
+    p, code = torch.Tensor.data_ptr, launch.dtype_code(dtype)
+    check(L.sihc_event_backward(p(y), p(gz), p(x), p(dz), p(w[0]), p(w[1]), *map(p, outs), batch, grid, k, channels,
+                                None, code, code, p(ws), ws.numel() * 4, launch._stream(x.device)))
+    part = ws[:ws.numel() // rows * rows].view(-1, rows)
+    written = part[~part.isnan().any(1)]
+    assert len(written) >= 1 and part.isnan().all(1).sum() == len(part) - len(written)
+    assert (written != 0).any(1).all()
+    want = O.event_backward(y.cpu(), gz.cpu(), x.cpu(), dz.cpu(), w[0].cpu(), w[1].cpu())
+    assert_parity(outs[2], want[2].to(dtype), dtype, what="dbeta", kind="reduced")
+    assert_parity(outs[3], want[3].to(dtype), dtype, what="dalpha", kind="reduced")
