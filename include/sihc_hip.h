@@ -88,8 +88,8 @@ int sihc_weight_grad(const void *x, const void *const *z, void *out, int events,
  * sihc_weight_grad and a zero-carry sihc_write):
  *   grad_x[m,s,c]     = sum_e alpha[e,c,s] * grads_e[m,c]
  *   grad_alpha[e,c,s] = sum_m x[m,s,c] * grads_e[m,c]    (as sihc_weight_grad)
- * alpha is in dtype. No output may overlap an input. Workspace:
- * sihc_weight_grad_workspace_size.
+ * alpha is in dtype. No output may overlap an input or another output (an output pointer that
+ * equals an input is refused). Workspace: sihc_weight_grad_workspace_size.
  * Replaces: sublayer_kernels.py:276-287 (the read's backward: `_write_impl` and
  * `_weights_backward` on the same gradients). */
 int sihc_read_backward(const void *x, const void *const *grads, const void *alpha, void *grad_x,
@@ -98,9 +98,12 @@ int sihc_read_backward(const void *x, const void *const *grads, const void *alph
                        void *workspace, size_t workspace_bytes, void *stream);
 
 /* Whole adjoint of sihc_write except the identity to x, in one pass over grad_out and the E
- * updates under the same conditions (otherwise sihc_weight_grad and sihc_read):
+ * updates for 4-slot cells, up to 8 events and at least 16 bytes of channels (otherwise
+ * sihc_weight_grad and sihc_read):
  *   grad_updates_e[m,c] = sum_s beta[e,c,s] * grad_out[m,s,c]
  *   grad_beta[e,c,s]    = sum_m grad_out[m,s,c] * updates_e[m,c]
+ * beta is in dtype. No output may overlap an input or another output (an output pointer that
+ * equals an input is refused). Workspace: sihc_weight_grad_workspace_size.
  * Replaces: sublayer_kernels.py:295-306 (the write's backward: `sublayer_read` and
  * `_weights_backward` on the same carrier gradient). */
 int sihc_write_backward(const void *grad_out, const void *const *updates, const void *beta,

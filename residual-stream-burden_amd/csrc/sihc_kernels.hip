@@ -4526,6 +4526,10 @@ int sihc_read_backward(const void* x, const void* const* grads, const void* alph
   if (g.M == 0) return fill_zero(out_dtype, grad_alpha, int64_t(events) * cell * cell * channels, st, what);
   if (!x || !alpha || !grad_x) return fail(SIHC_ERR_INVALID, "%s: null tensor", what);
   if (int rc = check_events(what, events, grads)) return rc;
+  const void* outs[] = {grad_x, grad_alpha};
+  const void* ins[] = {x, alpha};
+  if (any_equal(outs, 2, ins, 2) || any_equal(outs, 2, grads, events))
+    return fail(SIHC_ERR_INVALID, "%s: an output is one of the inputs", what);
   if (fused_backward(g, events, 24, dtype))
     return launch_stage_backward<MM_READ>(what, x, grads, alpha, grad_x, nullptr, grad_alpha, events, g, index, dtype,
                                           out_dtype, workspace, workspace_bytes, st);
@@ -4550,7 +4554,13 @@ int sihc_write_backward(const void* grad_out, const void* const* updates, const 
   if (g.M == 0) return fill_zero(out_dtype, grad_beta, int64_t(events) * cell * cell * channels, st, what);
   if (!grad_out || !beta) return fail(SIHC_ERR_INVALID, "%s: null tensor", what);
   if (int rc = check_events(what, events, updates)) return rc;
-  if (int rc = check_events(what, events, const_cast<const void* const*>(grad_updates))) return rc;
+  const void* const* outs = const_cast<const void* const*>(grad_updates);
+  if (int rc = check_events(what, events, outs)) return rc;
+  const void* out0 = grad_beta;
+  const void* ins[] = {grad_out, beta};
+  if (any_equal(outs, events, ins, 2) || any_equal(outs, events, updates, events) || any_equal(&out0, 1, ins, 2) ||
+      any_equal(&out0, 1, updates, events))
+    return fail(SIHC_ERR_INVALID, "%s: an output is one of the inputs", what);
   if (fused_backward(g, events, 8, dtype))
     return launch_stage_backward<MM_WRITE>(what, grad_out, updates, beta, nullptr, grad_updates, grad_beta, events, g,
                                            index, dtype, out_dtype, workspace, workspace_bytes, st);

@@ -233,3 +233,18 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "libsihc_hip.so")
     with pytest.raises(RuntimeError, match="missing"):
         _lib.lib()
+
+
+def test_stage_backwards_refuse_an_output_that_is_an_input():
+    lib, ws = _lib.lib(), 1 << 30
+    at = [FAKE + 0x1000 * i for i in range(8)]
+    two, outs = _lib.ptr_array(at[:2]), _lib.ptr_array(at[2:4])
+    for grad_x, grad_alpha in ((at[0], at[6]), (at[4], at[6]), (at[5], at[6]), (at[7], at[1]), (at[7], at[4])):
+        rc = lib.sihc_read_backward(at[4], two, at[5], grad_x, grad_alpha, 2, 2, 16, 2, 64, None, 1, 1, FAKE, ws, None)
+        assert rc == 1 and b"one of the inputs" in lib.sihc_last_error()
+    for updates, grads, grad_beta in ((two, two, at[6]), (two, _lib.ptr_array([at[2], at[4]]), at[6]),
+                                      (two, _lib.ptr_array([at[5], at[2]]), at[6]), (two, outs, at[5]),
+                                      (two, outs, at[0])):
+        rc = lib.sihc_write_backward(at[4], updates, at[5], grads, grad_beta, 2, 2, 16, 2, 64, None, 1, 1, FAKE, ws,
+                                     None)
+        assert rc == 1 and b"one of the inputs" in lib.sihc_last_error()
