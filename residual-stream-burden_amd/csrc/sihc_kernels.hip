@@ -272,11 +272,6 @@ template <> struct RawT<2> { using type = uint16_t; };
 // triangular with 7+ updates); hinted loads without hinted stores slow the balanced
 // streams down (1-3%); slices narrower than a 128-byte line take no hint (16-slot
 // read/write with 16+ events: 7-60% slower).
-// First channel of the lane whose vector nominally starts at channel cb of a C-wide row: the
-// last vector of a row that V does not divide is moved back to end with the row, so its first
-// channels are computed twice, with the same result, by two lanes. Lanes with cb >= C are idle.
-__device__ __forceinline__ int lane_channel(int cb, int V, int C) { return min(cb, C - V); }
-
 template <bool NT = false, typename R>
 __device__ __forceinline__ R ld(const R* p) {
   if constexpr (NT) {
@@ -297,6 +292,11 @@ __device__ __forceinline__ void st(R* p, R v) {
     *p = v;
   }
 }
+
+// First channel of the lane whose vector nominally starts at channel cb of a C-wide row: the
+// last vector of a row that V does not divide is moved back to end with the row, so its first
+// channels are computed twice, with the same result, by two lanes. Lanes with cb >= C are idle.
+__device__ __forceinline__ int lane_channel(int cb, int V, int C) { return min(cb, C - V); }
 
 // BYTES of a row at p. Rows of any width start at any element, so these promise only the
 // alignment of the element; the instruction is the same wide load or store (gfx950 takes
@@ -496,8 +496,9 @@ __device__ __forceinline__ void slice_chunk_unless8(int blk, int nslices, int& s
 
 // Block order of a kernel whose rows V does not divide (ragged): neighbouring slices share a
 // line at each end of every row piece, so they run on one XCD (contiguous order) and meet in
-// its L2; such launches also carry no non-temporal hints, which would let a shared line go
-// before its second use and write it in two partial pieces. The 16-slot per-event kernels take
+// its L2; such launches also carry no non-temporal hints (but k_event_fwd_rows, whose blocks hold
+// whole rows), which would let a shared line go before its second use and write it in two partial
+// pieces. The 16-slot per-event kernels take
 // this order where a slice row is narrower than a line (2,048 tokens x 768, 64-byte rows: 70 us
 // in the hardware's order, 63 in this one), and the hardware's, with the slice rotated, where
 // it is not, so that the 8 XCDs stream through one window of tokens (32,768 x 1152 bf16,
@@ -1080,14 +1081,14 @@ __global__ void __launch_bounds__(256) k_read_w(const bf16_t* __restrict__ x, co
   const uint32_t* aw = reinterpret_cast<const uint32_t*>(alpha);
   for (int i = tid; i < E * BC * 2; i += 256) {
     const int e = i / (BC * 2), r = i - e * BC * 2, cl = r >> 1, pr = r & 1;
-    const int cb = cs + cl / V * V, c = lane_channel(cb, V, g.C) + cl % V;
-    ap[(e * 2 + pr) * BC + cl] = cb < g.C ? aw[(int64_t(e) * g.C + c) * 2 + pr] : 0u;
+    const int c = cs + cl;
+    ap[(e * 2 + pr) * BC + cl] = c < g.C ? aw[(int64_t(e) * g.C + c) * 2 + pr] : 0u;
   }
   // cell tile: unit u = (token t, channel group j): 4 slot vectors of 8 channels ->
   // 8 pair words per slot pair
   for (int u = tid; u < RDW_TT * LX; u += 256) {
-    const int t = u / LX, j = u % LX, cb = cs + j * V, c = lane_channel(cb, V, g.C);
-    if (t < tn && cb < g.C) {
+    const int t = u / LX, j = u % LX, c = cs + j * V;
+    if (t < tn && c < g.C) {
       const int64_t p0 = cell_pixel0(m0 + t, g, index);
       u32x4 v[4];
 #pragma unroll
@@ -1111,8 +1112,8 @@ __global__ void __launch_bounds__(256) k_read_w(const bf16_t* __restrict__ x, co
     }
   }
   __syncthreads();
-  const int cb0 = cs + lx * V, c0 = lane_channel(cb0, V, g.C);
-  if (cb0 >= g.C) return;  // no barrier below
+  const int c0 = cs + lx * V;
+  if (c0 >= g.C) return;  // no barrier below
   for (int e = wave; e < E; e += 4) {
     const u32x4* ae = reinterpret_cast<const u32x4*>(ap + e * 2 * BC + lx * V);
     const u32x4 w00 = ae[0], w01 = ae[1];                       // pair 0, channels 0..3, 4..7
@@ -2762,6 +2763,8 @@ __global__ void __launch_bounds__(SIHC_EV_FWD_THREADS, SIHC_EV_MINW) k_event_fwd
 // are whole contiguous runs of a carrier pixel row (2 x C elements per slot pair) and of
 // the dz / z_out rows. k_event_fwd's arithmetic per element (same bits); one-shot, no
 // loop: token blockIdx.x * TR + threadIdx.y.
+// RAG: rows that V does not divide; they keep the hints, since a block holds whole rows and no
+// line is shared between blocks but at the ends of a token's pixels.
 // ----------------------------------------------------------------------------------
 template <typename T, int V, bool HAS_Z, bool RAG>
 __global__ void __launch_bounds__(1024) k_event_fwd_rows(const T* __restrict__ x, const T* __restrict__ dz,
