@@ -145,3 +145,18 @@ def test_scatter_add_lists_every_contributor_in_order(dtype, grid, slots, channe
     }[pattern].to(torch.int32).contiguous()
     got = launch.scatter_add_cells(cells.cuda(), idx.cuda())
     assert torch.equal(got.cpu(), O.scatter_add_cells(cells, idx))
+
+
+@pytest.mark.parametrize("grid", [64, 128])
+def test_gather_adjoint_of_the_largest_grids(grid):
+    """16,384 cells a batch row, the limit: the contributors' list takes 64 KB of LDS beside the
+    wave counts. Whole numbers, so that sums of repeated cells are exact in any order."""
+    announce(f"gather adjoint grid={grid}")
+    gen = torch.Generator().manual_seed(grid)
+    n = grid * grid
+    cells = torch.randint(-8, 9, (1, n, 4, 12), generator=gen).float()
+    index = torch.randint(0, n, (1, n), generator=gen, dtype=torch.int32)
+    index[0, : n // 4] = 7  # one cell with a quarter of the tokens
+    got = launch.scatter_add_cells(cells.cuda(), index.cuda()).cpu()
+    want = torch.zeros(n, 4, 12).index_add_(0, index[0].long(), cells[0])
+    assert torch.equal(O.high_to_cells(got, 4).reshape(n, 4, 12), want)

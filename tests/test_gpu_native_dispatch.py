@@ -13,6 +13,7 @@ import time
 
 import pytest
 import torch
+import torch._dynamo.compiled_autograd
 import torch.utils.checkpoint
 from torch.utils._python_dispatch import TorchDispatchMode
 
@@ -341,6 +342,22 @@ def test_other_threads_run_during_a_native_call(name):
         sys.setswitchinterval(interval)
         other.join()
     assert seen
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_compiled_autograd_traces_the_native_backward(name):
+    """Compiled autograd traces each node's backward with fake tensors, for which the node calls the
+    registered ops."""
+    op, args, _ = _calls(torch.float32)[name]
+    out, leaves = _outs(op(*args)), _leaves(args)
+    torch.manual_seed(3)
+    up = [torch.randn_like(o) for o in out]
+    want = torch.autograd.grad(out, leaves, up, retain_graph=True)
+    torch._dynamo.reset()
+    with torch._dynamo.compiled_autograd._enable(torch.compile(backend="eager")):
+        torch.autograd.backward(out, up)
+    # (the write's two gradients may come from two kernels there: other orders of 2,048 products)
+    assert all(torch.allclose(t.grad, w, rtol=1e-5, atol=2048 * 2 ** -24) for t, w in zip(leaves, want))
 
 
 def test_vmap_forward_mode_and_subclasses_take_the_registered_op():

@@ -105,9 +105,9 @@ def test_infinities_stay_in_their_token_event_and_channel(dtype, events):
 
 
 def test_long_chunks_walk_every_group():
-    # 65,537 + 255 tokens: chunks of many interleaved groups with a ragged last one.
+    # 65,925 tokens: chunks of many interleaved 8-token groups, 5 tokens in the last one.
     announce("stage backward long")
-    x, z, w, _ = _inputs(4, 5, 257, 16, 24, torch.bfloat16, False, 1)
+    x, z, w, _ = _inputs(4, 5, 293, 15, 24, torch.bfloat16, False, 1)
     gx, ga = launch.read_backward(x.cuda(), [t.cuda() for t in z], w.cuda(), out_dtype=torch.float32)
     assert_parity(ga, O.weight_grad(x, z, 4), torch.float32, what="dalpha")
     assert_parity(gx, O.write(torch.zeros_like(x), z, w, add_x=False), torch.bfloat16, what="dx")
