@@ -3458,12 +3458,13 @@ int rw_tokens_per_lane(int cell, int events, bool read, bool dot2) {
   if (cell == 2) return read ? (events == 1 ? 4 : 2) : (events >= 4 ? 4 : SIHC_RW_TPT);
   if (dot2) {
     // 16-slot bf16 on k_read_d2 / k_write_d2, whose packed weights are cheap to stage: reads 8
-    // tokens and 16 past 16 events, writes 16 and 32 past 16 (32,768 tokens x 1152: read E = 12
-    // 432 us with 32 tokens, 420 with 8; write E = 12 662 with 32, 645 with 16; E = 24 907 with
-    // 64, 861 with 32; 8,192 x 768: read E = 8 71 with 32, 65 with 8; write E = 24 302 with 64,
-    // 192 with 32, 157 with 16, where the grid rule below lands)
+    // tokens and 16 past 16 events, writes 16, 32 past 16 and 64 past 20 (32,768 tokens x 1152: read
+    // E = 12 432 us with 32 tokens, 420 with 8; write E = 12 662 with 32, 645 with 16; 65,536 x 768:
+    // write E = 20 1,020 with 32, 1,073 with 64, E = 32 1,560 with 32, 1,472 with 64; 8,192 x 768:
+    // read E = 8 71 with 32, 65 with 8; write E = 24 302 with 64, 192 with 32, 157 with 16, where
+    // the grid rule below lands)
     if (read) return events <= 16 ? 8 : 16;
-    return events <= 4 ? 8 : events <= 16 ? 16 : 32;
+    return events <= 4 ? 8 : events <= 16 ? 16 : events <= 20 ? 32 : 64;
   }
   // 16 slots: the weight slice staged per block grows with E, so blocks grow too; with
   // hinted loads and stores reads with 3-12 events and writes with 9-12 gain from twice
@@ -3485,9 +3486,9 @@ int rw_tokens_per_lane(int cell, int events, bool read, bool dot2) {
 //     blocks of 8 tokens, 15 with 1,024; fp32 2,048 x 1152, E = 8, write without carry 76 us with
 //     288, two of them per CU, 89 with 1,152; 1,024 x 768, E = 12: read 58 -> 32 us, write 88 -> 26
 //     against the longest run.
-//   16-slot bf16 writes of 9-12 and past 16 events: twice the tokens where that grid is two to
-//     three blocks per CU (16,384 x 768, E = 12, without carry: 154 us with 768 blocks, 177 with
-//     1,536; 16,384 x 1152, E = 17: 400 and 445).
+//   16-slot bf16 writes of 9-12 and past 16 events: twice the tokens (past 20 events, the 64 of
+//     above) where that grid is two to three blocks per CU (16,384 x 768, E = 12, without carry:
+//     154 us with 768 blocks, 177 with 1,536; 16,384 x 1152, E = 17: 400 and 445).
 int device_cus();
 int rw_tokens(int cell, int events, bool read, bool dot2, int unroll, int64_t M, int tl, int slices, size_t lds,
               double stage) {
@@ -3499,9 +3500,10 @@ int rw_tokens(int cell, int events, bool read, bool dot2, int unroll, int64_t M,
     while (t / 2 >= unroll && blocks(t) < 3 * cus) t /= 2;
     return t;
   }
-  if (dot2 && !read && (events > 16 || (events > 8 && events <= 12)) && blocks(2 * t) >= 2 * cus &&
-      blocks(2 * t) <= 3 * cus)
-    return 2 * t;
+  if (dot2 && !read && (events > 16 || (events > 8 && events <= 12))) {
+    const int n = events > 20 ? t : 2 * t;
+    if (blocks(n) >= 2 * cus && blocks(n) <= 3 * cus) return n;
+  }
   const int64_t r = std::min<int64_t>(6, std::max<int64_t>(1, 160 * 1024 / int64_t(std::max<size_t>(lds, 1))));
   auto share = [](int64_t n) { return n == 1 ? 1 / 0.7 : n == 2 ? 2. : n == 3 ? 3 / 1.05 : n / 1.1; };
   auto cost = [&](int n) {
