@@ -601,9 +601,9 @@ PyObject* guarded(PyObject* self, F&& f) {
     return not_implemented();
   }
 }
-// f() as a call of the op of `self`, with the GIL released: a launch waits where the queue is full, and an allocation may wait for
-// the device. (The registered ops release it around every dispatch and launch.) Saved-tensor hooks
-// take it again for their own calls.
+// f() as a call of the op of `self`, with the GIL released: a launch waits where the queue is full,
+// and an allocation may wait for the device. (The registered ops release it around every dispatch
+// and launch.) Saved-tensor hooks take it again for their own calls.
 template <typename A, typename F>
 auto call(PyObject* self, A&& args, F&& f) {
   RECORD_FUNCTION(entry_of(self).name(), args());
@@ -707,7 +707,8 @@ PyObject* py_block_write(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     };
     return THPVariable_Wrap(call(self, listing, [&] {
       return unrecorded() ? run_write(x, updates, at::stack(betas), Tensor())
-                          : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas), std::string(entry_of(self).name()));
+                          : BlockWriteFn::apply(x, TensorList(updates), TensorList(betas),
+                                                std::string(entry_of(self).name()));
     }));
   });
 }
