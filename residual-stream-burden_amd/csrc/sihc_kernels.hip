@@ -3515,27 +3515,47 @@ int rw_tokens(int cell, int events, bool read, bool dot2, int unroll, int64_t M,
   return t;
 }
 
-// 4-slot reads of ragged rows: 32 lanes where that covers the width with no more idle lanes than
-// 16 (fewer lines shared between slices: 16,384 tokens x 1154, E = 8, 136 -> 112 us).
-int read_lanes(int C, int V) {
+// Lanes of the 4-slot read. Ragged rows: 32 where that covers the width with no more idle lanes
+// than 16 (fewer lines shared between slices: 16,384 tokens x 1154, E = 8, 136 -> 112 us) and the
+// grid holds at least three blocks per CU, whose staged weights are twice as large (buffers out of
+// cache: 8,192 x 131 bf16, E = 16, 22 us with 16 lanes, 27 with 32; 4,096 x 195, E = 8, 10.6 and
+// 12.5; 16,384 x 195, E = 8, 27 and 26).
+int read_lanes(int C, int V, int events, int64_t M) {
   const int cg16 = ((C + V - 1) / V + 15) / 16;
-  return C % V && cg16 % 2 == 0 ? 2 * SIHC_RW_BCG : SIHC_RW_BCG;
+  if (C % V == 0 || cg16 % 2 != 0) return SIHC_RW_BCG;
+  const Shape2D sh = shape_for(C, V, 2 * SIHC_RW_BCG, 0);
+  const int64_t tpb = int64_t(sh.tl) * rw_tokens_per_lane(2, events, true, false);
+  return (M + tpb - 1) / tpb * sh.slices >= 3 * int64_t(device_cus()) ? 2 * SIHC_RW_BCG : SIHC_RW_BCG;
 }
-// Vector width of the 4-slot read and write. A dividing vector of at least 4 bytes also where the
-// wider one would leave over 40% of its lanes idle: 65,536 tokens x 130 bf16 (17 of 32 lanes), read
-// of 5 events 29 us with 2-element vectors, 38 with 8; write of 5 39 and 49; fp32 x 67 (17 of 32),
-// write of 3 31 us with one element, 39 with 4, but read of 12 20% slower.
+// Vector width of the 4-slot read and write: a dividing vector also where the wider one would
+// leave lanes idle. Lanes in use, and times with buffers out of cache:
+//   writes, dividing vector of at least 4 bytes: up to 60% (65,536 tokens x 130 bf16, 17 of 32,
+//     write of 5 39 us with 2-element vectors, 49 with 8; fp32 x 67, 17 of 32, write of 3 31 us
+//     with one element, 39 with 4); of 2 bytes, past 8 events: up to 55% (16,384 x 131, 17 of 32,
+//     E = 24, write 56 us with one element, 66 with 8; x 195, 25 of 32, 76 and 70)
+//   reads of 2-element bf16 vectors: up to 60% (65,536 x 130, E = 5, 29 us, with 8 38)
+//   reads of one element, 8 or more events, rows of at least 64 channels and at most five blocks
+//     per CU: fp32 up to 90% (8,192 x 67, E = 16, 16 us with one element, 21 with 4; 4,096 x 195,
+//     E = 24, 36 and 44; 32,768 x 99, E = 16, 84 and 71, past the line; 16,384 x 35, E = 24, 23 and
+//     21), bf16 up to 55%, and past 16 events of at least 128 channels 80% (16,384 x 131, E = 24,
+//     48 and 59; x 163 60 and 69; 32,768 x 67 48 and 39)
 int stage_vec(int C, int es, int events, bool read, bool in_place, int64_t M) {
-  auto shape = [&](int v) { return shape_for(C, v, read ? read_lanes(C, v) : SIHC_RW_BCG, 0); };
   const int t = rw_tokens_per_lane(2, read ? events : (events + 3) & ~3, read, false);
-  const int V = ragged_vec(C, es, 8, in_place, [&](int v) {
+  auto shape = [&](int v) { return shape_for(C, v, read ? read_lanes(C, v, events, M) : SIHC_RW_BCG, 0); };
+  auto blocks = [&](int v) {
     const Shape2D sh = shape(v);
     return (M + sh.tl * t - 1) / (sh.tl * t) * sh.slices;
-  });
+  };
+  const int V = ragged_vec(C, es, 8, in_place, blocks);
   const int whole = row_vec(C, es, 8, true);
-  if (C % V == 0 || whole * es < 4 || (read && es == 4)) return V;
+  if (C % V == 0) return V;
+  int limit = 0;  // % of lanes in use
+  if (!read) limit = whole * es >= 4 ? 60 : events > 8 ? 55 : 0;
+  else if (whole * es >= 4 && es == 2) limit = 60;
+  else if (whole == 1 && events >= 8 && C >= 64 && blocks(V) <= 5 * int64_t(device_cus()))
+    limit = es == 4 ? 90 : events > 16 && C >= 128 ? 80 : 55;
   const Shape2D sh = shape(V);
-  return 5 * ((C + V - 1) / V) < 3 * sh.bcg * sh.slices ? whole : V;
+  return 100 * ((C + V - 1) / V) < limit * sh.bcg * sh.slices ? whole : V;
 }
 
 int chunk_count(int64_t M, int tokens_per_chunk, int max_chunks) {
@@ -4345,7 +4365,7 @@ int sihc_read(const void* x, const void* alpha, void* const* out, int events, in
       return check_launch(what);
     });
   }
-  const Shape2D sh = cell == 2 ? shape_for(channels, V, read_lanes(channels, V), events * S * wbytes)
+  const Shape2D sh = cell == 2 ? shape_for(channels, V, read_lanes(channels, V, events, g.M), events * S * wbytes)
                                : shape_for(channels, V, events <= 8 ? 64 : SIHC_RW_BCG_K4, events * S * wbytes,
                                            SIHC_RW_LDS_K4);  // 64 lanes to 8 events: E = 4 569 -> 542 us
   const int unroll = d2 ? SIHC_RD2_U : cell == 2 ? SIHC_RW_UNROLL : SIHC_RW_UNROLL_K4;

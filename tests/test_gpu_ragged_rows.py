@@ -147,6 +147,25 @@ def test_ragged_rows_of_large_grids(dtype, channels):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("batch", [16, 64])  # 32-lane reads from three blocks per CU
+@pytest.mark.parametrize("channels,events", [(67, 12), (131, 12), (131, 20), (195, 20)])
+def test_ragged_rows_of_many_events(dtype, batch, channels, events):
+    """Both sides of the lines at which many-event reads and writes keep a dividing vector."""
+    announce(f"ragged rows, batch {batch} C={channels} E={events} {dtype}")
+    gen = torch.Generator().manual_seed(channels + events)
+    x = torch.randn(batch, 32, 32, channels, generator=gen).to(dtype)
+    z = [torch.randn(batch, 256, channels, generator=gen).to(dtype) for _ in range(events)]
+    w = (0.25 + 0.1 * torch.randn(events, channels, 4, generator=gen)).to(dtype)
+    outs = [Out(z[0].shape, dtype) for _ in range(events)]
+    launch.read(_off(x.cuda()), w.cuda(), out=[o.t for o in outs])
+    for o, want in zip(outs, O.read(x, w)):
+        assert_parity(o.check(), want, dtype, what="read")
+    out = Out(x.shape, dtype)
+    launch.write(_off(x.cuda()), [_off(t.cuda()) for t in z], w.cuda(), out=out.t)
+    assert_parity(out.check(), O.write(x, z, w), dtype, what="write")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("channels", [67, 130, 259])
 def test_outputs_that_are_inputs(dtype, channels):
     """Every entry point that lets an output be one of its inputs, at widths whose last lane
