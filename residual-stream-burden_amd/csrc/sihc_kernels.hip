@@ -4003,13 +4003,21 @@ int launch_wgrad(const char* what, const void* x, const void* const* z, void* ou
     const void* const* outs = const_cast<const void* const*>(dout);
     in_place = any_equal(z, events, outs, events) || any_equal(&x, 1, outs, events);
   }
-  // Rows too narrow for a vector that does not divide them (65,536 x 9 bf16: fused backward of 5
-  // updates 25 us with one element, 37 with 8; gamma gradient of 5 24 and 20), and one or two
-  // updates where the launch has no lanes to spare (4,096 x 130 bf16, one update: fused backward
-  // 8.4 us with 2-element vectors, 10.4 with 8, alone 6.4 and 8.7; alone also up to 256 channels,
-  // 65,536 x 99 22 and 26).
-  const bool few = !carrier && events <= 2 &&
-                   (int64_t(g.M) * g.C < (1 << 20) || (!dout && events == 1 && es == 2 && g.C < 256));
+  // A dividing vector for rows too narrow for another one (65,536 x 9 bf16: fused backward of 5
+  // updates 25 us with one element, 37 with 8; gamma gradient of 5 24 and 20), and where the
+  // launch has no lanes to spare:
+  //   one or two updates (4,096 x 130 bf16, one update: fused backward 8.4 us with 2-element
+  //     vectors, 10.4 with 8, alone 6.4 and 8.7; alone also up to 256 channels, 65,536 x 99 22 and
+  //     26);
+  //   the fused backward of many updates of few rows (bf16: 5 of 1,024 x 67 9.0 and 10.8, 11 of
+  //     2,048 x 99 14.5 and 16; past the lines 3 of 1,024 x 67 10.7 and 8.5, 23 of 2,048 x 99 42
+  //     and 26, 5 of 8,192 x 67 15 and 12; fp32: 23 of 256 x 67 8.4 and 17, 5 of 1,024 x 67 8.9
+  //     with either).
+  const int64_t size = int64_t(g.M) * g.C;
+  bool few = false;
+  if (!carrier && events <= 2) few = size < (1 << 20) || (!dout && events == 1 && es == 2 && g.C < 256);
+  else if (dout && es == 2) few = events > 4 && size < (1 << 18) && size * events < (3 << 20);
+  else if (dout) few = events > 8 && size < (1 << 16);
   const int narrow = carrier ? 24 : dout ? (es == 2 ? 24 : 12) : events <= 2 ? 24 : 8;
   const int V = row_vec(g.C, es, 8, in_place || g.C < narrow || few);
   int bcg, slices;

@@ -166,6 +166,20 @@ def test_ragged_rows_of_many_events(dtype, batch, channels, events):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("rows,updates", [(1, 9), (1, 32), (4, 4), (4, 5), (4, 11), (64, 5)])
+def test_ragged_triangular_backward_of_few_rows(dtype, rows, updates):
+    """Both sides of the lines up to which many updates keep a dividing vector."""
+    gen = torch.Generator().manual_seed(updates)
+    grad, *z = (torch.randn(rows, 256, 67, generator=gen).to(dtype) for _ in range(updates + 1))
+    gamma = torch.randn(updates, 67, generator=gen)
+    got, dgamma = launch.triangular_backward(grad.cuda(), [t.cuda() for t in z], gamma.cuda())
+    want, dwant = O.triangular_backward(grad, z, gamma)
+    for a, e in zip(got, want):
+        assert_parity(a, e, dtype, what="dz")
+    assert_parity(dgamma, dwant, torch.float32, what="dgamma", kind="reduced")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("channels", [67, 130, 259])
 def test_outputs_that_are_inputs(dtype, channels):
     """Every entry point that lets an output be one of its inputs, at widths whose last lane
